@@ -2468,6 +2468,16 @@ struct RowsN {         // softmax state of the 16 RB rows of one wave
     f32x4 o[RB][8];    // O^T per row block: dims 16db + 4grp + i of row 16rb + lane%16
 };
 
+// 0 when every partial output of the wave's row block is finite, else NaN.
+__device__ __forceinline__ float finite_zero(const f32x4 (&o)[8]) {
+    float z = 0.0f;
+#pragma unroll
+    for (int db = 0; db < 8; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z = __fmaf_rn(o[db][i], 0.0f, z);
+    return z;
+}
+
 // p = 2^(u - m) for the log2-domain scores u[rb][0..7] of the RB row blocks (keys
 // 16(e/4) + 4grp + e%4 of the block; masked keys -inf), l += p, O^T += V^T P^T.  SHIFTED:
 // the scores are u - m already.
@@ -2502,6 +2512,17 @@ constexpr size_t ROUTE_LDS_MAX = 160 * 1024;         // LDS of one workgroup on 
 // Passes of a tile in the route kernels: one at the select launch's reference, and when a row
 // total leaves range one more at every row's exact largest score (in range by construction).
 constexpr int MAX_PASSES = 2;
+// The fixed softmax reference of a row is its largest far-field score plus REF_SHIFT octaves.  A leaf's
+// far-field score is a lower bound of the leaf's exact log-mass (the log-sum-exp is convex in the row),
+// so a near leaf's exact score can lie far above the reference and hardly below: over heads of 40759
+// tokens whose scores spread by 11 nats a row's total is -0.2 to 116 octaves above its largest far-field score,
+// and with the range [-60, 64] a quarter of the tiles were computed twice.  Totals in [REF_MIN, REF_MAX]
+// are 48 octaves below to 136 above it, and keep every key of weight 2^-42 or more in a float's normal
+// range; a row of outputs that overflows at such a total (values past 2^27) also sends its tile to the redo.
+constexpr float REF_SHIFT = 36.0f, REF_MIN = 0x1p-84f, REF_MAX = 0x1p100f;
+__device__ __forceinline__ float row_reference(float m) {
+    return m == -INFINITY ? 0.0f : __fadd_rn(__fmul_rn(m, LOG2E), REF_SHIFT);
+}
 // Merge: the wave pairs' partial O, 64 rows x 128 dims each, rows padded to 132 floats.
 constexpr int MRG_STRIDE = 132;
 // Ring slots per pair: blocks are loaded RS - 1 ahead.  Two slots (one block in flight while the
@@ -2701,6 +2722,14 @@ __global__ __launch_bounds__(256, 4) void route_select_kernel(
     if (kxe > 0) topk_row([&](int l) { return keys[l]; }, nb, kxe, sm, idx + gs * kxe, nullptr, nullptr);
 }
 
+// The lane index computed anew (not from a register held since the kernel's start): code after a
+// kernel's key loops uses it where holding lane values across the loops would spill.
+__device__ __forceinline__ int fresh_lane() {
+    int lane;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+    return lane;
+}
+
 // Largest scores of a wave's rows: the repair of a missed softmax reference in the route kernels.
 template <int RB>
 struct RowMax {
@@ -2721,8 +2750,7 @@ __device__ __forceinline__ RowMax<RB> route_exact_max(const int8_t* dq8, const f
                                                    const float* lz, const uint32_t* exbits, int64_t srow0, int lo,
                                                    int hi, const int8_t* k8, const float* ks, const uint32_t* sidx,
                                                    int64_t kh, int e_lo, int e_hi, int64_t rowb) {
-    int lane = threadIdx.x & 63;
-    asm volatile("" : "+v"(lane));
+    const int lane = fresh_lane();
     const int col = lane & 15, grp = lane >> 4;
     const int64_t row0 = rowb + col;
     RowMax<RB> mx;
@@ -2759,6 +2787,7 @@ __device__ __forceinline__ RowMax<RB> route_exact_max(const int8_t* dq8, const f
         bq[rb][1] = *(const i32x4*)(q8 + p * D + 64 + 16 * grp);
         srow[rb] = __fmul_rn(__fmul_rn(sq[p], scale), LOG2E);
     }
+    asm volatile("" : "+s"(e_lo));                // (its LDS address likewise)
     for (int j = e_lo; j < e_hi; j += 16) {       // 16-token runs of the near leaves
         const int64_t tok = kh + (int64_t)__builtin_amdgcn_readfirstlane(sidx[j / LEAF]) * LEAF + (j % LEAF);
         const i32x4 A0 = *(const i32x4*)(k8 + (tok + col) * D + 16 * grp);
@@ -2835,8 +2864,7 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
     float mref[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
-        const float m = rowmax[row0 + 16 * rb];
-        mref[rb] = m == -INFINITY ? 0.0f : __fmul_rn(m, LOG2E);
+        mref[rb] = row_reference(rowmax[row0 + 16 * rb]);
     }
     __syncthreads();
     for (int j = threadIdx.x; j < kxe; j += NT) atomicOr(&exbits[sidx[j] >> 5], 1u << (sidx[j] & 31));
@@ -2888,7 +2916,9 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
     auto run_pos = [&](int j) { return j < e_hi ? j : e_lo; };
     auto issue_near = [&](int bi, int slot) {
         if (bi >= nn) return;
-        const int e0 = e_lo + 32 * bi, ja = run_pos(e0), jb = run_pos(e0 + 16);
+        int e0 = e_lo + 32 * bi;
+        asm volatile("" : "+s"(e0));     // (a loop-invariant LDS address would be held, and spilled, across the far loop)
+        const int ja = run_pos(e0), jb = run_pos(e0 + 16);
         const int64_t r0 = kh + (int64_t)__builtin_amdgcn_readfirstlane(sidx[ja / LEAF]) * LEAF + (ja % LEAF);
         const int64_t r1 = kh + (int64_t)__builtin_amdgcn_readfirstlane(sidx[jb / LEAF]) * LEAF + (jb % LEAF);
         load_block(std::false_type{}, pring_lds + slot * SLOT_BYTES, k8, v, r0, r1, ks + r0, ks + r1, 3);
@@ -3034,18 +3064,17 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         // score - m in one rounding
-                        if constexpr (LEAF % 32 == 0) {   // the near list is whole 32-token blocks
 #pragma unroll
-                            for (int rb = 0; rb < RB; ++rb)
-                                sc[rb][4 * hh + i] = __fmaf_rn((float)acc[rb][i], __fmul_rn(srow[rb], ksv[i]), -st.m[rb]);
-                        } else {                          // leaf 16: the last block may be half empty
-                            const bool ok = (e0 + 16 * hh + 4 * grp + i) < e_hi;
-#pragma unroll
-                            for (int rb = 0; rb < RB; ++rb)
-                                sc[rb][4 * hh + i] = __fmaf_rn((float)acc[rb][i], __fmul_rn(srow[rb], ksv[i]),
-                                                               ok ? -st.m[rb] : -INFINITY);
-                        }
+                        for (int rb = 0; rb < RB; ++rb)
+                            sc[rb][4 * hh + i] = __fmaf_rn((float)acc[rb][i], __fmul_rn(srow[rb], ksv[i]), -st.m[rb]);
                     }
+                }
+                // leaf 16: the second run of the last block may lie past the list (else whole 32-token blocks)
+                if (LEAF % 32 != 0 && e0 + 16 >= e_hi) {
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) sc[rb][4 + i] = -INFINITY;
                 }
                 u32x2 pvop[8][2];
 #pragma unroll
@@ -3061,13 +3090,12 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
             }
         }
         // Row totals over the NP key parts (all at the same reference).  A total outside
-        // [2^-60, 2^64] means the reference missed the row's maximum by more than 60 octaves
-        // (an outlier key far above the far-field maximum, or rows under a sampled tile
-        // reference far below it; never observed on real scores): the tile is redone once at
-        // every row's exact largest score, where each row total lies in [1, keys].
+        // [REF_MIN, REF_MAX] means the reference missed the row's maximum (an outlier key far above
+        // the far-field maximum, or rows under a sampled tile reference far below it): the tile
+        // is redone once at every row's exact largest score, where each row total lies in [1, keys].
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-            const float lt = grp_sum(st.l[rb]);
+            const float lt = grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero(st.o[rb])) : st.l[rb]);
             if (grp == 0) red_l[pr][16 * RB * hr + 16 * rb + col] = lt;
         }
         if (threadIdx.x == 0) redo = 0;
@@ -3076,7 +3104,7 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
             const float tot = row_total(16 * RB * hr + 16 * rb + col);
-            if (!(tot >= 0x1p-60f && tot <= 0x1p64f)) bad = true;
+            if (!(tot >= REF_MIN && tot <= REF_MAX)) bad = true;
         }
         if (bad) redo = 1;
         __syncthreads();
@@ -3097,6 +3125,7 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
         }
     }
     if constexpr (NP == 1) {
+        const int ln = fresh_lane(), col = ln & 15, grp = ln >> 4;
         // one pair: each wave holds its rows' finished O^T; lanes (col, grp) write dims
         // 16 db + 4 grp .. + 3 of row 16 RB hr + 16 rb + col, normalised by the row total
 #pragma unroll
@@ -3175,8 +3204,8 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
 //     are read.  Far: score = (dq . g) (* 256 sg) + lz, PV with
 //     fp16(p * 256 sv) . vb (fp8) or bf16(p) . vb (bf16); near: score = (q . k) * scale (bf16),
 //     PV bf16(p) . v -- the products of tile16_kernel, in one softmax whose reference is the
-//     row's far-field maximum (redone with a moved reference if a row total leaves
-//     [2^-60, 2^64], as route_kernel).
+//     row's far-field maximum, REF_SHIFT octaves up for the bf16 store (redone with a moved reference
+//     if a row total leaves its range, as route_kernel).
 // ---------------------------------------------------------------------------------------------
 // 16-byte position of chunk c of row r of 128-byte rows (e4m3 codes) staged in LDS: c ^ sw8(r).
 // A read of 8 bytes per lane whose 32 lanes touch 16 rows, rows 16 h + 0..15 or 4 g + 0..3,
@@ -3517,7 +3546,7 @@ __global__ __launch_bounds__(64 * NW, 2) void route16_kernel(
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
         const float m = rowmax[prow0 + 16 * rb];
-        mref[rb] = m == -INFINITY ? 0.0f : __fmul_rn(m, LOG2E);
+        mref[rb] = FP8 ? (m == -INFINITY ? 0.0f : __fmul_rn(m, LOG2E)) : row_reference(m);   // (fp8: far P is fp16)
     }
     // B operands of the rows: q - mu through the far blocks, then q through the near blocks (one
     // register set, reloaded at the switch)
@@ -3754,13 +3783,12 @@ __global__ __launch_bounds__(64 * NW, 2) void route16_kernel(
                 if (bi + 1 < nblk) near_step(P1(), bi + 1);
             }
         }
-        // row totals: outside [2^-60, 2^64] the reference missed the row's maximum by more than 60
-        // octaves (2^-8 with the fp8 store: its far-field P is fp16, whose subnormals would hold
+        // row totals: outside [REF_MIN, REF_MAX] the reference missed the row's maximum (below 2^-8 with the fp8 store: its far-field P is fp16, whose subnormals would hold
         // the far leaves of a row whose total is that small with too few bits): the tile is redone
         // once at every row's exact largest score, where each row total lies in [1, keys]
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-            const float lt = grp_sum(st.l[rb]);
+            const float lt = grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero(st.o[rb])) : st.l[rb]);
             if (grp == 0) red_l[16 * RB * wv + 16 * rb + col] = lt;
         }
         if (threadIdx.x == 0) redo = 0;
@@ -3769,7 +3797,7 @@ __global__ __launch_bounds__(64 * NW, 2) void route16_kernel(
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
             const float tot = red_l[16 * RB * wv + 16 * rb + col];
-            if (!(tot >= (FP8 ? 0x1p-8f : 0x1p-60f) && tot <= 0x1p64f)) bad = true;
+            if (!(tot >= (FP8 ? 0x1p-8f : REF_MIN) && tot <= REF_MAX)) bad = true;
         }
         if (bad) redo = 1;
         __syncthreads();
