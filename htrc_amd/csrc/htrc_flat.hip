@@ -2805,16 +2805,46 @@ __device__ __forceinline__ RowMax<RB> route_exact_max(const int8_t* dq8, const f
     return mx;
 }
 
+// Long tiles: a tile whose far and near fields are more than SEG_MIN_BLOCKS 32-key blocks has its
+// block stream (far, then near) cut into route_segments() equal segments, each summed from zero,
+// and the segments' sums added in order.  That order is fixed by the tile's block count alone, so the
+// segments may run as workgroups of their own (route_part_kernel, partial sums in workspace,
+// combined by route_seg_kernel) or one after the other in one workgroup (route_seg_kernel), bit for bit alike:
+// the launch takes the first where a window's tiles alone leave the CUs short of waves.
+// Measured on heads of 40759 tokens (leaf 16): a 128-tile window of 208 blocks 178 us whole (one wave
+// pair a tile: 256 waves for 1024 SIMDs), 50 + 22 us in parts (the head 965 -> 706 us a call); 256 tiles
+// of 592 blocks 507 -> 270 + 30 us; 768 tiles of 318 blocks 605 whole, 587 + 92 in parts, 556 in turn,
+// so launches of more than 512 tiles run in turn.  4 segments against 6, 8 and 16: 706 / 715 / 720 /
+// 720 us.  Below 128 blocks the whole-tile kernels' key halves and quarters serve.
+constexpr int SEG_MIN_BLOCKS = 128;
+constexpr int SEG_MAX = 4;
+constexpr int64_t SEG_SPLIT_TILES = 512;             // launches of at most this many tiles run the segments apart
+enum RouteMode { ROUTE_WHOLE = 0, ROUTE_PART = 1, ROUTE_SEGS = 2 };
+constexpr int SEG_QUARTERS = 4;                      // workgroups per tile that combine its partial sums
+
+// (heads of more than ROUTE_NB_LDS leaves, whose select works from global keys, keep whole tiles)
+inline int route_segments(int64_t nb, int kxe, int leaf) {
+    const int64_t blocks = (nb + 31) / 32 + ((int64_t)kxe * leaf + 31) / 32;
+    if (blocks <= SEG_MIN_BLOCKS || nb > ROUTE_NB_LDS) return 1;
+    const int64_t n = (blocks + 31) / 32;
+    return (int)(n < SEG_MAX ? n : SEG_MAX);
+}
+
 // RB = tile / 32: 16-row blocks per wave (tiles of 64 or 32 rows); NP wave pairs split the keys;
-// RS ring slots per pair.
-template <int LEAF, int RB, int NP, int RS>
-__global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_kernel(
+// RS ring slots per pair.  MODE ROUTE_WHOLE: the tile's keys in one sum.  ROUTE_PART: workgroup
+// (tile, segment), the segment's O and row sums to part_o / part_l [tile of the launch][segment].
+// ROUTE_SEGS: with part_o, SEG_QUARTERS workgroups per tile add the tile's partial sums (the redo of a
+// tile whose reference missed is the first one's); without, one workgroup runs the segments in turn.
+template <int LEAF, int RB, int NP, int RS, int MODE>
+__device__ __forceinline__ void route_body(
     const int8_t* __restrict__ q8, const float* __restrict__ sq, const int8_t* __restrict__ dq8,
     const float* __restrict__ sdq, const int8_t* __restrict__ g8, const float* __restrict__ sg,
     const float* __restrict__ lz, const uint16_t* __restrict__ vb, const int8_t* __restrict__ k8,
     const float* __restrict__ ks, const uint16_t* __restrict__ v, const int32_t* __restrict__ idx,
     const float* __restrict__ rowmax, int64_t nq, int nt, int group, int g0, int ng, const int32_t* __restrict__ perm,
-    int64_t nk, int nb, int nb_pad, int kxe, float scale, float* __restrict__ out, float* __restrict__ logz) {
+    int64_t nk, int nb, int nb_pad, int kxe, float scale, float* __restrict__ out, float* __restrict__ logz,
+    float* __restrict__ part_o, float* __restrict__ part_l, int nseg) {
+    static_assert(MODE == ROUTE_WHOLE || NP == 1, "segments run on one wave pair");
     constexpr int NT = 128 * NP;                               // threads
     __shared__ __align__(16) char ring[NP][RS][SLOT_BYTES];    // one per wave pair; also merge staging
     // sized by the launch: exclusion bits [nb / 32 + 1], then the tile's near leaves [kxe], so
@@ -2847,10 +2877,64 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
     // launch's own.
     const int tb = g0 * group, ntw = min(nt, (g0 + ng) * group) - tb;
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-    const int t = tb + (int)(blk % (uint32_t)ntw), h = (int)(blk / (uint32_t)ntw);
+    // segments: tile fastest, so an XCD runs one segment of consecutive tiles, whose near leaves (in
+    // ascending order) come from one stretch of the head's keys
+    const uint32_t units = MODE == ROUTE_PART ? gridDim.x / (uint32_t)nseg
+                                              : (MODE == ROUTE_SEGS && part_o ? gridDim.x / SEG_QUARTERS : gridDim.x);
+    const uint32_t unit = MODE == ROUTE_WHOLE ? blk : blk % units;
+    const int sub = MODE == ROUTE_WHOLE ? 0 : (int)(blk / units);        // segment, or quarter of the rows
+    const int t = tb + (int)(unit % (uint32_t)ntw), h = (int)(unit / (uint32_t)ntw);
     const int64_t th = (int64_t)h * nt + t;
     const int64_t gs = (int64_t)h * ng + (t / group - g0);    // state / routing row: the tile's group
     const int64_t kh = (int64_t)h * nk;
+    if constexpr (MODE == ROUTE_SEGS) {
+        if (part_o) {
+            // the tile's row totals over its segments, added in segment order; a total out of range
+            // (see the end of a pass) sends the tile to the redo below
+            const float* pl = part_l + (int64_t)unit * nseg * TR;
+            if (threadIdx.x == 0) redo = 0;
+            __syncthreads();
+            if (threadIdx.x < TR) {
+                float tot = 0.0f;
+                for (int s = 0; s < nseg; ++s) tot = __fadd_rn(tot, pl[s * TR + threadIdx.x]);
+                red_l[0][threadIdx.x] = tot;
+                if (!(tot >= REF_MIN && tot <= REF_MAX)) redo = 1;
+            }
+            __syncthreads();
+            if (__builtin_expect(redo == 0, 1)) {
+                constexpr int CH = TR / SEG_QUARTERS * (D / 4) / NT;     // 16-byte chunks per thread
+                const int r0 = TR / SEG_QUARTERS * sub;
+                const float* po = part_o + ((int64_t)unit * nseg * TR + r0) * D;
+                f32x4 acc[CH];
+#pragma unroll
+                for (int c = 0; c < CH; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int s = 0; s < nseg; ++s) {
+#pragma unroll
+                    for (int c = 0; c < CH; ++c) {
+                        const f32x4 y = *(const f32x4*)(po + (int64_t)s * TR * D + 4 * (NT * c + threadIdx.x));
+                        acc[c] = f32x4{__fadd_rn(acc[c][0], y[0]), __fadd_rn(acc[c][1], y[1]),
+                                       __fadd_rn(acc[c][2], y[2]), __fadd_rn(acc[c][3], y[3])};
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < CH; ++c) {
+                    const int e = NT * c + threadIdx.x, r = r0 + e / (D / 4), dl = 4 * (e % (D / 4));
+                    const int64_t qi = (int64_t)t * TR + r;
+                    if (qi >= nq) continue;
+                    const float den = red_l[0][r];
+                    const float inv = 1.0f / (den < 1e-30f ? 1e-30f : den);
+                    const int64_t orow = (int64_t)h * nq + perm_row(perm, h, nq, qi);
+                    *(f32x4*)(out + orow * D + dl) = f32x4{__fmul_rn(acc[c][0], inv), __fmul_rn(acc[c][1], inv),
+                                                           __fmul_rn(acc[c][2], inv), __fmul_rn(acc[c][3], inv)};
+                    if (dl == 0) {
+                        logz[orow] = __fadd_rn(__fmul_rn(row_reference(rowmax[th * TR + r]), LN2), __logf(den));
+                    }
+                }
+                return;
+            }
+            if (sub != 0) return;
+        }
+    }
     const int64_t row0 = th * TR + 16 * RB * hr + col;         // this lane's rows: row0 (+ 16 when RB = 2)
     // ---- routing of this tile (route_select_kernel)
     // exclusion bits: the selected (near) leaves, and every leaf >= nb, so the far loop needs no
@@ -2873,15 +2957,25 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
     const int lpw = ((nb + NP - 1) / NP + 31) / 32 * 32;
     const int e_n = kxe * LEAF;
     const int epw = ((e_n + NP - 1) / NP + 31) / 32 * 32;
-    const int lo = pr * lpw, hi = min(nb, lo + lpw);
-    const int e_lo = pr * epw, e_hi = min(e_n, e_lo + epw);
-    const int nf = hi > lo ? (hi - lo + 31) / 32 : 0;
-    const int nn = e_hi > e_lo ? (e_hi - e_lo + 31) / 32 : 0;
-    const int sf_steps = min(nb, lpw) > 0 ? (min(nb, lpw) + 31) / 32 : 0;        // pair 0 is the longest
-    const int sn_steps = min(e_n, epw) > 0 ? (min(e_n, epw) + 31) / 32 : 0;
+    int lo = pr * lpw, hi = min(nb, lo + lpw);
+    int e_lo = pr * epw, e_hi = min(e_n, e_lo + epw);
+    int nf = hi > lo ? (hi - lo + 31) / 32 : 0;
+    int nn = e_hi > e_lo ? (e_hi - e_lo + 31) / 32 : 0;
+    int sf_steps = min(nb, lpw) > 0 ? (min(nb, lpw) + 31) / 32 : 0;              // pair 0 is the longest
+    int sn_steps = min(e_n, epw) > 0 ? (min(e_n, epw) + 31) / 32 : 0;
+    // segment s: blocks [s len, s len + len) of the tile's far blocks followed by its near blocks
+    auto set_segment = [&](int s) {
+        const int nbf = (nb + 31) / 32, nbn = (e_n + 31) / 32, len = (nbf + nbn + nseg - 1) / nseg;
+        const int b0 = min(nbf + nbn, s * len), b1 = min(nbf + nbn, b0 + len);
+        lo = 32 * min(nbf, b0), hi = min(nb, 32 * min(nbf, b1));
+        e_lo = 32 * max(0, b0 - nbf), e_hi = min(e_n, 32 * max(0, b1 - nbf));
+        sf_steps = nf = hi > lo ? (hi - lo + 31) / 32 : 0;
+        sn_steps = nn = e_hi > e_lo ? (e_hi - e_lo + 31) / 32 : 0;
+    };
+    if constexpr (MODE == ROUTE_PART) set_segment(sub);
     // far steps rounded up to even (an odd count takes one empty step), so the near blocks
     // start in ring slot 0 and the last far step issues the first of them
-    const int sf_even = (sf_steps + 1) & ~1;
+    int sf_even = (sf_steps + 1) & ~1;
     const int64_t srow0 = gs * nb_pad;
     char* pring = &ring[pr][0][0];
     const uint32_t pring_lds = lds_addr(pring);
@@ -2933,8 +3027,25 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
         asm volatile("" : "+v"(tra[db]));   // one register each: no add at every read
     }
     RowsN<RB> st;
+    RowsN<MODE == ROUTE_SEGS ? RB : 1> sum;                    // ROUTE_SEGS: the segments' sums so far
+    bool redone = false;                                       // ROUTE_SEGS: combining found the tile out of range
+    if constexpr (MODE == ROUTE_SEGS) redone = part_o != nullptr;
 #pragma unroll 1
     for (int pass = 0; pass < MAX_PASSES; ++pass) {
+        if constexpr (MODE == ROUTE_SEGS) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                sum.l[rb] = 0.0f;
+#pragma unroll
+                for (int db = 0; db < 8; ++db) sum.o[rb][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
+#pragma unroll 1
+        for (int seg = MODE == ROUTE_SEGS && redone && pass == 0 ? nseg : 0; seg < (MODE == ROUTE_SEGS ? nseg : 1); ++seg) {
+        if constexpr (MODE == ROUTE_SEGS) {
+            set_segment(seg);
+            sf_even = (sf_steps + 1) & ~1;
+        }
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
             st.m[rb] = mref[rb];
@@ -3089,13 +3200,39 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
                 if (bi + 1 < sn_steps) step(std::integral_constant<int, 1>{}, bi + 1);
             }
         }
+        if constexpr (MODE == ROUTE_SEGS) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                sum.l[rb] = __fadd_rn(sum.l[rb], grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero(st.o[rb])) : st.l[rb]));
+#pragma unroll
+                for (int db = 0; db < 8; ++db)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) sum.o[rb][db][i] = __fadd_rn(sum.o[rb][db][i], st.o[rb][db][i]);
+            }
+        }
+        }
+        if constexpr (MODE == ROUTE_PART) {
+            // the segment's sums: row r's O^T in lanes (col, grp), dims 16 db + 4 grp ..
+            const int64_t pb = ((int64_t)unit * nseg + sub) * TR;
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                const int r = 16 * RB * hr + 16 * rb + col;
+                const float lt = grp_sum(__fadd_rn(st.l[rb], finite_zero(st.o[rb])));
+                if (grp == 0) part_l[pb + r] = lt;
+#pragma unroll
+                for (int db = 0; db < 8; ++db) *(f32x4*)(part_o + (pb + r) * D + 16 * db + 4 * grp) = st.o[rb][db];
+            }
+            return;
+        }
         // Row totals over the NP key parts (all at the same reference).  A total outside
         // [REF_MIN, REF_MAX] means the reference missed the row's maximum (an outlier key far above
         // the far-field maximum, or rows under a sampled tile reference far below it): the tile
         // is redone once at every row's exact largest score, where each row total lies in [1, keys].
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-            const float lt = grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero(st.o[rb])) : st.l[rb]);
+            float lt;
+            if constexpr (MODE == ROUTE_SEGS) lt = sum.l[rb];
+            else lt = grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero(st.o[rb])) : st.l[rb]);
             if (grp == 0) red_l[pr][16 * RB * hr + 16 * rb + col] = lt;
         }
         if (threadIdx.x == 0) redo = 0;
@@ -3109,6 +3246,8 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
         if (bad) redo = 1;
         __syncthreads();
         if (__builtin_expect(redo == 0 || pass + 1 == MAX_PASSES, 1)) break;
+        
+        if constexpr (MODE == ROUTE_SEGS) lo = 0, hi = nb, e_lo = 0, e_hi = e_n;
         const RowMax<RB> mx = route_exact_max<LEAF, RB>(dq8, sdq, q8, sq, scale, g8, sg, lz, exbits, srow0, lo, hi, k8,
                                                         ks, sidx, kh, e_lo, e_hi, th * TR + 16 * RB * hr);
 #pragma unroll
@@ -3138,7 +3277,9 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
                 const int64_t orow = (int64_t)h * nq + perm_row(perm, h, nq, qi);
 #pragma unroll
                 for (int db = 0; db < 8; ++db) {
-                    const f32x4 o = st.o[rb][db];
+                    f32x4 o;
+                    if constexpr (MODE == ROUTE_SEGS) o = sum.o[rb][db];
+                    else o = st.o[rb][db];
                     *(f32x4*)(out + orow * D + 16 * db + 4 * grp) =
                         f32x4{__fmul_rn(o[0], inv), __fmul_rn(o[1], inv), __fmul_rn(o[2], inv), __fmul_rn(o[3], inv)};
                 }
@@ -3146,7 +3287,7 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
             }
         }
         return;
-    }
+    } else {
     // ---- merge: every pair used the same reference per row, so the partial sums simply add
     // (h3/htrc_flat_triton.py:263-273 with equal maxima).  MRG2: two rounds, the rows of row
     // half 0, then of row half 1, so the staging fits a 2-slot ring.
@@ -3187,7 +3328,36 @@ __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_ke
         }
         if (MRG2 && round == 0) __syncthreads();                   // the staging is reused
     }
+    }
 }
+
+#define ROUTE_PARAMS                                                                                                   \
+    const int8_t *__restrict__ q8, const float *__restrict__ sq, const int8_t *__restrict__ dq8,                       \
+        const float *__restrict__ sdq, const int8_t *__restrict__ g8, const float *__restrict__ sg,                    \
+        const float *__restrict__ lz, const uint16_t *__restrict__ vb, const int8_t *__restrict__ k8,                  \
+        const float *__restrict__ ks, const uint16_t *__restrict__ v, const int32_t *__restrict__ idx,                 \
+        const float *__restrict__ rowmax, int64_t nq, int nt, int group, int g0, int ng,                               \
+        const int32_t *__restrict__ perm, int64_t nk, int nb, int nb_pad, int kxe, float scale,                        \
+        float *__restrict__ out, float *__restrict__ logz
+#define ROUTE_ARGS                                                                                                     \
+    q8, sq, dq8, sdq, g8, sg, lz, vb, k8, ks, v, idx, rowmax, nq, nt, group, g0, ng, perm, nk, nb, nb_pad, kxe, scale, \
+        out, logz
+template <int LEAF, int RB, int NP, int RS>
+__global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_kernel(ROUTE_PARAMS) {
+    route_body<LEAF, RB, NP, RS, ROUTE_WHOLE>(ROUTE_ARGS, nullptr, nullptr, 1);
+}
+template <int LEAF, int RB>
+__global__ __launch_bounds__(128, 3) void route_part_kernel(ROUTE_PARAMS, float* __restrict__ part_o,
+                                                            float* __restrict__ part_l, int nseg) {
+    route_body<LEAF, RB, 1, ROUTE_RS, ROUTE_PART>(ROUTE_ARGS, part_o, part_l, nseg);
+}
+template <int LEAF, int RB>
+__global__ __launch_bounds__(128, 2) void route_seg_kernel(ROUTE_PARAMS, float* __restrict__ part_o,
+                                                           float* __restrict__ part_l, int nseg) {
+    route_body<LEAF, RB, 1, ROUTE_RS, ROUTE_SEGS>(ROUTE_ARGS, part_o, part_l, nseg);
+}
+#undef ROUTE_PARAMS
+#undef ROUTE_ARGS
 
 // ---------------------------------------------------------------------------------------------
 // route16: the fused production path for the 16-bit state stores (store="fp8": e4m3 g / vb with
@@ -4968,11 +5138,12 @@ static size_t route_dyn_bytes(int64_t nb, int kxe) { return ((size_t)(nb / 32 + 
 // Static LDS of route_kernel with NP wave pairs: the ring plus the row reductions.
 static size_t route_static_bytes(int np) { return (size_t)np * ROUTE_RS * SLOT_BYTES + 64 * 4 * (1 + np) + 16; }
 
-int htrc_route_attend(const int8_t* q8, const float* sq, const int8_t* dq8, const float* sdq, const int8_t* g8,
-                      const float* sg, const float* lz, const uint16_t* vb, const int8_t* k8, const float* ks,
-                      const uint16_t* v, const int32_t* idx, const float* rowmax, int64_t heads, int64_t nq,
-                      int64_t nk, int leaf, int d, int kx, int tile, int group, int64_t g0, int64_t gn,
-                      const int32_t* perm, float scale, float* out, float* logz, void* stream) {
+static int route_attend_launch(const int8_t* q8, const float* sq, const int8_t* dq8, const float* sdq, const int8_t* g8,
+                               const float* sg, const float* lz, const uint16_t* vb, const int8_t* k8, const float* ks,
+                               const uint16_t* v, const int32_t* idx, const float* rowmax, int64_t heads, int64_t nq,
+                               int64_t nk, int leaf, int d, int kx, int tile, int group, int64_t g0, int64_t gn,
+                               const int32_t* perm, float scale, float* out, float* logz, bool segs, float* parts,
+                               void* stream) {
     REQUIRE(q8 && sq && dq8 && sdq && g8 && sg && lz && vb && k8 && ks && v && rowmax && out && logz,
             "htrc_route_attend: null pointer");
     REQUIRE(aligned(vb, 16) && aligned(v, 16) && aligned(g8, 16) && aligned(k8, 16) && aligned(sg, 16) &&
@@ -4995,6 +5166,40 @@ int htrc_route_attend(const int8_t* q8, const float* sq, const int8_t* dq8, cons
     // every windowing of one layer give identical bits.
     const int64_t cus = device_cus();
     const size_t dyn = route_dyn_bytes(nb, kxe);
+    // Long tiles (segs: the caller runs them segmented, with workspace for the partial sums where
+    // the launch is small; see route_segments)
+    const int nseg = segs ? route_segments(nb, kxe, leaf) : 1;
+    if (nseg > 1) {
+        REQUIRE(route_static_bytes(1) + dyn <= ROUTE_LDS_MAX, "htrc_route_attend: near list and exclusion bits exceed the LDS");
+        const int64_t units = ntw * heads;
+        const bool split = parts && units <= SEG_SPLIT_TILES;
+        REQUIRE(!split || aligned(parts, 16), "htrc_route_attend: misaligned buffer");
+        float* part_o = split ? parts : nullptr;
+        float* part_l = split ? parts + units * nseg * tile * D : nullptr;
+#define SEG_LAUNCH(K, L, RB, N)                                                                                 \
+    hipLaunchKernelGGL((K<L, RB>), dim3((unsigned)(units * (N))), dim3(128), dyn, s, q8, sq, dq8, sdq, g8, sg, lz, vb, k8, ks, \
+                       v, idx, rowmax, nq, (int)nt, group, (int)g0, (int)gn, perm, nk, (int)nb, nbp, kxe, scale, out, \
+                       logz, part_o, part_l, nseg)
+#define SEG_CASE(L)                                                                                             \
+    case L:                                                                                                     \
+        if (tile == 64) {                                                                                       \
+            if (split) SEG_LAUNCH(route_part_kernel, L, 2, nseg);                                               \
+            SEG_LAUNCH(route_seg_kernel, L, 2, split ? SEG_QUARTERS : 1);                                       \
+        } else {                                                                                                \
+            if (split) SEG_LAUNCH(route_part_kernel, L, 1, nseg);                                               \
+            SEG_LAUNCH(route_seg_kernel, L, 1, split ? SEG_QUARTERS : 1);                                       \
+        }                                                                                                       \
+        break;
+        switch (leaf) {
+            SEG_CASE(16)
+            SEG_CASE(32)
+            SEG_CASE(64)
+            SEG_CASE(128)
+        }
+#undef SEG_CASE
+#undef SEG_LAUNCH
+        return launched("htrc_route_attend");
+    }
     int np = nt * heads >= 2 * cus ? 1 : (nt * heads > cus ? 2 : 4);
     while (np > 1 && route_static_bytes(np) + dyn > ROUTE_LDS_MAX) np /= 2;
     REQUIRE(route_static_bytes(np) + dyn <= ROUTE_LDS_MAX, "htrc_route_attend: near list and exclusion bits exceed the LDS");
@@ -5023,6 +5228,38 @@ int htrc_route_attend(const int8_t* q8, const float* sq, const int8_t* dq8, cons
 #undef ROUTE_CASE
 #undef ROUTE_LAUNCH
     return launched("htrc_route_attend");
+}
+
+int htrc_route_attend(const int8_t* q8, const float* sq, const int8_t* dq8, const float* sdq, const int8_t* g8,
+                      const float* sg, const float* lz, const uint16_t* vb, const int8_t* k8, const float* ks,
+                      const uint16_t* v, const int32_t* idx, const float* rowmax, int64_t heads, int64_t nq,
+                      int64_t nk, int leaf, int d, int kx, int tile, int group, int64_t g0, int64_t gn,
+                      const int32_t* perm, float scale, float* out, float* logz, void* stream) {
+    return route_attend_launch(q8, sq, dq8, sdq, g8, sg, lz, vb, k8, ks, v, idx, rowmax, heads, nq, nk, leaf, d, kx, tile,
+                               group, g0, gn, perm, scale, out, logz, false, nullptr, stream);
+}
+
+int htrc_route_segments(int64_t heads, int64_t nq, int64_t nk, int leaf, int kx, int tile, int group, int64_t g0,
+                        int64_t gn) {
+    int64_t nb, nt, ng, tb, ntw;
+    int kxe;
+    if (route_shapes("htrc_route_segments", heads, nq, nk, leaf, D, kx, tile, group, g0, gn, nb, nt, ng, tb, ntw, kxe) !=
+        HTRC_OK)
+        return 0;
+    return ntw * heads <= SEG_SPLIT_TILES ? route_segments(nb, kxe, leaf) : 1;
+}
+
+int htrc_route_seg(const int8_t* q8, const float* sq, const int8_t* dq8, const float* sdq, const int8_t* g8,
+                   const float* sg, const float* lz, const uint16_t* vb, const int8_t* k8, const float* ks,
+                   const uint16_t* v, int64_t heads, int64_t nq, int64_t nk, int leaf, int d, int kx, int sink,
+                   int stride, int tile, int group, int64_t g0, int64_t gn, const int32_t* perm, float scale, float* out,
+                   float* logz, int32_t* idx, float* rowmax, uint32_t* keys_ws, float* parts, void* stream) {
+    REQUIRE(q8 && sq && vb && k8 && ks && v && out && logz, "htrc_route_seg: null pointer");
+    int rc = htrc_route_select(dq8, sdq, g8, sg, lz, heads, nq, nk, leaf, d, kx, sink, stride, tile, group, g0, gn, idx,
+                               rowmax, keys_ws, stream);
+    if (rc != HTRC_OK) return rc;
+    return route_attend_launch(q8, sq, dq8, sdq, g8, sg, lz, vb, k8, ks, v, idx, rowmax, heads, nq, nk, leaf, d, kx,
+                               tile, group, g0, gn, perm, scale, out, logz, true, parts, stream);
 }
 
 int htrc_route(const int8_t* q8, const float* sq, const int8_t* dq8, const float* sdq, const int8_t* g8,

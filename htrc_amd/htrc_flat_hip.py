@@ -21,6 +21,7 @@ import torch
 
 from . import _lib
 from ._lib import call, ptr, stream_handle, nb_pad
+from .htrc_flat_runner import route_segments
 
 TILE = 64
 TILES = (64, 32)          # query rows per tile the kernels take (32: the runner's mode "max")
@@ -466,9 +467,13 @@ def route(packed: dict, state: dict, *, nq: int, leaf: int, kx: int, scale: floa
         idx = _rows(ws, "idx", h, gn, (kxe,), torch.int32, dev)
     rowmax = _rowmax(ws, rowmax, h, nt * tile, dev)
     keys = _keys_ws(ws, h, gn, nb, dev)
-    call("htrc_route", ptr(q8), ptr(sq), ptr(dq8), ptr(sdq), ptr(g8), ptr(sg), ptr(lz), ptr(vb), ptr(k8), ptr(ks),
+    # partial sums of the segments of a long tile, where a small window runs them apart
+    units = h * (min(nt, (g0 + gn) * int(group)) - g0 * int(group))
+    segs = route_segments(units, nb, kxe, int(leaf))
+    parts = _buf(ws, "parts", (units * segs * tile * (D + 1),), torch.float32, dev) if segs > 1 else None
+    call("htrc_route_seg", ptr(q8), ptr(sq), ptr(dq8), ptr(sdq), ptr(g8), ptr(sg), ptr(lz), ptr(vb), ptr(k8), ptr(ks),
          ptr(v), h, nq, nk, int(leaf), d, int(kx), int(sink), int(stride), tile, int(group), g0, gn, ptr(perm),
-         float(scale), ptr(out), ptr(logz), ptr(idx), ptr(rowmax), ptr(keys), stream_handle(dev))
+         float(scale), ptr(out), ptr(logz), ptr(idx), ptr(rowmax), ptr(keys), ptr(parts), stream_handle(dev))
     return out, logz
 
 

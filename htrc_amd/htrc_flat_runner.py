@@ -63,6 +63,19 @@ def _ceil(a: int, b: int) -> int:
 F32_UNSPLIT_TILES = 2048
 
 
+# Fused int8 route: the segments whose partial sums a launch of ``units`` (head, tile) pairs keeps in
+# workspace (htrc_route_segments of the C ABI): tiles of more than 128 blocks of 32 keys, in launches of at
+# most 512 pairs and heads of at most 16384 leaves.
+SEG_MIN_BLOCKS, SEG_MAX, SEG_SPLIT_TILES, SEG_MAX_NB = 128, 4, 512, 16384
+
+
+def route_segments(units: int, nb: int, kx: int, leaf: int) -> int:
+    blocks = _ceil(nb, 32) + _ceil(kx * leaf, 32)
+    if units > SEG_SPLIT_TILES or blocks <= SEG_MIN_BLOCKS or nb > SEG_MAX_NB:
+        return 1
+    return min(SEG_MAX, _ceil(blocks, 32))
+
+
 def workspace_bytes(queries: int, keys: int, leaf: int = 16, dim: int = 128, heads: int = 1, splits: int = 1,
                     kx: int = 0, group: int = 1, order: str = "seq", tile: int = TILE, tile_chunk: int | None = None,
                     store: str = "int8", fused: bool = True, bf16_inputs: bool = True, window_streams: int = 2,
@@ -101,6 +114,13 @@ def workspace_bytes(queries: int, keys: int, leaf: int = 16, dim: int = 128, hea
     fused = fused and kx <= 8192 and nb <= (262144 if store == "int8" else 16384)
     if fused:
         layer += 4 * rows                                               # rowmax, shared by the windows
+    if fused and store == "int8":
+        # partial sums of long tiles (the last window's where only that one is small enough)
+        for t in (tw, nt - (_ceil(nt, tw) - 1) * tw):
+            segs = route_segments(int(heads) * t, nb, kx, int(leaf))
+            if segs > 1:
+                window += t * segs * int(tile) * (dim + 1) * 4
+                break
     if fused and nb > 16384:
         window += 4 * gw * nbp                                          # route_select top-k keys
     if not fused:

@@ -54,7 +54,7 @@
 extern "C" {
 #endif
 
-#define HTRC_ABI_VERSION 15
+#define HTRC_ABI_VERSION 16
 
 #define HTRC_OK 0
 #define HTRC_ERR_ARG 1 /* invalid argument: shape, alignment, null pointer, knob */
@@ -158,6 +158,22 @@ int htrc_route(const int8_t* q8, const float* sq, const int8_t* dq8, const float
                const uint16_t* v, int64_t heads, int64_t nq, int64_t nk, int leaf, int d, int kx, int sink,
                int stride, int tile, int group, int64_t g0, int64_t gn, const int32_t* perm, float scale, float* out,
                float* logz, int32_t* idx, float* rowmax, uint32_t* keys_ws, void* stream);
+
+/* htrc_route for tiles of many keys: a tile of more than 128 32-key blocks (far leaves and near
+ * tokens) is summed in htrc_route_segments() segments whose order the tile's block count alone
+ * fixes, so every window and launch of a layer gives the same bits.  parts (fp32, 16-byte aligned,
+ * heads * tiles of the window * segments * T * 129 floats; NULL when htrc_route_segments() is 1)
+ * takes the segments' sums where the window is small enough that they run as workgroups of their
+ * own; without it, and in larger windows, one workgroup runs a tile's segments in turn.
+ * htrc_route_segments: the segments per tile that the window's launch keeps in parts, 1 when it needs
+ * none, 0 with an error set when the arguments are invalid. */
+int htrc_route_segments(int64_t heads, int64_t nq, int64_t nk, int leaf, int kx, int tile, int group, int64_t g0,
+                        int64_t gn);
+int htrc_route_seg(const int8_t* q8, const float* sq, const int8_t* dq8, const float* sdq, const int8_t* g8,
+                   const float* sg, const float* lz, const uint16_t* vb, const int8_t* k8, const float* ks,
+                   const uint16_t* v, int64_t heads, int64_t nq, int64_t nk, int leaf, int d, int kx, int sink,
+                   int stride, int tile, int group, int64_t g0, int64_t gn, const int32_t* perm, float scale, float* out,
+                   float* logz, int32_t* idx, float* rowmax, uint32_t* keys_ws, float* parts, void* stream);
 
 /* htrc_route without caller workspace: rowmax, the near leaves and the top-k keys live in a
  * scratch array of 32 MiB that the library keeps on each device (resolved at the first call on
