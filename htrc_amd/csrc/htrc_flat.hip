@@ -4188,17 +4188,24 @@ __global__ __launch_bounds__(128) void km_init_kernel(const void* __restrict__ q
     cen[((int64_t)h * C + j) * D + i] = qval<IN_BF16>(q, ((int64_t)h * nq + row) * D + i);
 }
 
-// Nearest centre of 256 rows (of the sample when sm > 0, else of the queries): one row per
+// Nearest centre of 256 / NS rows (of the sample when sm > 0, else of the queries): one row per
 // lane, its 128 values in registers.  The centres are wave-uniform: read straight from memory
 // (scalar loads into operands, no per-lane copies), four centres per step as independent sums
 // (then pairs, then one), compared in increasing order so that ties keep the lower centre.
-template <bool IN_BF16>
-__global__ __launch_bounds__(256) void km_assign_kernel(const void* __restrict__ q, int64_t nq, int64_t nrows, int sm,
+// NS > 1: the NS waves of a workgroup take the same 64 rows and a share of the centres each,
+// compared across the waves through LDS in centre order.  One wave per 64 rows leaves SIMDs idle, and
+// each busy one waiting on its own sums, where the launch has no more waves than SIMDs: 4096 sample rows of
+// one head (64 waves) 40.7 us a launch, NS = 4 17.9; 40759 rows 40.5 -> 21.2 us.
+template <bool IN_BF16, int NS>
+__global__ __launch_bounds__(NS == 1 ? 256 : 64 * NS) void km_assign_kernel(const void* __restrict__ q, int64_t nq, int64_t nrows, int sm,
                                                         int C, const float* __restrict__ cen,
                                                         int32_t* __restrict__ assign) {
     const int h = blockIdx.y, tid = threadIdx.x;
     const float* __restrict__ ch = cen + (int64_t)h * C * D;
-    const int64_t ri = (int64_t)blockIdx.x * 256 + tid;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t ri = NS == 1 ? (int64_t)blockIdx.x * 256 + tid : (int64_t)blockIdx.x * 64 + (tid & 63);
+    const int cpw = NS == 1 ? C : (C + NS - 1) / NS;
+    const int ce = NS == 1 ? C : min(C, (wv + 1) * cpw);       // this wave's centres [j, ce)
     const int64_t rc = ri < nrows ? ri : nrows - 1;
     const int64_t row = sm > 0 ? linspace_round(nq - 1, sm, rc) : rc;
     const int64_t base = ((int64_t)h * nq + row) * D;
@@ -4230,8 +4237,8 @@ __global__ __launch_bounds__(256) void km_assign_kernel(const void* __restrict__
             bj = j;
         }
     };
-    int j = 0;
-    for (; j + 3 < C; j += 4) {
+    int j = NS == 1 ? 0 : wv * cpw;
+    for (; j + 3 < ce; j += 4) {
         const float* c0 = ch + (int64_t)j * D;
         float a[4];
 #pragma unroll
@@ -4247,7 +4254,7 @@ __global__ __launch_bounds__(256) void km_assign_kernel(const void* __restrict__
 #pragma unroll
         for (int u = 0; u < 4; ++u) consider(a[u], j + u);
     }
-    for (; j + 1 < C; j += 2) {
+    for (; j + 1 < ce; j += 2) {
         const float* c0 = ch + (int64_t)j * D;
         const float* c1 = c0 + D;
         float a0 = 0.0f, a1 = 0.0f;
@@ -4260,7 +4267,7 @@ __global__ __launch_bounds__(256) void km_assign_kernel(const void* __restrict__
         consider(a0, j);
         consider(a1, j + 1);
     }
-    if (j < C) {                        // an odd last centre
+    if (j < ce) {                       // an odd last centre
         const float* c0 = ch + (int64_t)j * D;
         float a0 = 0.0f;
 #pragma unroll
@@ -4269,6 +4276,16 @@ __global__ __launch_bounds__(256) void km_assign_kernel(const void* __restrict__
             a0 = __fadd_rn(a0, __fmul_rn(e0, e0));
         }
         consider(a0, j);
+    }
+    if constexpr (NS > 1) {             // the waves' nearest centres, in centre order (ties: the lower)
+        __shared__ float sb[NS][64];
+        __shared__ int sj[NS][64];
+        sb[wv][tid & 63] = best;
+        sj[wv][tid & 63] = bj;
+        __syncthreads();
+        if (wv > 0) return;
+#pragma unroll
+        for (int u = 1; u < NS; ++u) consider(sb[u][tid], sj[u][tid]);
     }
     if (bj >= C) bj = 0;                // no finite distance (non-finite rows): centre 0
     if (ri < nrows) assign[(int64_t)h * nq + ri] = bj;
@@ -4334,6 +4351,71 @@ __global__ __launch_bounds__(128) void km_update_kernel(const void* __restrict__
         }
     }
     if (cnt > 0) cen[((int64_t)h * C + j) * D + tid] = __fdiv_rn(acc, (float)cnt);
+}
+
+// The same for few centres in flight (heads x clusters <= KM_WIDE): eight waves per centre list its samples,
+// each its own run of the sample, and gather 64 rows at a time into one of two LDS buffers, the next
+// 64 on their way while lane d sums dim d of the current ones in list order.  With a centre on every CU the other
+// kernel's two waves hide each other's gathers (24 heads: 45 us; staged rows were slower there); with one head's 32 centres on 256
+// CUs each gather's latency stood alone: 16.7 -> 9.8 us.
+constexpr int KM_WIDE = 256;
+template <bool IN_BF16>
+__global__ __launch_bounds__(512) void km_update_wide_kernel(const void* __restrict__ q, int64_t nq, int m, int C,
+                                                             const int32_t* __restrict__ assign,
+                                                             float* __restrict__ cen) {
+    constexpr int B = 64, PR = IN_BF16 ? 16 : 32, NL = B * PR / 512;   // 16-byte pieces per row, loads per thread
+    __shared__ uint16_t list[KM_MAX_SAMPLE];
+    __shared__ __align__(16) uint32_t buf[2][B * PR * 4];
+    __shared__ int wcnt[8];
+    const int j = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int32_t* a = assign + (int64_t)h * nq;
+    const int per = ((m + 7) / 8 + 63) / 64 * 64, s0 = min(m, w * per), s1 = min(m, s0 + per);
+    int n = 0;
+#pragma unroll 8
+    for (int i = s0; i < s1; i += 64) n += __popcll(__ballot(i + lane < s1 && a[min(i + lane, s1 - 1)] == j));
+    if (lane == 0) wcnt[w] = n;
+    __syncthreads();
+    int at = 0, cnt = 0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        if (u < w) at += wcnt[u];
+        cnt += wcnt[u];
+    }
+#pragma unroll 8
+    for (int i = s0; i < s1; i += 64) {
+        const bool hit = i + lane < s1 && a[min(i + lane, s1 - 1)] == j;
+        const uint64_t bal = __ballot(hit);
+        if (hit) list[at + __popcll(bal & ((1ull << lane) - 1ull))] = (uint16_t)(i + lane);
+        at += __popcll(bal);
+    }
+    __syncthreads();
+    if (cnt == 0) return;                          // a centre without samples keeps its position
+    u32x4 r[NL];
+    auto load = [&](int k0) {                      // rows past the list repeat its last one
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+            const int e = 512 * u + tid, row = min(k0 + e / PR, cnt - 1);
+            const int64_t src = ((int64_t)h * nq + linspace_round(nq - 1, m, list[row])) * (PR * 4);
+            r[u] = *(const u32x4*)((const uint32_t*)q + src + 4 * (e % PR));
+        }
+    };
+    load(0);
+    float acc = 0.0f;
+    for (int k0 = 0, p = 0; k0 < cnt; k0 += B, p ^= 1) {
+#pragma unroll
+        for (int u = 0; u < NL; ++u) *(u32x4*)(&buf[p][4 * (512 * u + tid)]) = r[u];
+        __syncthreads();                           // (the buffer's readers of two steps ago passed the last barrier)
+        if (k0 + B < cnt) load(k0 + B);
+        if (tid < D) {
+            const int e = min(B, cnt - k0);
+#pragma unroll 16
+            for (int u = 0; u < e; ++u) {
+                const float x = IN_BF16 ? bf2f(((const uint16_t*)&buf[p][u * PR * 4])[tid]) : __uint_as_float(buf[p][u * PR * 4 + tid]);
+                acc = __fadd_rn(acc, x);
+            }
+        }
+    }
+    if (tid < D) cen[((int64_t)h * C + j) * D + tid] = __fdiv_rn(acc, (float)cnt);
 }
 
 // perm = the rows ordered by centre, the rows of one centre in row order: a stable counting sort
@@ -5564,19 +5646,37 @@ int htrc_kmeans_order(const void* q, int q_is_bf16, int64_t heads, int64_t nq, i
     REQUIRE(m <= KM_MAX_SAMPLE, "htrc_kmeans_order: at most 16384 sample rows");
     hipStream_t s = (hipStream_t)stream;
     const dim3 gc((unsigned)clusters, (unsigned)heads);
-    const dim3 gs((unsigned)((m + 255) / 256), (unsigned)heads), ga((unsigned)((nq + 255) / 256), (unsigned)heads);
-#define KM_LAUNCH(BF)                                                                                              \
-    hipLaunchKernelGGL(km_init_kernel<BF>, gc, dim3(D), 0, s, q, nq, (int)m, clusters, centres);                 \
-    for (int it = 0; it < iters; ++it) {                                                                           \
-        hipLaunchKernelGGL(km_assign_kernel<BF>, gs, dim3(256), 0, s, q, nq, m, (int)m, clusters, centres, assign); \
-        hipLaunchKernelGGL(km_update_kernel<BF>, gc, dim3(D), 0, s, q, nq, (int)m, clusters, assign, centres);    \
-    }                                                                                                              \
-    hipLaunchKernelGGL(km_assign_kernel<BF>, ga, dim3(256), 0, s, q, nq, nq, 0, clusters, centres, assign);
+    const bool wide = heads * clusters <= KM_WIDE;
+    // at most a wave per SIMD by rows alone: the centres split over four waves per 64 rows, or eight
+#define KM_ASSIGN_NS(BF, NS, ROWS, SM)                                                                                \
+    hipLaunchKernelGGL((km_assign_kernel<BF, NS>),                                                                    \
+                       dim3((unsigned)(NS == 1 ? (ROWS + 255) / 256 : (ROWS + 63) / 64), (unsigned)heads),             \
+                       dim3(NS == 1 ? 256 : 64 * NS), 0, s, q, nq, ROWS, SM, clusters, centres, assign);
+#define KM_ASSIGN(BF, ROWS, SM)                                                                                       \
+    if (heads * ((ROWS + 63) / 64) <= device_cus()) {                                                                 \
+        KM_ASSIGN_NS(BF, 8, ROWS, SM)                                                                                 \
+    } else if (heads * ((ROWS + 63) / 64) <= 4 * device_cus()) {                                                      \
+        KM_ASSIGN_NS(BF, 4, ROWS, SM)                                                                                 \
+    } else {                                                                                                          \
+        KM_ASSIGN_NS(BF, 1, ROWS, SM)                                                                                 \
+    }
+#define KM_LAUNCH(BF)                                                                                                 \
+    hipLaunchKernelGGL(km_init_kernel<BF>, gc, dim3(D), 0, s, q, nq, (int)m, clusters, centres);                      \
+    for (int it = 0; it < iters; ++it) {                                                                              \
+        KM_ASSIGN(BF, m, (int)m)                                                                                      \
+        if (wide)                                                                                                     \
+            hipLaunchKernelGGL(km_update_wide_kernel<BF>, gc, dim3(512), 0, s, q, nq, (int)m, clusters, assign, centres); \
+        else                                                                                                          \
+            hipLaunchKernelGGL(km_update_kernel<BF>, gc, dim3(D), 0, s, q, nq, (int)m, clusters, assign, centres);    \
+    }                                                                                                                 \
+    KM_ASSIGN(BF, nq, 0)
     if (q_is_bf16) {
         KM_LAUNCH(true)
     } else {
         KM_LAUNCH(false)
     }
+#undef KM_ASSIGN
+#undef KM_ASSIGN_NS
 #undef KM_LAUNCH
     // the sort's per-range counts go to the centres workspace, spent once the last assignment
     // has run: at most KM_SORT_RANGES * clusters <= clusters * D words per head
