@@ -992,22 +992,28 @@ __global__ __launch_bounds__(256) void select_kernel(const int8_t* __restrict__ 
 // compaction (ties at the threshold go to the lower leaf index).  Leaves < sink are
 // forced in (h3/htrc_flat.py:262-265).  Used by the topk kernel and the fused route kernel.
 // ---------------------------------------------------------------------------------------------
+template <int NTH = 256>      // threads of the workgroup
 struct TopkSmem {
     uint32_t hist[256];
-    uint32_t cnt_gt[257];
-    uint32_t cnt_eq[257];
+    uint32_t cnt_gt[NTH + 1];
+    uint32_t cnt_eq[NTH + 1];
     uint32_t prefix, remaining;
 };
 
-// Small kx (<= 64), idx only: the same set as the radix select below, from a lower bound of the
+// Small kx (<= TOPK_SMALL), idx only: the same set as the radix select below, from a lower bound of the
 // threshold.  Wave 0 takes the maxima of the 64 strided subsets l = j (mod 64) and sorts them
 // (bitonic, across the lanes); the kx-th largest, L, has kx subsets holding a key >= L, so at
 // least kx keys are >= L and the kx-th largest key is too.  The keys >= L (a few more than kx
 // for score rows) are compacted in leaf order and each is ranked exactly: keys above it, and
 // equal keys at lower leaves.  More than 256 candidates (many equal keys): returns false before
-// anything is written, and the radix select runs.  Five barriers, every thread through each.
-template <typename Keys>
-__device__ bool topk_small(Keys keys, int nb, int kx, TopkSmem& sm, int32_t* idx_out) {
+// anything is written, and the radix select runs.  Every thread passes every barrier.  64 subsets
+// bring 64 ln(64 / (64 - kx)) candidates, 44 at kx = 32 and 300 at 64, so above TOPK_SMALL the radix select
+// runs at once: the fp8 select of 12 x 504 tiles x 1008 leaves 218 us at kx = 32, 235 at 56 and 261 at 64, against
+// 232 by the radix select (256 subsets ranked in LDS: 262 at 64).
+constexpr int TOPK_SMALL = 48;
+template <int NTH, typename Keys>
+__device__ bool topk_small(Keys keys, int nb, int kx, TopkSmem<NTH>& sm, int32_t* idx_out) {
+    constexpr int NWV = NTH / 64;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     uint32_t* ck = sm.hist;        // candidate keys
     uint32_t* cl = sm.cnt_gt;      // candidate leaves
@@ -1026,7 +1032,7 @@ __device__ bool topk_small(Keys keys, int nb, int kx, TopkSmem& sm, int32_t* idx
     }
     __syncthreads();
     const uint32_t lb = sm.prefix;
-    const int chunk = (nb + 255) / 256;
+    const int chunk = (nb + NTH - 1) / NTH;
     const int a = min(nb, tid * chunk), b = min(nb, a + chunk);
     uint32_t n = 0;
     for (int l = a; l < b; ++l) n += keys(l) >= lb;
@@ -1040,7 +1046,7 @@ __device__ bool topk_small(Keys keys, int nb, int kx, TopkSmem& sm, int32_t* idx
     __syncthreads();
     uint32_t off = incl - n, nc = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < NWV; ++j) {
         const uint32_t c = sm.cnt_eq[j];
         if (j < wv) off += c;
         nc += c;
@@ -1069,10 +1075,10 @@ __device__ bool topk_small(Keys keys, int nb, int kx, TopkSmem& sm, int32_t* idx
         leaf = cl[tid];
     }
     const uint64_t bal = __ballot(sel);   // output position: selected candidates before this one
-    if (lane == 0) sm.cnt_eq[4 + wv] = (uint32_t)__popcll(bal);
+    if (lane == 0) sm.cnt_eq[NWV + wv] = (uint32_t)__popcll(bal);
     __syncthreads();
     uint32_t pos = (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
-    for (int j = 0; j < wv; ++j) pos += sm.cnt_eq[4 + j];
+    for (int j = 0; j < wv; ++j) pos += sm.cnt_eq[NWV + j];
     if (sel) idx_out[pos] = (int32_t)leaf;
     __syncthreads();
     return true;
@@ -1080,12 +1086,12 @@ __device__ bool topk_small(Keys keys, int nb, int kx, TopkSmem& sm, int32_t* idx
 
 // keys(l) is order_key(sel[l]) for l < nb (an LDS array, or computed from global memory for rows
 // longer than the LDS holds).  Writes idx[0..kx) ascending and (optionally) excl.
-template <typename Keys>
-__device__ void topk_row(Keys keys, int nb, int kx, TopkSmem& sm, int32_t* idx_out,
+template <int NTH, typename Keys>
+__device__ void topk_row(Keys keys, int nb, int kx, TopkSmem<NTH>& sm, int32_t* idx_out,
                          int8_t* excl_out, int32_t* idx_lds) {
     const int tid = threadIdx.x;
     if (kx >= nb) {               // everything is selected
-        for (int l = tid; l < nb; l += 256) {
+        for (int l = tid; l < nb; l += NTH) {
             if (idx_out) idx_out[l] = l;
             if (idx_lds) idx_lds[l] = l;
             if (excl_out) excl_out[l] = 1;
@@ -1093,17 +1099,17 @@ __device__ void topk_row(Keys keys, int nb, int kx, TopkSmem& sm, int32_t* idx_o
         __syncthreads();
         return;
     }
-    if (kx <= 64 && idx_out && !excl_out && !idx_lds && topk_small(keys, nb, kx, sm, idx_out)) return;
+    if (kx <= TOPK_SMALL && idx_out && !excl_out && !idx_lds && topk_small<NTH>(keys, nb, kx, sm, idx_out)) return;
     if (tid == 0) {
         sm.prefix = 0;
         sm.remaining = (uint32_t)kx;
     }
     uint32_t mask = 0;
     for (int shift = 24; shift >= 0; shift -= 8) {
-        sm.hist[tid] = 0;
+        if (tid < 256) sm.hist[tid] = 0;
         __syncthreads();
         const uint32_t prefix = sm.prefix;
-        for (int l = tid; l < nb; l += 256) {
+        for (int l = tid; l < nb; l += NTH) {
             const uint32_t key = keys(l);
             if ((key & mask) == prefix) atomicAdd(&sm.hist[(key >> shift) & 255u], 1u);
         }
@@ -1140,7 +1146,7 @@ __device__ void topk_row(Keys keys, int nb, int kx, TopkSmem& sm, int32_t* idx_o
     }
     const uint32_t thr = sm.prefix, need_eq = sm.remaining;
     // ascending compaction: thread owns a contiguous chunk of leaves
-    const int chunk = (nb + 255) / 256;
+    const int chunk = (nb + NTH - 1) / NTH;
     const int a = min(nb, tid * chunk), b = min(nb, a + chunk);
     uint32_t ngt = 0, neq = 0;
     for (int l = a; l < b; ++l) {
@@ -1148,7 +1154,7 @@ __device__ void topk_row(Keys keys, int nb, int kx, TopkSmem& sm, int32_t* idx_o
         ngt += key > thr;
         neq += key == thr;
     }
-    {   // exclusive prefix over the 256 threads: in-wave inclusive scan, then wave offsets
+    {   // exclusive prefix over the threads: in-wave inclusive scan, then wave offsets
         const int lane = tid & 63, wv = tid >> 6;
         uint32_t ig = ngt, ie = neq;
 #pragma unroll
@@ -1203,16 +1209,16 @@ __global__ __launch_bounds__(256) void topk_kernel(const float* __restrict__ sel
                                                    int kx, int sink, int32_t* __restrict__ idx,
                                                    int8_t* __restrict__ excl) {
     __shared__ uint32_t keys[LDS_KEYS ? MAX_NB_LDS : 1];
-    __shared__ TopkSmem sm;
+    __shared__ TopkSmem<> sm;
     const int64_t row = blockIdx.x;
     const float* srow = sel + row * nb_pad;
     for (int l = nb + threadIdx.x; l < nb_pad; l += 256) excl[row * nb_pad + l] = 0;
     if constexpr (LDS_KEYS) {
         for (int l = threadIdx.x; l < nb; l += 256) keys[l] = l < sink ? 0xffffffffu : order_key(srow[l]);
         __syncthreads();
-        topk_row([&](int l) { return keys[l]; }, nb, kx, sm, idx + row * kx, excl + row * nb_pad, nullptr);
+        topk_row<256>([&](int l) { return keys[l]; }, nb, kx, sm, idx + row * kx, excl + row * nb_pad, nullptr);
     } else {
-        topk_row([&](int l) { return l < sink ? 0xffffffffu : order_key(srow[l]); }, nb, kx, sm, idx + row * kx,
+        topk_row<256>([&](int l) { return l < sink ? 0xffffffffu : order_key(srow[l]); }, nb, kx, sm, idx + row * kx,
                  excl + row * nb_pad, nullptr);
     }
 }
@@ -2596,20 +2602,23 @@ __device__ __forceinline__ void dma_rows27(const uint16_t* x0, const uint16_t* x
 // LDS, for rows of more leaves than the LDS holds.  The launch covers tile groups
 // [g0, g0 + ng) of each head; the state rows and idx are the launch's own ([H, ng, ...]).
 constexpr int SEL_RING = 3;                         // route_select ring slots per wave
+// NW waves per workgroup: the leaf groups are dealt over them, so a launch of few tile groups takes 8 or 16 (the
+// device has four SIMDs a CU whatever the groups are): 128 groups of 2547 leaves (kx 256) 42 -> 28.6 us.  With fewer
+// leaves than eight 16-leaf groups a wave the extra waves cost more in barriers (256 leaves: 11.3 us at 4 waves, 13.1 at 16).
 constexpr int ROUTE_NB_LDS = 16384;                 // leaves per head whose keys route_select keeps in LDS
-template <bool MULTI, int NRB, bool GK>
-__global__ __launch_bounds__(256, 4) void route_select_kernel(
+template <bool MULTI, int NRB, bool GK, int NW>
+__global__ __launch_bounds__(64 * NW, 4) void route_select_kernel(
     const int8_t* __restrict__ dq8, const float* __restrict__ sdq, const int8_t* __restrict__ g8,
     const float* __restrict__ sg, const float* __restrict__ lz, int nt, int group, int g0, int ng, int nb,
     int nb_pad, int kx, int sink, int stride, int32_t* __restrict__ idx, float* __restrict__ rowmax,
     uint32_t* __restrict__ keys_ws) {
     extern __shared__ uint32_t keys_lds[];    // [nb] unless GK
-    __shared__ TopkSmem sm;
-    __shared__ float red_m[4][64];
+    __shared__ TopkSmem<64 * NW> sm;
+    __shared__ float red_m[NW][64];
     // each wave's own ring of 16-leaf groups: g8 rows as the two 1 KB QK operand chunks
     // (kss = 0, 1; lane-linear), then sg (64 B) and lz (64 B)
     constexpr int SEL_SLOT = 2048 + 128;
-    __shared__ __align__(16) char sring[4][SEL_RING][SEL_SLOT];
+    __shared__ __align__(16) char sring[NW][SEL_RING][SEL_SLOT];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
     // one workgroup per tile group (G tiles sharing a centre, state and near leaves; G = 1: a tile)
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
@@ -2624,11 +2633,11 @@ __global__ __launch_bounds__(256, 4) void route_select_kernel(
     };
     const uint32_t ring_lds = lds_addr(&sring[w][0][0]);
     const uint32_t voff0 = (uint32_t)(col * D + 16 * grp), voff1 = voff0 + 64;
-    // group gj of this wave (leaves c = 16 w + 64 gj ..) into ring slot gj % SEL_RING: three
+    // group gj of this wave (leaves c = 16 w + 16 NW gj ..) into ring slot gj % SEL_RING: three
     // direct loads; lane (col, grp) of operand chunk kss gets bytes 64 kss + 16 grp of row col
     auto sel_issue = [&](int gj, int ngr) {
         if (gj >= ngr) return;
-        const int64_t s0 = gs * nb_pad + 16 * w + 64 * gj;
+        const int64_t s0 = gs * nb_pad + 16 * w + 16 * NW * gj;
         const uint32_t slot = ring_lds + (uint32_t)(gj % SEL_RING) * SEL_SLOT;
         dma16s<SEL_NT>(g8 + s0 * D, voff0, slot);
         dma16s<SEL_NT>(g8 + s0 * D, voff1, slot + 1024);
@@ -2691,8 +2700,8 @@ __global__ __launch_bounds__(256, 4) void route_select_kernel(
             // otherwise drain the ring
             asm volatile("" : : "v"(b[rb][0]), "v"(b[rb][1]), "v"(srow[rb]));
         }
-        // wave w: 16-leaf groups c = 16 w + 64 gj through its ring, loaded SEL_RING - 1 ahead
-        const int ngr = 16 * w < nb ? (nb - 16 * w + 63) / 64 : 0;
+        // wave w: 16-leaf groups c = 16 w + 16 NW gj through its ring, loaded SEL_RING - 1 ahead
+        const int ngr = 16 * w < nb ? (nb - 16 * w + 16 * NW - 1) / (16 * NW) : 0;
 #pragma unroll
         for (int gj = 0; gj < SEL_RING - 1; ++gj) sel_issue(gj, ngr);
         for (int gj = 0; gj < ngr; ++gj) {
@@ -2701,7 +2710,7 @@ __global__ __launch_bounds__(256, 4) void route_select_kernel(
             SelOps o;
             sel_read(o, gj);
             sel_issue(gj + SEL_RING - 1, ngr);       // into the slot of group gj - 1, read last iteration
-            sel_block(o, 16 * w + 64 * gj);
+            sel_block(o, 16 * w + 16 * NW * gj);
         }
 #pragma unroll
         for (int rb = 0; rb < NRB; ++rb) {    // row r = stride * (16 rb + col) of the sampled rows
@@ -2711,7 +2720,11 @@ __global__ __launch_bounds__(256, 4) void route_select_kernel(
         __syncthreads();
         if (w == 0) {
             const int r = lane;
-            float m = r < ts ? fmaxf(fmaxf(red_m[0][r], red_m[1][r]), fmaxf(red_m[2][r], red_m[3][r])) : -INFINITY;
+            float m = -INFINITY;
+            if (r < ts) {
+#pragma unroll
+                for (int u = 0; u < NW; ++u) m = fmaxf(m, red_m[u][r]);
+            }
             if (stride != 1) m = wave_max(m); // sampled rows: one reference for the whole tile
             if (r < TR) rowmax[th * TR + r] = m;
         }
@@ -2719,7 +2732,7 @@ __global__ __launch_bounds__(256, 4) void route_select_kernel(
         first = false;
     }
     const int kxe = min(kx, nb);
-    if (kxe > 0) topk_row([&](int l) { return keys[l]; }, nb, kxe, sm, idx + gs * kxe, nullptr, nullptr);
+    if (kxe > 0) topk_row<64 * NW>([&](int l) { return keys[l]; }, nb, kxe, sm, idx + gs * kxe, nullptr, nullptr);
 }
 
 // The lane index computed anew (not from a register held since the kernel's start): code after a
@@ -3390,7 +3403,7 @@ __global__ __launch_bounds__(256, 3) void route_select16_kernel(
     const float* __restrict__ lz, int nt, int group, int g0, int ng, int nb, int nb_pad, int kx, int sink,
     int stride, int32_t* __restrict__ idx, float* __restrict__ rowmax) {
     extern __shared__ uint32_t keys16[];      // [nb]
-    __shared__ TopkSmem sm;
+    __shared__ TopkSmem<> sm;
     __shared__ float red_m[4][64];
     constexpr int S16_RING = 3, S16_SLOT = 2048 + 128;
     __shared__ __align__(16) char s16ring[4][FP8 ? S16_RING : 1][FP8 ? S16_SLOT : 16];
@@ -3537,7 +3550,7 @@ __global__ __launch_bounds__(256, 3) void route_select16_kernel(
         first = false;
     }
     const int kxe = min(kx, nb);
-    if (kxe > 0) topk_row([&](int l) { return keys16[l]; }, nb, kxe, sm, idx + gs * kxe, nullptr, nullptr);
+    if (kxe > 0) topk_row<256>([&](int l) { return keys16[l]; }, nb, kxe, sm, idx + gs * kxe, nullptr, nullptr);
 }
 
 // One ring slot of route16_kernel: QK rows and PV rows, 32 rows of 128 16-bit values each, then
@@ -5264,6 +5277,11 @@ static int route_shapes(const char* who, int64_t heads, int64_t nq, int64_t nk, 
     return HTRC_OK;
 }
 
+// Static LDS of route_select_kernel with nw waves: the rings, the row maxima and the top-k's tables.
+static size_t route_select_static_bytes(int nw) {
+    return (size_t)nw * (SEL_RING * 2176 + 256) + 4 * (256 + 2 * ((size_t)64 * nw + 1) + 2) + 64;
+}
+
 int htrc_route_select(const int8_t* dq8, const float* sdq, const int8_t* g8, const float* sg, const float* lz,
                       int64_t heads, int64_t nq, int64_t nk, int leaf, int d, int kx, int sink, int stride,
                       int tile, int group, int64_t g0, int64_t gn, int32_t* idx, float* rowmax, uint32_t* keys_ws,
@@ -5282,12 +5300,18 @@ int htrc_route_select(const int8_t* dq8, const float* sdq, const int8_t* g8, con
     REQUIRE(!gk || keys_ws, "htrc_route_select: keys_ws [H, gn, nb_pad] is required above 16384 leaves per head");
     const int nbp = htrc_nb_pad(nb);
     const size_t dyn = gk ? 0 : (size_t)4 * nbp;
-#define RSEL(M, N, G)                                                                                           \
-    hipLaunchKernelGGL((route_select_kernel<M, N, G>), dim3((unsigned)(gn * heads)), dim3(256), dyn,             \
+    // waves per group: four where the groups alone give every SIMD two waves or a wave would have fewer than eight
+    // 16-leaf groups, more below that (the keys in global memory: heads of many leaves, four)
+    const int64_t cus = device_cus();
+    int nw = gk || nb < 1024 || gn * heads > 2 * cus ? 4 : (nb < 2048 || gn * heads > cus ? 8 : 16);
+    if (nw == 16 && route_select_static_bytes(16) + dyn > ROUTE_LDS_MAX) nw = 8;   // (11 k leaves beside 16 rings)
+#define RSEL(M, N, G, NW)                                                                                       \
+    hipLaunchKernelGGL((route_select_kernel<M, N, G, NW>), dim3((unsigned)(gn * heads)), dim3(64 * NW), dyn,     \
                        (hipStream_t)stream, dq8, sdq, g8, sg, lz, (int)nt, group, (int)g0, (int)gn, (int)nb, nbp, kxe, \
                        sink, stride, idx, rowmax, keys_ws)
 #define RSEL_G(M, N) \
-    if (gk) RSEL(M, N, true); else RSEL(M, N, false);
+    if (gk) RSEL(M, N, true, 4); else if (nw == 4) RSEL(M, N, false, 4); else if (nw == 8) RSEL(M, N, false, 8); \
+    else RSEL(M, N, false, 16);
     if (tile == 64) {
         if (group == 1) { RSEL_G(false, 4) } else { RSEL_G(true, 4) }
     } else {

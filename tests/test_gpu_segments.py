@@ -65,3 +65,37 @@ def test_segmented_route(device, n, m, leaf, kx, tile, heads, group, spike, segs
     assert bool(torch.isfinite(o1).all()) and bool(torch.isfinite(z1).all())
     assert float((o1 - o3).norm() / o3.norm()) <= 1e-5
     assert float(((z1 - z3).abs() / z3.abs().clamp_min(1.0)).max()) <= 1e-5
+
+
+@pytest.mark.parametrize("groups,nb,kx,sink,group", [
+    (300, 1008, 64, 0, 1), (40, 2547, 256, 0, 1), (40, 2547, 476, 220, 1), (300, 300, 128, 3, 1), (40, 130, 129, 0, 2), (300, 1500, 49, 0, 1), (300, 1500, 48, 0, 1),
+    (600, 500, 57, 0, 1), (600, 1008, 56, 0, 1), (3, 12000, 100, 0, 1), (3, 11264, 129, 0, 1), (20, 257, 128, 0, 1),
+    (20, 66, 60, 0, 1)])
+@pytest.mark.parametrize("ties", [False, True])
+def test_route_select_wave_counts(device, groups, nb, kx, sink, group, ties):
+    """route_select's launches of 4, 8 and 16 waves per tile group (more than 512, 257 to 512, fewer groups; heads
+    whose keys leave no room for 16 rings), and its top-k at and beside each bound of its methods: index sets
+    equal to the stage select and top-k on the same state, row maxima to a 4-wave launch's."""
+    torch.manual_seed(nb + kx)
+    nbp, nt = -(-nb // 32) * 32, groups * group
+    dq8 = torch.randint(-127, 128, (1, nt * 64, 128), device=device, dtype=torch.int8)
+    sdq = torch.rand((1, nt * 64), device=device) * 1e-4
+    g8 = torch.randint(-127, 128, (1, groups, nbp, 128), device=device, dtype=torch.int8)
+    sg, lz = torch.rand((1, groups, nbp), device=device), torch.randn((1, groups, nbp), device=device)
+    if ties:
+        g8.zero_()
+        lz = torch.round(lz)
+    sg[..., nb:], lz[..., nb:] = 0, -math.inf
+    g8[..., nb:, :] = 0
+    packed = {"dq8": dq8, "sdq": sdq, "k8": torch.empty((1, nb * 16, 128), device=device, dtype=torch.int8)}
+    state = {"g8": g8, "sg": sg, "lz": lz}
+    idx, rowmax = hip.route_select(packed, state, nq=nt * 64, leaf=16, kx=kx, sink=sink, group=group)
+    sel = hip.rowmax_select(g=g8, lz=lz, sg=sg, nb=nb, dq8=dq8, sdq=sdq, group=group)
+    want, _ = hip.topk_excl(sel, nb, kx, sink)
+    assert torch.equal(idx, want)
+    # the same groups inside a window: the launch's first groups alone
+    few = min(groups, 2)
+    part = {k: x[:, :few].contiguous() for k, x in state.items()}
+    idx2, rowmax2 = hip.route_select(packed, part, nq=nt * 64, leaf=16, kx=kx, sink=sink, group=group)
+    rows = few * group * 64
+    assert torch.equal(idx2, idx[:, :few]) and torch.equal(rowmax2[:, :rows], rowmax[:, :rows])
