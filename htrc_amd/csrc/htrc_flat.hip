@@ -2581,11 +2581,14 @@ template <bool NT>
 __device__ __forceinline__ void dma_rows01(const uint16_t* x0, const BlockOffsets& bo, uint32_t slot) {
     dma_x2<NT>(sbase(x0), bo.rows[0], sbase(x0, 1024), bo.rows[1], slot + 4096);
 }
-// chunks 2..7:
+// chunks 2, 3:
 template <bool NT>
-__device__ __forceinline__ void dma_rows27(const uint16_t* x0, const uint16_t* x1, const BlockOffsets& bo,
-                                           uint32_t slot) {
+__device__ __forceinline__ void dma_rows23(const uint16_t* x0, const BlockOffsets& bo, uint32_t slot) {
     dma_x2<NT>(sbase(x0), bo.rows[2], sbase(x0, 1024), bo.rows[3], slot + 4096 + 2048);
+}
+// chunks 4..7:
+template <bool NT>
+__device__ __forceinline__ void dma_rows47(const uint16_t* x1, const BlockOffsets& bo, uint32_t slot) {
     dma_x4<NT>(sbase(x1), bo.rows[0], sbase(x1, 1024), bo.rows[1], sbase(x1, 2048), bo.rows[2], sbase(x1, 3072),
            bo.rows[3], slot + 8192);
 }
@@ -2800,6 +2803,7 @@ __device__ __forceinline__ RowMax<RB> route_exact_max(const int8_t* dq8, const f
         bq[rb][1] = *(const i32x4*)(q8 + p * D + 64 + 16 * grp);
         srow[rb] = __fmul_rn(__fmul_rn(sq[p], scale), LOG2E);
     }
+    e_lo = __builtin_amdgcn_readfirstlane(e_lo);
     asm volatile("" : "+s"(e_lo));                // (its LDS address likewise)
     for (int j = e_lo; j < e_hi; j += 16) {       // 16-token runs of the near leaves
         const int64_t tok = kh + (int64_t)__builtin_amdgcn_readfirstlane(sidx[j / LEAF]) * LEAF + (j % LEAF);
@@ -2827,11 +2831,11 @@ __device__ __forceinline__ RowMax<RB> route_exact_max(const int8_t* dq8, const f
 // Measured on heads of 40759 tokens (leaf 16): a 128-tile window of 208 blocks 178 us whole (one wave
 // pair a tile: 256 waves for 1024 SIMDs), 50 + 22 us in parts (the head 965 -> 706 us a call); 256 tiles
 // of 592 blocks 507 -> 270 + 30 us; 768 tiles of 318 blocks 605 whole, 587 + 92 in parts, 556 in turn,
-// so launches of more than 512 tiles run in turn.  4 segments against 6, 8 and 16: 706 / 715 / 720 /
+// so launches of more than 384 tiles run in turn (384 tiles split 1521, in turn 1559 us a call; 512 1983 and 1911).  4 segments against 6, 8 and 16: 706 / 715 / 720 /
 // 720 us.  Below 128 blocks the whole-tile kernels' key halves and quarters serve.
 constexpr int SEG_MIN_BLOCKS = 128;
 constexpr int SEG_MAX = 4;
-constexpr int64_t SEG_SPLIT_TILES = 512;             // launches of at most this many tiles run the segments apart
+constexpr int64_t SEG_SPLIT_TILES = 384;             // launches of at most this many tiles run the segments apart
 enum RouteMode { ROUTE_WHOLE = 0, ROUTE_PART = 1, ROUTE_SEGS = 2 };
 constexpr int SEG_QUARTERS = 4;                      // workgroups per tile that combine its partial sums
 
@@ -2843,12 +2847,12 @@ inline int route_segments(int64_t nb, int kxe, int leaf) {
     return (int)(n < SEG_MAX ? n : SEG_MAX);
 }
 
-// RB = tile / 32: 16-row blocks per wave (tiles of 64 or 32 rows); NP wave pairs split the keys;
-// RS ring slots per pair.  MODE ROUTE_WHOLE: the tile's keys in one sum.  ROUTE_PART: workgroup
+// RB 16-row blocks per wave, NH waves per key part (NH = 2: halves of the tile's rows; NH = 4, RB = 1: quarters of
+// a 64-row tile, the same sums per row); NP key parts of NH waves; RS ring slots per part.  MODE ROUTE_WHOLE: the tile's keys in one sum.  ROUTE_PART: workgroup
 // (tile, segment), the segment's O and row sums to part_o / part_l [tile of the launch][segment].
 // ROUTE_SEGS: with part_o, SEG_QUARTERS workgroups per tile add the tile's partial sums (the redo of a
 // tile whose reference missed is the first one's); without, one workgroup runs the segments in turn.
-template <int LEAF, int RB, int NP, int RS, int MODE>
+template <int LEAF, int RB, int NP, int RS, int MODE, int NH>
 __device__ __forceinline__ void route_body(
     const int8_t* __restrict__ q8, const float* __restrict__ sq, const int8_t* __restrict__ dq8,
     const float* __restrict__ sdq, const int8_t* __restrict__ g8, const float* __restrict__ sg,
@@ -2857,8 +2861,9 @@ __device__ __forceinline__ void route_body(
     const float* __restrict__ rowmax, int64_t nq, int nt, int group, int g0, int ng, const int32_t* __restrict__ perm,
     int64_t nk, int nb, int nb_pad, int kxe, float scale, float* __restrict__ out, float* __restrict__ logz,
     float* __restrict__ part_o, float* __restrict__ part_l, int nseg) {
-    static_assert(MODE == ROUTE_WHOLE || NP == 1, "segments run on one wave pair");
-    constexpr int NT = 128 * NP;                               // threads
+    static_assert(MODE == ROUTE_WHOLE || NP == 1, "segments run on one key part");
+    static_assert(NH == 2 || (NH == 4 && RB == 1), "row parts");
+    constexpr int NT = 64 * NH * NP;                           // threads
     __shared__ __align__(16) char ring[NP][RS][SLOT_BYTES];    // one per wave pair; also merge staging
     // sized by the launch: exclusion bits [nb / 32 + 1], then the tile's near leaves [kxe], so
     // small shapes leave room for more tiles per CU
@@ -2867,15 +2872,15 @@ __device__ __forceinline__ void route_body(
     uint32_t* sidx = route_dyn + (nb / 32 + 1);
     __shared__ float red_m[64], red_l[NP][64];
     __shared__ int redo;
-    constexpr int TR = 32 * RB;                                // rows per tile
-    // merge staging in the ring: all rows at once, or one row half (one wave of each pair) at a time
+    constexpr int TR = 16 * RB * NH;                           // rows per tile
+    // merge staging in the ring: all rows at once, or one row half (half the waves of each part) at a time
     constexpr bool MRG2 = NP * TR * MRG_STRIDE * 4 > NP * RS * SLOT_BYTES;
     constexpr int RR = MRG2 ? TR / 2 : TR;                     // rows per merge round
     static_assert(NP * RR * MRG_STRIDE * 4 <= NP * RS * SLOT_BYTES, "merge staging");
     float* mrg = (float*)&ring[0][0][0];                       // merge staging: NP x 64 x MRG_STRIDE floats
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: scalar bookkeeping
     const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
-    const int pr = wv % NP, hr = wv / NP;                      // key part (wave pair), row half
+    const int pr = wv % NP, hr = wv / NP;                      // key part, row part
     auto row_total = [&](int r) {                              // a row's sum over the NP parts
         if constexpr (NP == 4)
             return __fadd_rn(__fadd_rn(red_l[0][r], red_l[1][r]), __fadd_rn(red_l[2][r], red_l[3][r]));
@@ -3008,14 +3013,27 @@ __device__ __forceinline__ void route_body(
     auto load_block = [&](auto nt_, uint32_t slot, const int8_t* X8, const uint16_t* XV, int64_t r0, int64_t r1,
                           const float* s_lo, const float* s_hi, int nlim) {
         constexpr bool NTL = decltype(nt_)::value;
-        if (hr == 0) {
+        if constexpr (NH == 4) {       // four waves: QK rows; PV chunks 0, 1 and the scales; 2, 3; 4 to 7
+            if (hr == 0) {
+                dma_qk<NTL>(X8 + r0 * D, X8 + r1 * D, bo, slot);
+            } else if (hr == 1) {
+                dma_rows01<NTL>(XV + r0 * D, bo, slot);
+                if (lane < 8) dma16s<NTL>(s_lo, (uint32_t)(16 * (lane & nlim)), slot + 12288);
+                else if (lane < 16) dma16s<NTL>(s_hi, (uint32_t)(16 * (lane & nlim)), slot + 12288);
+            } else if (hr == 2) {
+                dma_rows23<NTL>(XV + r0 * D, bo, slot);
+            } else {
+                dma_rows47<NTL>(XV + r1 * D, bo, slot);
+            }
+        } else if (hr == 0) {
             dma_qk<NTL>(X8 + r0 * D, X8 + r1 * D, bo, slot);
             dma_rows01<NTL>(XV + r0 * D, bo, slot);
             // (the saddr form, one base per lane half: no 64-bit lane address held across the loop)
             if (lane < 8) dma16s<NTL>(s_lo, (uint32_t)(16 * (lane & nlim)), slot + 12288);
             else if (lane < 16) dma16s<NTL>(s_hi, (uint32_t)(16 * (lane & nlim)), slot + 12288);
         } else {
-            dma_rows27<NTL>(XV + r0 * D, XV + r1 * D, bo, slot);
+            dma_rows23<NTL>(XV + r0 * D, bo, slot);
+            dma_rows47<NTL>(XV + r1 * D, bo, slot);
         }
     };
     // near block bi (list positions e_lo + 32 bi, + 16): the 16-token runs start there (past
@@ -3023,7 +3041,7 @@ __device__ __forceinline__ void route_body(
     auto run_pos = [&](int j) { return j < e_hi ? j : e_lo; };
     auto issue_near = [&](int bi, int slot) {
         if (bi >= nn) return;
-        int e0 = e_lo + 32 * bi;
+        int e0 = __builtin_amdgcn_readfirstlane(e_lo + 32 * bi);
         asm volatile("" : "+s"(e0));     // (a loop-invariant LDS address would be held, and spilled, across the far loop)
         const int ja = run_pos(e0), jb = run_pos(e0 + 16);
         const int64_t r0 = kh + (int64_t)__builtin_amdgcn_readfirstlane(sidx[ja / LEAF]) * LEAF + (ja % LEAF);
@@ -3306,7 +3324,7 @@ __device__ __forceinline__ void route_body(
     // half 0, then of row half 1, so the staging fits a 2-slot ring.
 #pragma unroll
     for (int round = 0; round < (MRG2 ? 2 : 1); ++round) {
-        if (!MRG2 || hr == round) {
+        if (!MRG2 || hr / (NH / 2) == round) {
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
                 const int r = 16 * RB * hr + 16 * rb + col;
@@ -3357,17 +3375,17 @@ __device__ __forceinline__ void route_body(
         out, logz
 template <int LEAF, int RB, int NP, int RS>
 __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_kernel(ROUTE_PARAMS) {
-    route_body<LEAF, RB, NP, RS, ROUTE_WHOLE>(ROUTE_ARGS, nullptr, nullptr, 1);
+    route_body<LEAF, RB, NP, RS, ROUTE_WHOLE, 2>(ROUTE_ARGS, nullptr, nullptr, 1);
 }
-template <int LEAF, int RB>
-__global__ __launch_bounds__(128, 3) void route_part_kernel(ROUTE_PARAMS, float* __restrict__ part_o,
-                                                            float* __restrict__ part_l, int nseg) {
-    route_body<LEAF, RB, 1, ROUTE_RS, ROUTE_PART>(ROUTE_ARGS, part_o, part_l, nseg);
+template <int LEAF, int RB, int NH>
+__global__ __launch_bounds__(64 * NH, RB == 2 ? 3 : 4) void route_part_kernel(ROUTE_PARAMS, float* __restrict__ part_o,
+                                                                             float* __restrict__ part_l, int nseg) {
+    route_body<LEAF, RB, 1, ROUTE_RS, ROUTE_PART, NH>(ROUTE_ARGS, part_o, part_l, nseg);
 }
-template <int LEAF, int RB>
-__global__ __launch_bounds__(128, 2) void route_seg_kernel(ROUTE_PARAMS, float* __restrict__ part_o,
-                                                           float* __restrict__ part_l, int nseg) {
-    route_body<LEAF, RB, 1, ROUTE_RS, ROUTE_SEGS>(ROUTE_ARGS, part_o, part_l, nseg);
+template <int LEAF, int RB, int NH>
+__global__ __launch_bounds__(64 * NH, RB == 2 ? 2 : 3) void route_seg_kernel(ROUTE_PARAMS, float* __restrict__ part_o,
+                                                                            float* __restrict__ part_l, int nseg) {
+    route_body<LEAF, RB, 1, ROUTE_RS, ROUTE_SEGS, NH>(ROUTE_ARGS, part_o, part_l, nseg);
 }
 #undef ROUTE_PARAMS
 #undef ROUTE_ARGS
@@ -5366,18 +5384,23 @@ static int route_attend_launch(const int8_t* q8, const float* sq, const int8_t* 
         REQUIRE(!split || aligned(parts, 16), "htrc_route_attend: misaligned buffer");
         float* part_o = split ? parts : nullptr;
         float* part_l = split ? parts + units * nseg * tile * D : nullptr;
-#define SEG_LAUNCH(K, L, RB, N)                                                                                 \
-    hipLaunchKernelGGL((K<L, RB>), dim3((unsigned)(units * (N))), dim3(128), dyn, s, q8, sq, dq8, sdq, g8, sg, lz, vb, k8, ks, \
-                       v, idx, rowmax, nq, (int)nt, group, (int)g0, (int)gn, perm, nk, (int)nb, nbp, kxe, scale, out, \
-                       logz, part_o, part_l, nseg)
+#define SEG_LAUNCH(K, L, RB, NH, N)                                                                             \
+    hipLaunchKernelGGL((K<L, RB, NH>), dim3((unsigned)(units * (N))), dim3(64 * NH), dyn, s, q8, sq, dq8, sdq, g8, sg, lz, \
+                       vb, k8, ks, v, idx, rowmax, nq, (int)nt, group, (int)g0, (int)gn, perm, nk, (int)nb, nbp, kxe,  \
+                       scale, out, logz, part_o, part_l, nseg)
+        // A 64-row tile's segments run with its rows over four waves (16 each, three or four waves a SIMD): the
+        // launches are short of waves, and each hides the others' loads (128-tile windows of the 40759-token head
+        // 648 -> 587 us a call, 512-tile ones of four heads 1978 -> 1946).  In turn, two waves of 32 rows, whose LDS reads feed twice
+        // the products: 768 tiles a window 3530 against 3612 us a call with four, 2048 tiles 2100 against 2236.
+#define SEG_SPLIT(L, RB, NH)                                                                                    \
+    SEG_LAUNCH(route_part_kernel, L, RB, NH, nseg);                                                             \
+    SEG_LAUNCH(route_seg_kernel, L, RB, NH, SEG_QUARTERS);
 #define SEG_CASE(L)                                                                                             \
     case L:                                                                                                     \
-        if (tile == 64) {                                                                                       \
-            if (split) SEG_LAUNCH(route_part_kernel, L, 2, nseg);                                               \
-            SEG_LAUNCH(route_seg_kernel, L, 2, split ? SEG_QUARTERS : 1);                                       \
+        if (tile == 32) {                                                                                       \
+            if (split) { SEG_SPLIT(L, 1, 2) } else { SEG_LAUNCH(route_seg_kernel, L, 1, 2, 1); }                \
         } else {                                                                                                \
-            if (split) SEG_LAUNCH(route_part_kernel, L, 1, nseg);                                               \
-            SEG_LAUNCH(route_seg_kernel, L, 1, split ? SEG_QUARTERS : 1);                                       \
+            if (split) { SEG_SPLIT(L, 1, 4) } else { SEG_LAUNCH(route_seg_kernel, L, 2, 2, 1); }                \
         }                                                                                                       \
         break;
         switch (leaf) {
@@ -5387,6 +5410,7 @@ static int route_attend_launch(const int8_t* q8, const float* sq, const int8_t* 
             SEG_CASE(128)
         }
 #undef SEG_CASE
+#undef SEG_SPLIT
 #undef SEG_LAUNCH
         return launched("htrc_route_attend");
     }

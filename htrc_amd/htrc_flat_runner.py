@@ -65,8 +65,8 @@ F32_UNSPLIT_TILES = 2048
 
 # Fused int8 route: the segments whose partial sums a launch of ``units`` (head, tile) pairs keeps in
 # workspace (htrc_route_segments of the C ABI): tiles of more than 128 blocks of 32 keys, in launches of at
-# most 512 pairs and heads of at most 16384 leaves.
-SEG_MIN_BLOCKS, SEG_MAX, SEG_SPLIT_TILES, SEG_MAX_NB = 128, 4, 512, 16384
+# most 384 pairs and heads of at most 16384 leaves.
+SEG_MIN_BLOCKS, SEG_MAX, SEG_SPLIT_TILES, SEG_MAX_NB = 128, 4, 384, 16384
 
 
 def route_segments(units: int, nb: int, kx: int, leaf: int) -> int:
