@@ -49,30 +49,36 @@ __device__ __forceinline__ int64_t perm_row(const int32_t* perm, int64_t h, int6
 // Shared centres of tile groups (h3/htrc_flat.py:223-229): mu_g is the mean of the G * tile
 // rows of tiles gG .. gG + G - 1, where tiles past the last repeat the last tile and rows past
 // the last query repeat the last query (the reference pads the tiles, then averages every
-// padded row).  One thread per dim: sequential fp32 sum over the group's rows in order, then
-// one IEEE division.
+// padded row).  One wave per group, two dims per lane: sequential fp32 sums over the group's rows in order,
+// then one IEEE division.  The sums are short; what counts is the rows in flight: 32 row loads
+// before their adds, each the row's whole 256 (bf16) or 512 bytes (one dim per lane and 8 rows ahead:
+// 24 heads x 157 groups of 128 bf16 rows 82.6 us for 123 MB, 27.1 now).
 template <bool IN_BF16>
-__global__ __launch_bounds__(128) void group_centres_kernel(const void* __restrict__ qin, int64_t nq, int nt,
-                                                            int tile, int group, int ng,
-                                                            const int32_t* __restrict__ perm, float* __restrict__ mu) {
+__global__ __launch_bounds__(64) void group_centres_kernel(const void* __restrict__ qin, int64_t nq, int nt,
+                                                           int tile, int group, int ng,
+                                                           const int32_t* __restrict__ perm, float* __restrict__ mu) {
     const int g = blockIdx.x, h = blockIdx.y, i = threadIdx.x;
     const int64_t qbase = (int64_t)h * nq * D;
-    const int rows = group * tile;
-    float s = 0.0f;
-    for (int j0 = 0; j0 < rows; j0 += 8) {
-        float x[8];
+    const int rows = group * tile;                  // a multiple of 32
+    float s0 = 0.0f, s1 = 0.0f;
+    for (int j0 = 0; j0 < rows; j0 += 32) {
+        u32x2 x[32];
+        const int64_t p0 = (int64_t)min(g * group + j0 / tile, nt - 1) * tile + j0 % tile;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int j = j0 + u;
-            const int t = min(g * group + j / tile, nt - 1);
-            const int64_t pp = min((int64_t)t * tile + j % tile, nq - 1);
-            const int64_t p = perm_row(perm, h, nq, pp);
-            x[u] = IN_BF16 ? bf2f(((const uint16_t*)qin)[qbase + p * D + i]) : ((const float*)qin)[qbase + p * D + i];
+        for (int u = 0; u < 32; ++u) {
+            const int64_t p = perm_row(perm, h, nq, min(p0 + u, nq - 1));
+            if constexpr (IN_BF16) x[u].x = ((const uint32_t*)qin)[(qbase + p * D) / 2 + i];
+            else x[u] = ((const u32x2*)qin)[(qbase + p * D) / 2 + i];
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) s = __fadd_rn(s, x[u]);
+        for (int u = 0; u < 32; ++u) {
+            s0 = __fadd_rn(s0, IN_BF16 ? __uint_as_float(x[u].x << 16) : __uint_as_float(x[u].x));
+            s1 = __fadd_rn(s1, IN_BF16 ? __uint_as_float(x[u].x & 0xffff0000u) : __uint_as_float(x[u].y));
+        }
     }
-    mu[((int64_t)h * ng + g) * D + i] = __fdiv_rn(s, (float)rows);
+    float* dst = mu + ((int64_t)h * ng + g) * D + 2 * i;
+    dst[0] = __fdiv_rn(s0, (float)rows);
+    dst[1] = __fdiv_rn(s1, (float)rows);
 }
 
 // One workgroup per tile of `tile` (32 or 64) rows.  group == 1: the tile's centre over its
@@ -4779,10 +4785,10 @@ int htrc_pack_q(const void* q, int q_is_bf16, int64_t heads, int64_t nq, int d, 
     if (group > 1) {
         const dim3 gg((unsigned)ng, (unsigned)heads);
         if (q_is_bf16)
-            hipLaunchKernelGGL(group_centres_kernel<true>, gg, dim3(D), 0, s, q, nq, (int)nt, tile, group, (int)ng,
+            hipLaunchKernelGGL(group_centres_kernel<true>, gg, dim3(64), 0, s, q, nq, (int)nt, tile, group, (int)ng,
                                perm, mu);
         else
-            hipLaunchKernelGGL(group_centres_kernel<false>, gg, dim3(D), 0, s, q, nq, (int)nt, tile, group, (int)ng,
+            hipLaunchKernelGGL(group_centres_kernel<false>, gg, dim3(64), 0, s, q, nq, (int)nt, tile, group, (int)ng,
                                perm, mu);
     }
     dim3 grid((unsigned)nt, (unsigned)heads);
@@ -5201,10 +5207,10 @@ int htrc_pack_q16(const void* q, int q_is_bf16, int64_t heads, int64_t nq, int d
     if (group > 1) {
         const dim3 gg((unsigned)ng, (unsigned)heads);
         if (q_is_bf16)
-            hipLaunchKernelGGL(group_centres_kernel<true>, gg, dim3(D), 0, s, q, nq, (int)nt, tile, group, (int)ng,
+            hipLaunchKernelGGL(group_centres_kernel<true>, gg, dim3(64), 0, s, q, nq, (int)nt, tile, group, (int)ng,
                                perm, mu);
         else
-            hipLaunchKernelGGL(group_centres_kernel<false>, gg, dim3(D), 0, s, q, nq, (int)nt, tile, group, (int)ng,
+            hipLaunchKernelGGL(group_centres_kernel<false>, gg, dim3(64), 0, s, q, nq, (int)nt, tile, group, (int)ng,
                                perm, mu);
     }
     dim3 grid((unsigned)nt, (unsigned)heads);
