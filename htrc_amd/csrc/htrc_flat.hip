@@ -2285,7 +2285,7 @@ __global__ __launch_bounds__(256, 3) void tile_f32_kernel(
 }
 
 // SEL[g, l] = max over every stride-th row of the group's tiles of (q - mu_g) . g_l, + lz_l, with
-// fp32 dots (h3/htrc_flat_triton.py:214-254, DOT = 0).  Workgroup = one group x SEL_F32_LPW
+// fp32 dots (h3/htrc_flat_triton.py:214-254, DOT = 0).  Workgroup = one group x lpw
 // leaves, 4 waves; wave w holds the split q - mu of 16 of the group's sampled rows (rows 64 c +
 // 16 w .. of row chunk c; rows past the last repeat it, tiles past the last repeat it, as the
 // reference pads them, which leaves every maximum unchanged) and the workgroup streams its
@@ -2296,21 +2296,21 @@ __global__ __launch_bounds__(256, 3) void tile_f32_kernel(
 // dims 32 ks + 8 grp .. + 7): g and q - mu each split into bf16 terms that sum to them exactly (a
 // bf16 g: one term; TF32 operands: two; fp32: three), every term product formed, so each dim's
 // product is exactly the one the fp32 MFMA forms and only the grouping of the fp32 sums differs.
-constexpr int SEL_F32_LPW = 1024;  // leaves per workgroup
+constexpr int SEL_F32_LPW = 1024;  // leaves per workgroup, at most (lpw: the launch's)
 template <bool QBF, bool SB, bool TF32>
 __global__ __launch_bounds__(256) void select_f32_kernel(const void* __restrict__ q, const float* __restrict__ mu,
                                                          int mu_stride, const void* __restrict__ g,
                                                          const float* __restrict__ lz, int64_t nq, int nt, int tile,
                                                          int stride, int group, int g0, int ng,
                                                          const int32_t* __restrict__ perm, int nb, int nb_pad,
-                                                         float* __restrict__ sel) {
+                                                         int lpw, float* __restrict__ sel) {
     constexpr int QB = QBF ? 2 : 4, SBB = SB ? 2 : 4;
     constexpr int NG = SB ? 1 : (TF32 ? 2 : 3), ND = TF32 ? 2 : 3;
     constexpr int RW = SB ? 1 : 2;                             // 16-byte pieces per 8 dims of g
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, col = lane & 15,
               grp = lane >> 4, tid = threadIdx.x;
     const int gi = blockIdx.y, h = blockIdx.z, gg = g0 + gi;
-    const int lw0 = blockIdx.x * SEL_F32_LPW, nlw = min(nb - lw0, SEL_F32_LPW);   // leaves [lw0, lw0 + nlw)
+    const int lw0 = blockIdx.x * lpw, nlw = min(nb - lw0, lpw);   // leaves [lw0, lw0 + nlw)
     const int nblk = (nlw + 15) / 16;
     const int64_t srow = ((int64_t)h * ng + gi) * nb_pad;
     __shared__ __align__(16) char terms[2][NG][16 * 256];     // block terms: leaf row of 256 B, chunk c at c ^ leaf
@@ -2351,7 +2351,7 @@ __global__ __launch_bounds__(256) void select_f32_kernel(const void* __restrict_
 #pragma unroll
         for (int a = 0; a < NG; ++a) *(bf16x8*)(&terms[buf][a][lf * 256 + ((c ^ lf) << 4)]) = t[a];
     };
-    for (int i = lane; i < SEL_F32_LPW; i += 64) wmax[w][i] = -INFINITY;
+    for (int i = lane; i < lpw; i += 64) wmax[w][i] = -INFINITY;
     const float* murow = mu + ((int64_t)h * mu_stride + gg) * D + 8 * grp;
     const int rpt = tile / stride, nsel = group * rpt;
     for (int rc = 0; rc < nsel; rc += 64) {
@@ -2418,45 +2418,38 @@ __global__ __launch_bounds__(256) void select_f32_kernel(const void* __restrict_
     }
 }
 
-// merge: (h3/htrc_flat_triton.py:257-273) + logZ = mm + log(den).  One workgroup (4 * tile
-// threads) per tile.
-// Tiles [t0, t0 + gridDim.x) of each head; the partials are the launch's own [H, gridDim.x, ns, tile].
+// merge: (h3/htrc_flat_triton.py:257-273) + logZ = mm + log(den).  32 threads per row, four dims each, 8 rows per
+// workgroup: every load and store is a row's contiguous 512 bytes, and a tile's rows spread over 8 workgroups
+// (with four threads per row and one workgroup per tile, 32 tiles of 8 splits took 14.4 us for 9.4 MB; 8.3 now).
+// Tiles [t0, t0 + tn) of each head (gridDim.x = tn * tile / 8); the partials are the launch's own [H, tn, ns, tile].
 __global__ __launch_bounds__(256) void merge_kernel(const float* __restrict__ pm, const float* __restrict__ pl,
                                                     const float* __restrict__ pacc, int ns, int64_t nq, int t0,
                                                     int tile, const int32_t* __restrict__ perm,
                                                     float* __restrict__ out, float* __restrict__ logz) {
-    const int t = t0 + blockIdx.x, h = blockIdx.y;
-    const int64_t th = (int64_t)h * gridDim.x + blockIdx.x;   // partial row of the tile
-    const int r = threadIdx.x >> 2, part = threadIdx.x & 3;   // 4 threads per row, 32 dims each
+    const int rpt = tile / 8, tl = blockIdx.x / rpt, t = t0 + tl, h = blockIdx.y;
+    const int64_t th = (int64_t)h * (gridDim.x / rpt) + tl;   // partial row of the tile
+    const int r = (blockIdx.x % rpt) * 8 + (threadIdx.x >> 5), dl = 4 * (threadIdx.x & 31);
     const int64_t qi = (int64_t)t * tile + r;
     if (qi >= nq) return;
     float mm = -INFINITY;
     for (int s = 0; s < ns; ++s) mm = fmaxf(mm, pm[(th * ns + s) * tile + r]);
     if (mm == -INFINITY) mm = 0.0f;
     float den = 0.0f;
-    float num[32];
-#pragma unroll
-    for (int i = 0; i < 32; ++i) num[i] = 0.0f;
+    f32x4 num = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
     for (int s = 0; s < ns; ++s) {
         const int64_t b = (th * ns + s) * tile + r;
+        const f32x4 x = *(const f32x4*)(pacc + b * D + dl);
         const float wv = __expf(__fsub_rn(pm[b], mm));
         den = __fadd_rn(den, __fmul_rn(pl[b], wv));
 #pragma unroll
-        for (int i = 0; i < 32; i += 4) {
-            const f32x4 x = *(const f32x4*)(pacc + b * D + part * 32 + i);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) num[i + j] = __fadd_rn(num[i + j], __fmul_rn(x[j], wv));
-        }
+        for (int j = 0; j < 4; ++j) num[j] = __fadd_rn(num[j], __fmul_rn(x[j], wv));
     }
     const float dd = den < 1e-30f ? 1e-30f : den;
     const int64_t orow = (int64_t)h * nq + perm_row(perm, h, nq, qi);
-#pragma unroll
-    for (int i = 0; i < 32; i += 4) {
-        f32x4 o = {__fdiv_rn(num[i], dd), __fdiv_rn(num[i + 1], dd), __fdiv_rn(num[i + 2], dd),
-                   __fdiv_rn(num[i + 3], dd)};
-        *(f32x4*)(out + orow * D + part * 32 + i) = o;
-    }
-    if (part == 0) logz[orow] = __fadd_rn(mm, __logf(den));
+    *(f32x4*)(out + orow * D + dl) = f32x4{__fdiv_rn(num[0], dd), __fdiv_rn(num[1], dd), __fdiv_rn(num[2], dd),
+                                           __fdiv_rn(num[3], dd)};
+    if (dl == 0) logz[orow] = __fadd_rn(mm, __logf(den));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -5153,11 +5146,14 @@ int htrc_select_f32(const void* q, int q_is_bf16, const float* mu, const void* g
     int64_t ng, tb, ntw;
     REQUIRE(group_window(nt, group, g0, gn, ng, tb, ntw), "htrc_select_f32: group window [g0, g0 + gn) must lie in the head's groups");
     REQUIRE(gn <= 65535, "htrc_select_f32: at most 65535 groups per launch");
-    const int64_t per = SEL_F32_LPW;                       // leaves per workgroup
+    // leaves per workgroup: as many as the LDS holds (one row prologue per group) where the groups fill the
+    // device, halved while two workgroups per CU are short (32 groups x 771 leaves: 37.3 us at 1024, 9.0 now)
+    int64_t per = SEL_F32_LPW;
+    while (per > 64 && (nb + per - 1) / per * gn * heads < 2 * device_cus()) per /= 2;
     const dim3 grid((unsigned)((nb + per - 1) / per), (unsigned)gn, (unsigned)heads);
     hipStream_t s = (hipStream_t)stream;
     F32_DISPATCH(select_f32_kernel, grid, dim3(256), q, mu, (int)ng, g, lz, nq, (int)nt, tile, stride, group, (int)g0,
-                 (int)gn, perm, (int)nb, htrc_nb_pad(nb), sel);
+                 (int)gn, perm, (int)nb, htrc_nb_pad(nb), (int)per, sel);
     return launched("htrc_select_f32");
 }
 
@@ -5269,7 +5265,7 @@ int htrc_merge(const float* pm, const float* pl, const float* pacc, int64_t head
     const int64_t nt = (nq + tile - 1) / tile;
     REQUIRE(nt <= 0x7fffffff, "htrc_merge: too many tiles");
     REQUIRE(t0 >= 0 && tn > 0 && t0 + tn <= nt, "htrc_merge: tile window [t0, t0 + tn) must lie in the head's tiles");
-    hipLaunchKernelGGL(merge_kernel, dim3((unsigned)tn, (unsigned)heads), dim3(4 * tile), 0, (hipStream_t)stream, pm,
+    hipLaunchKernelGGL(merge_kernel, dim3((unsigned)(tn * (tile / 8)), (unsigned)heads), dim3(256), 0, (hipStream_t)stream, pm,
                        pl, pacc, splits, nq, (int)t0, tile, perm, out, logz);
     return launched("htrc_merge");
 }
