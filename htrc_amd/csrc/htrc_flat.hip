@@ -4846,9 +4846,14 @@ static int leaf_stats_launch(const char* who, const float* mu, const uint16_t* m
     // leaf-stationary: NL leaves (64 KB of K / V) per workgroup; the centre groups of a head dealt
     // over ncs workgroups when the leaf groups alone give fewer than two workgroups per CU (each
     // wave keeps at least one group of 16 centres)
-    const int nl = 65536 / (512 * leaf);
-    const int64_t nlg = nbp / nl, ncg = (cn + 15) / 16;
+    // (leaf 16: 32 KB where the leaf groups are fewer than two per CU: three workgroups then share a CU's registers and LDS
+    // with TF32 operands, and twice the workgroups share the few centre groups of a short window.  One head of 40752 keys,
+    // 128 centres 46.2 -> 40.0 us, 637 centres 172.6 -> 156.2; 32 centres of 12336 keys, fp32 store, 31.0 -> 21.5.  Not the
+    // IEEE operands of longer windows (637 centres, fp8: 144 -> 161), nor six heads (231 -> 249).)
     const int64_t want = 2 * (int64_t)device_cus();
+    const bool half = leaf == 16 && nbp / 8 * heads < want && (TF32 || cn <= 64) && mut;
+    const int nl = half ? 4 : 65536 / (512 * leaf);
+    const int64_t nlg = nbp / nl, ncg = (cn + 15) / 16;
     int64_t ncs = (want + nlg * heads - 1) / (nlg * heads);
     ncs = ncs < 1 ? 1 : (ncs > (ncg + 3) / 4 ? (ncg + 3) / 4 : ncs);
     const int64_t nblocks = ncs * nlg * heads;
@@ -4866,6 +4871,11 @@ static int leaf_stats_launch(const char* who, const float* mu, const uint16_t* m
                                nt, c0, (int)cn, k, v, nk, (int)nb, nbp, (int)ncs, scale, (int8_t*)g, sg,            \
                                (uint16_t*)vb, sv, lz);                                                             \
         break;
+    if (half) {
+        hipLaunchKernelGGL((stats_ls_kernel<16, STORE, 4, TF32, true>), grid, dim3(256), 0, s, mu, mut, nt, c0, (int)cn, k, v,
+                           nk, (int)nb, nbp, (int)ncs, scale, (int8_t*)g, sg, (uint16_t*)vb, sv, lz);
+        return launched(who);
+    }
     switch (leaf) {
         STATS_CASE(16)
         STATS_CASE(32)
