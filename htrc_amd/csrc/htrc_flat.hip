@@ -5599,6 +5599,93 @@ int htrc_route16(const uint16_t* q16, const uint16_t* dq16, const void* g, const
                                g0, gn, perm, fp8, scale, out, logz, stream);
 }
 
+// The tile windows of a layer, each the centres' terms, the statistics and the routing of `chunk` tile groups, dealt in
+// turn over the caller's streams: the launches of the entry points above in their order, issued here because a window's
+// five to seven launches cost a Python caller longer than a small window runs (the fp32 path on 12345 queries in seven
+// windows of 32 tiles: 554 us of host time a call launched one by one, 321 here, the call 563 -> 373).
+int htrc_windows_i8(const float* mu, const uint16_t* k, const uint16_t* v, const int8_t* q8, const float* sq,
+                    const int8_t* dq8, const float* sdq, const int8_t* k8, const float* ks, int64_t heads, int64_t nq,
+                    int64_t nk, int leaf, int d, int kx, int sink, int stride, int tile, int group, int64_t chunk,
+                    const int32_t* perm, int tf32, float scale, float* rowmax, float* out, float* logz, int nstreams,
+                    void* const* bufs, void* const* streams) {
+    REQUIRE(bufs && streams && nstreams >= 1 && chunk >= 1, "htrc_windows_i8: need buffers, streams and chunk >= 1");
+    REQUIRE((tile == 32 || tile == 64) && group >= 1 && nq > 0, "htrc_windows_i8: bad sizes");
+    const int64_t nt = (nq + tile - 1) / tile, ng = (nt + group - 1) / group;
+    for (int64_t g0 = 0, w = 0; g0 < ng; g0 += chunk, ++w) {
+        const int64_t gn = chunk < ng - g0 ? chunk : ng - g0;
+        void* const* b = bufs + 8 * (w % nstreams);
+        void* s = streams[w % nstreams];
+        int rc = htrc_centre_terms(mu, heads, ng, g0, gn, d, tf32, (uint16_t*)b[0], s);
+        if (rc == HTRC_OK)
+            rc = htrc_leaf_stats_terms((const uint16_t*)b[0], k, v, heads, gn, nk, leaf, d, scale, 0, tf32, b[1], (float*)b[2],
+                                       b[3], nullptr, (float*)b[4], s);
+        if (rc == HTRC_OK)
+            rc = htrc_route_seg(q8, sq, dq8, sdq, (const int8_t*)b[1], (const float*)b[2], (const float*)b[4],
+                                (const uint16_t*)b[3], k8, ks, v, heads, nq, nk, leaf, d, kx, sink, stride, tile, group, g0,
+                                gn, perm, scale, out, logz, (int32_t*)b[5], rowmax, (uint32_t*)b[6], (float*)b[7], s);
+        if (rc != HTRC_OK) return rc;
+    }
+    return HTRC_OK;
+}
+
+int htrc_windows_16(const float* mu, const uint16_t* k, const uint16_t* v, const uint16_t* q16, const uint16_t* dq16,
+                    int64_t heads, int64_t nq, int64_t nk, int leaf, int d, int kx, int sink, int stride, int tile,
+                    int group, int64_t chunk, const int32_t* perm, int fp8, int tf32, float scale, float* rowmax,
+                    float* out, float* logz, int nstreams, void* const* bufs, void* const* streams) {
+    REQUIRE(bufs && streams && nstreams >= 1 && chunk >= 1, "htrc_windows_16: need buffers, streams and chunk >= 1");
+    REQUIRE((tile == 32 || tile == 64) && group >= 1 && nq > 0, "htrc_windows_16: bad sizes");
+    const int64_t nt = (nq + tile - 1) / tile, ng = (nt + group - 1) / group;
+    for (int64_t g0 = 0, w = 0; g0 < ng; g0 += chunk, ++w) {
+        const int64_t gn = chunk < ng - g0 ? chunk : ng - g0;
+        void* const* b = bufs + 7 * (w % nstreams);
+        void* s = streams[w % nstreams];
+        int rc = htrc_centre_terms(mu, heads, ng, g0, gn, d, tf32, (uint16_t*)b[0], s);
+        if (rc == HTRC_OK)
+            rc = htrc_leaf_stats_terms((const uint16_t*)b[0], k, v, heads, gn, nk, leaf, d, scale, fp8 ? 2 : 1, tf32, b[1],
+                                       (float*)b[2], b[3], (float*)b[4], (float*)b[5], s);
+        if (rc == HTRC_OK)
+            rc = htrc_route16(q16, dq16, b[1], (const float*)b[2], (const float*)b[5], b[3], (const float*)b[4], k, v, heads,
+                              nq, nk, leaf, d, kx, sink, stride, tile, group, g0, gn, perm, fp8, scale, out, logz,
+                              (int32_t*)b[6], rowmax, s);
+        if (rc != HTRC_OK) return rc;
+    }
+    return HTRC_OK;
+}
+
+int htrc_windows_f32(const void* q, int q_is_bf16, const float* mu, const uint16_t* k, const uint16_t* v, int64_t heads,
+                     int64_t nq, int64_t nk, int leaf, int d, int kx, int sink, int stride, int tile, int group,
+                     int64_t chunk, int splits, int bn, int64_t unsplit, const int32_t* perm, int state_bf16, int tf32,
+                     float scale, float* out, float* logz, int nstreams, void* const* bufs, void* const* streams) {
+    REQUIRE(bufs && streams && nstreams >= 1 && chunk >= 1, "htrc_windows_f32: need buffers, streams and chunk >= 1");
+    REQUIRE((tile == 32 || tile == 64) && group >= 1 && nq > 0 && leaf > 0 && kx > 0, "htrc_windows_f32: bad sizes");
+    const int64_t nt = (nq + tile - 1) / tile, ng = (nt + group - 1) / group, nb = nk / leaf;
+    for (int64_t g0 = 0, w = 0; g0 < ng; g0 += chunk, ++w) {
+        const int64_t gn = chunk < ng - g0 ? chunk : ng - g0, tb = g0 * group;
+        const int64_t ntw = (nt < (g0 + gn) * group ? nt : (g0 + gn) * group) - tb;
+        void* const* b = bufs + 10 * (w % nstreams);
+        void* s = streams[w % nstreams];
+        const int ns = heads * ntw >= unsplit || splits < 1 ? 1 : splits;
+        int rc = htrc_centre_terms(mu, heads, ng, g0, gn, d, tf32, (uint16_t*)b[0], s);
+        if (rc == HTRC_OK)
+            rc = htrc_leaf_stats_terms((const uint16_t*)b[0], k, v, heads, gn, nk, leaf, d, scale, state_bf16 ? 1 : 3, tf32,
+                                       b[1], nullptr, b[2], nullptr, (float*)b[3], s);
+        if (rc == HTRC_OK)
+            rc = htrc_select_f32(q, q_is_bf16, mu, b[1], state_bf16, (const float*)b[3], heads, nq, nb, stride, tile, group,
+                                 g0, gn, perm, tf32, d, (float*)b[4], s);
+        if (rc == HTRC_OK) rc = htrc_topk((const float*)b[4], heads * gn, nb, kx, sink, (int32_t*)b[5], (int8_t*)b[6], s);
+        if (rc == HTRC_OK)
+            rc = htrc_tile_f32(q, q_is_bf16, mu, b[1], state_bf16, (const float*)b[3], b[2], (const int8_t*)b[6],
+                               (const int32_t*)b[5], k, v, heads, nq, nk, leaf, d, kx, tile, group, g0, gn, perm, ns, bn, tf32,
+                               scale, ns > 1 ? (float*)b[7] : nullptr, ns > 1 ? (float*)b[8] : nullptr,
+                               ns > 1 ? (float*)b[9] : nullptr, out, logz, s);
+        if (rc == HTRC_OK && ns > 1)
+            rc = htrc_merge((const float*)b[7], (const float*)b[8], (const float*)b[9], heads, nq, tile, tb, ntw, ns, d, perm,
+                            out, logz, s);
+        if (rc != HTRC_OK) return rc;
+    }
+    return HTRC_OK;
+}
+
 // Device address of `scratch` on the current device, resolved once per device (with that device
 // current) and kept; nullptr with the error set when the runtime cannot resolve it.
 static void* scratch_ptr() {

@@ -17,6 +17,8 @@ shapes.  ``prec`` is always IEEE fp32 accumulate (there is no TF32 on CDNA4).
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -581,6 +583,79 @@ def route16(packed: dict, state: dict, *, nq: int, leaf: int, kx: int, scale: fl
 def route16_fits(nb: int, kx: int) -> bool:
     """Whether the fused 16-bit route takes this shape (else the split tile path runs it)."""
     return int(nb) <= ROUTE_NB_LDS and min(int(kx), int(nb)) <= ROUTE_MAX_KX
+
+
+def run_windows(packed: dict, q, mu, *, nb: int, leaf: int, kx: int, scale: float, store, f32dots: bool, wins, sink: int,
+                stride: int, tile: int, group: int, perm, prec: str, splits: int, bn: int, unsplit: int, rowmax, out, logz,
+                wss, streams):
+    """The tile windows ``wins`` [(g0, gn), ...] of a layer in one native call (htrc_windows_*): window i on the stream
+    handle streams[i % n] with the buffers of the workspace wss[i % n] (the names and sizes of the per-stage
+    functions above).  packed, q, mu as flat_attention builds them; kx > 0 for the fp32 dots."""
+    k, v = packed["k"], packed["v"]
+    _need(mu, torch.float32, "mu")
+    _need(k, torch.bfloat16, "k")
+    _need(v, torch.bfloat16, "v")
+    h, nk, d = (int(x) for x in k.shape)
+    if nb * leaf != nk or tuple(v.shape) != tuple(k.shape):
+        raise ValueError("keys and values must be [H, nb * leaf, D]")
+    nq, dev, nbp = int(out.shape[1]), k.device, nb_pad(nb)
+    nt = -(-nq // tile)
+    tf32 = int(prec == "tf32")
+    gname, vname, vdt = {torch.int8: ("g", "vb", torch.bfloat16), torch.bfloat16: ("g_bf16", "vb", torch.bfloat16),
+                         torch.float8_e4m3fn: ("g_fp8", "vb_fp8", torch.float8_e4m3fn),
+                         torch.float32: ("g_f32", "vb_f32", torch.float32)}[store]
+
+    def tiles(g0, gn):
+        return min(nt, (g0 + gn) * group) - g0 * group
+
+    live, bufs = [], []
+    n = len(streams)
+    for i in range(n):
+        ws, mine = wss[i], wins[i::n]
+        gn = mine[0][1]                                 # the largest window of the stream (only the layer's last is smaller)
+
+        def rows(name, tail, dtype, r=gn):
+            t = _buf(ws, name, (h * r, *tail), dtype, dev)
+            live.append(t)
+            return t.data_ptr()
+
+        b = {"terms": rows("mu_terms", (MUT_ROW,), torch.int16), "g": rows(gname, (nbp, d), store),
+             "vb": rows(vname, (nbp, d), vdt), "lz": rows("lz", (nbp,), torch.float32),
+             "idx": rows("idx", (kx,), torch.int32) if kx > 0 else None}
+        if f32dots:
+            b["sel"], b["excl"] = rows("sel", (nbp,), torch.float32), rows("excl", (nbp,), torch.int8)
+            part = next((tiles(*w) for w in mine if splits > 1 and h * tiles(*w) < unsplit), 0)
+            for name, tail in (("pm", (splits, tile)), ("pl", (splits, tile)), ("pacc", (splits, tile, d))):
+                b[name] = rows(name, tail, torch.float32, part) if part else None
+            names = ("terms", "g", "vb", "lz", "sel", "idx", "excl", "pm", "pl", "pacc")
+        elif store == torch.int8:
+            b["sg"] = rows("sg", (nbp,), torch.float32)
+            b["keys"] = rows("route_keys", (nbp,), torch.int32) if nb > ROUTE_NB_LDS else None
+            size = max(h * tiles(*w) * (s if (s := route_segments(h * tiles(*w), nb, kx, leaf)) > 1 else 0) for w in mine)
+            b["parts"] = None
+            if size:
+                live.append(_buf(ws, "parts", (size * tile * (D + 1),), torch.float32, dev))
+                b["parts"] = live[-1].data_ptr()
+            names = ("terms", "g", "sg", "vb", "lz", "idx", "keys", "parts")
+        else:
+            fp8 = store == torch.float8_e4m3fn
+            b["sg"] = rows("sg", (nbp,), torch.float32) if fp8 else None
+            b["sv"] = rows("sv", (nbp,), torch.float32) if fp8 else None
+            names = ("terms", "g", "sg", "vb", "sv", "lz", "idx")
+        bufs += [b[x] for x in names]
+    bufs = (ctypes.c_void_p * len(bufs))(*bufs)
+    handles = (ctypes.c_void_p * n)(*streams)
+    shape = (h, nq, nk, leaf, d, kx, sink, stride, tile, group, wins[0][1])
+    tail = (float(scale), ptr(rowmax), ptr(out), ptr(logz), n, bufs, handles)
+    if f32dots:
+        call("htrc_windows_f32", ptr(q), int(q.dtype == torch.bfloat16), ptr(mu), ptr(k), ptr(v), *shape, splits, bn, unsplit,
+             ptr(perm), int(store == torch.bfloat16), tf32, tail[0], *tail[2:])
+    elif store == torch.int8:
+        call("htrc_windows_i8", ptr(mu), ptr(k), ptr(v), *(ptr(packed[x]) for x in ("q8", "sq", "dq8", "sdq", "k8", "ks")),
+             *shape, ptr(perm), tf32, *tail)
+    else:
+        call("htrc_windows_16", ptr(mu), ptr(k), ptr(v), ptr(packed["q16"]), ptr(packed["dq16"]), *shape, ptr(perm),
+             int(fp8), tf32, *tail)
 
 
 def tail_merge(q, tk, tv, *, scale: float, out, logz, f32dots: bool = False, prec: str = "ieee"):

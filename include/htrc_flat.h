@@ -175,6 +175,28 @@ int htrc_route_seg(const int8_t* q8, const float* sq, const int8_t* dq8, const f
                    int stride, int tile, int group, int64_t g0, int64_t gn, const int32_t* perm, float scale, float* out,
                    float* logz, int32_t* idx, float* rowmax, uint32_t* keys_ws, float* parts, void* stream);
 
+/* A layer's tile windows in one call: for every window of `chunk` tile groups, htrc_centre_terms,
+ * htrc_leaf_stats_terms, then htrc_route_seg (i8), htrc_route16 (16) or htrc_select_f32, htrc_topk, htrc_tile_f32 and
+ * (for fewer than `unsplit` (head, tile) pairs, run in `splits` splits) htrc_merge (f32), window w on streams[w % nstreams]
+ * with the buffers bufs[(w % nstreams) * n ..] of that stream (host arrays of device pointers; NULL where the entry
+ * point takes NULL), each of the largest window dealt to it.  The caller orders the streams against its own.
+ *   i8, n = 8: terms, g8, sg, vb, lz, idx, keys_ws, parts      16, n = 7: terms, g, sg, vb, sv, lz, idx
+ *   f32, n = 10: terms, g, vb, lz, sel, idx, excl, pm, pl, pacc
+ * Replaces the chunk loop of _flat_triton (h3/htrc_flat.py:236-273). */
+int htrc_windows_i8(const float* mu, const uint16_t* k, const uint16_t* v, const int8_t* q8, const float* sq,
+                    const int8_t* dq8, const float* sdq, const int8_t* k8, const float* ks, int64_t heads, int64_t nq,
+                    int64_t nk, int leaf, int d, int kx, int sink, int stride, int tile, int group, int64_t chunk,
+                    const int32_t* perm, int tf32, float scale, float* rowmax, float* out, float* logz, int nstreams,
+                    void* const* bufs, void* const* streams);
+int htrc_windows_16(const float* mu, const uint16_t* k, const uint16_t* v, const uint16_t* q16, const uint16_t* dq16,
+                    int64_t heads, int64_t nq, int64_t nk, int leaf, int d, int kx, int sink, int stride, int tile,
+                    int group, int64_t chunk, const int32_t* perm, int fp8, int tf32, float scale, float* rowmax,
+                    float* out, float* logz, int nstreams, void* const* bufs, void* const* streams);
+int htrc_windows_f32(const void* q, int q_is_bf16, const float* mu, const uint16_t* k, const uint16_t* v, int64_t heads,
+                     int64_t nq, int64_t nk, int leaf, int d, int kx, int sink, int stride, int tile, int group,
+                     int64_t chunk, int splits, int bn, int64_t unsplit, const int32_t* perm, int state_bf16, int tf32,
+                     float scale, float* out, float* logz, int nstreams, void* const* bufs, void* const* streams);
+
 /* htrc_route without caller workspace: rowmax, the near leaves and the top-k keys live in a
  * scratch array of 32 MiB that the library keeps on each device (resolved at the first call on
  * a device); the call allocates nothing, so callers that cannot allocate (code under HIP graph
