@@ -257,9 +257,9 @@ def flat_attention(q, k, v, *, tile=64, exact_leaves=64, order="seq", curvature=
         # head dims below 128 (the reference takes any power-of-two D, h3/htrc_flat_triton.py:43, 90):
         # zero dims leave every row maximum, int32 dot, state code and softmax as they are, so the
         # kernels run at 128 on copies padded with zeros and the output keeps the first d dims
-        qh = _pad_dims(qh, ws, "q_pad", qh.dtype)
-        kh = _pad_dims(kh, ws, "k_pad", torch.bfloat16)
-        vh = _pad_dims(vh, ws, "v_pad", torch.bfloat16)
+        want = (("q_pad", qh.dtype), ("k_pad", torch.bfloat16), ("v_pad", torch.bfloat16))
+        qh, kh, vh = (hip.pad_dims((qh, kh, vh), ws, *zip(*want))
+                      or [_pad_dims(x, ws, *w) for x, w in zip((qh, kh, vh), want)])
         d = hip.D
     perm = hip.kmeans_order(qh, ws=ws) if order == "kmeans" else None   # query rows regrouped by k-means
     qsrc = qh.contiguous()                               # the query rows select="bound" measures

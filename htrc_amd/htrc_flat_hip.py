@@ -30,6 +30,23 @@ TILES = (64, 32)          # query rows per tile the kernels take (32: the runner
 D = 128
 
 
+def pad_dims(xs, ws, names, dtypes):
+    """Up to three tensors [H, n, d < 128] -> workspace copies [H, n, 128] of ``dtypes`` whose dims past d are zero, in one
+    launch (written whole on every call, so a reused buffer and a graph replay see zeros there).  None where a tensor
+    is not contiguous fp32 or bf16 of the launch's alignment, or a dtype not one of those."""
+    ok = (torch.float32, torch.bfloat16)
+    if not all(x.is_cuda and x.dtype in ok and t in ok and x.is_contiguous() and x.data_ptr() % 4 == 0
+               for x, t in zip(xs, dtypes)):
+        return None
+    outs = [_buf(ws, n, (*x.shape[:-1], D), t, x.device) for x, n, t in zip(xs, names, dtypes)]
+    args = []
+    for x, o in zip(xs, outs):
+        args += [ptr(x), int(x.dtype == torch.bfloat16), x.numel() // int(x.shape[-1]), ptr(o), int(o.dtype == torch.bfloat16)]
+    args += [None, 0, 0, None, 0] * (3 - len(xs))
+    call("htrc_pad_dims", *args, int(xs[0].shape[-1]), stream_handle(xs[0].device))
+    return outs
+
+
 def _tile(tile) -> int:
     tile = int(tile)
     if tile not in TILES:

@@ -75,6 +75,13 @@ int htrc_nb_pad(int64_t nb);
 int htrc_pack_q(const void* q, int q_is_bf16, int64_t heads, int64_t nq, int d, int tile, int group,
                 const int32_t* perm, float* mu, int8_t* q8, float* sq, int8_t* dq8, float* sdq, void* stream);
 
+/* Rows of d < 128 values to rows of 128 with zeros past d, for up to three tensors in one launch (rows = 0: none): each
+ * fp32 or bf16 in (contiguous, 4-byte aligned), fp32 or bf16 out (nearest even; 16-byte aligned).
+ * No reference counterpart (its kernels are compiled per head dim). */
+int htrc_pad_dims(const void* a, int a_bf16, int64_t a_rows, void* a_out, int a_out_bf16, const void* b, int b_bf16,
+                  int64_t b_rows, void* b_out, int b_out_bf16, const void* c, int c_bf16, int64_t c_rows, void* c_out,
+                  int c_out_bf16, int d, void* stream);
+
 /* K int8 pack (round half to even, per-row scale).
  * Replaces the host-side K pack of _flat_triton (h3/htrc_flat.py:213-219). */
 int htrc_pack_k(const uint16_t* k, int64_t heads, int64_t nk, int d, int8_t* k8, float* ks, void* stream);

@@ -7,7 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from htrc_amd import htrc_flat, workloads
+from htrc_amd import htrc_flat, htrc_flat_hip as hip, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +35,32 @@ def test_host_values_are_refused(device, kw):
     q, k, v = workloads.clustered_runs(n=256, runs=4, heads=1, seed=1)
     with pytest.raises(ValueError):
         htrc_flat.flat_attention(q.to(device), k.to(device), v, backend="hip", leaf=32, exact_leaves=2, tile_chunk=2, **kw)
+
+
+@pytest.mark.parametrize("d", [1, 3, 32, 64, 80, 127])
+@pytest.mark.parametrize("kinds", [("bf16", "bf16", "bf16"), ("fp32", "fp32", "bf16"), ("fp32", "bf16", "fp32")])
+def test_pad_dims_equals_torch(device, d, kinds):
+    """One launch for q, k, v: the rows' values (fp32 keys rounded to bf16 as torch rounds them, infinities and NaN kept),
+    zeros past d in a buffer that held other values."""
+    dt = {"bf16": torch.bfloat16, "fp32": torch.float32}
+    g = torch.Generator().manual_seed(d)
+    xs = [(torch.randn((2, n, d), generator=g) * 3).to(dt[k]).to(device) for n, k in zip((7, 33, 33), kinds)]
+    xs[1][0, 0, 0], xs[1][0, 1, 0], xs[2][1, 2, d - 1] = float("inf"), float("nan"), -float("inf")
+    outs_dt = (xs[0].dtype, torch.bfloat16, torch.bfloat16)
+    ws = {n: torch.full((2, x.shape[1], 128), 9.0, device=device, dtype=t) for n, x, t in zip("abc", xs, outs_dt)}
+    outs = hip.pad_dims(xs, ws, tuple("abc"), outs_dt)
+    for x, o, t in zip(xs, outs, outs_dt):
+        assert torch.equal(o[..., :d].nan_to_num(123.0), x.to(t).nan_to_num(123.0))
+        assert bool((o[..., d:] == 0).all())
+
+
+def test_odd_address_keys_take_the_copying_path(device):
+    """Rows of 31 bf16 values at an address that is not a multiple of four: the same result."""
+    q, k, v = (x[..., :31].contiguous().to(device) for x in workloads.clustered_runs(n=256, runs=4, heads=1, seed=2))
+    kw = dict(store="int8", dot="bf16", backend="hip", leaf=32, exact_leaves=2)
+    want = htrc_flat.flat_attention(q, k, v, **kw).clone()
+    raw = torch.empty((k.numel() + 1,), dtype=torch.bfloat16, device=device)
+    k2 = raw[1:].view(k.shape)
+    k2.copy_(k)
+    assert k2.data_ptr() % 4 == 2 and hip.pad_dims((k2,), None, ("a",), (torch.bfloat16,)) is None
+    assert torch.equal(htrc_flat.flat_attention(q, k2, v, **kw), want)
