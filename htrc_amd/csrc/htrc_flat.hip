@@ -3402,6 +3402,14 @@ template <int LEAF, int RB, int NP, int RS>
 __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_kernel(ROUTE_PARAMS) {
     route_body<LEAF, RB, NP, RS, ROUTE_WHOLE, 2>(ROUTE_ARGS, nullptr, nullptr, 1);
 }
+// 64-row tiles with four waves of 16 rows per key part, where there are several: the same sums per row, twice the waves to hide
+// each block's loads in (16 x 32-leaf tiles of two heads of 11008 tokens 97.8 -> 95.5 us a call, one head of 24000
+// tokens 94.9 -> 93.4; 256 tiles and fewer within 1 %).  One key part keeps two waves of 32 rows: there
+// several tiles share a CU, and each LDS read feeds twice the products.
+template <int LEAF, int NP>
+__global__ __launch_bounds__(256 * NP, NP == 4 ? 4 : 2) void route_rows_kernel(ROUTE_PARAMS) {
+    route_body<LEAF, 1, NP, ROUTE_RS, ROUTE_WHOLE, 4>(ROUTE_ARGS, nullptr, nullptr, 1);
+}
 template <int LEAF, int RB, int NH>
 __global__ __launch_bounds__(64 * NH, RB == 2 ? 3 : 4) void route_part_kernel(ROUTE_PARAMS, float* __restrict__ part_o,
                                                                              float* __restrict__ part_l, int nseg) {
@@ -5478,12 +5486,16 @@ static int route_attend_launch(const int8_t* q8, const float* sq, const int8_t* 
     hipLaunchKernelGGL((route_kernel<L, RB, NP, ROUTE_RS>), grid, dim3(128 * NP), dyn, s, q8, sq, dq8, sdq, g8, sg, lz, vb, \
                        k8, ks, v, idx, rowmax, nq, (int)nt, group, (int)g0, (int)gn, perm, nk, (int)nb, nbp, kxe, scale, \
                        out, logz)
+#define ROUTE_ROWS(L, NP)                                                                                      \
+    hipLaunchKernelGGL((route_rows_kernel<L, NP>), grid, dim3(256 * NP), dyn, s, q8, sq, dq8, sdq, g8, sg, lz, vb, \
+                       k8, ks, v, idx, rowmax, nq, (int)nt, group, (int)g0, (int)gn, perm, nk, (int)nb, nbp, kxe, scale, \
+                       out, logz)
 #define ROUTE_CASE(L)                                                                                          \
     case L:                                                                                                    \
         if (tile == 64) {                                                                                      \
             if (np == 1) ROUTE_LAUNCH(L, 2, 1);                                                                \
-            else if (np == 2) ROUTE_LAUNCH(L, 2, 2);                                                           \
-            else ROUTE_LAUNCH(L, 2, 4);                                                                        \
+            else if (np == 2) ROUTE_ROWS(L, 2);                                                           \
+            else ROUTE_ROWS(L, 4);                                                                        \
         } else {                                                                                               \
             if (np == 1) ROUTE_LAUNCH(L, 1, 1);                                                                \
             else if (np == 2) ROUTE_LAUNCH(L, 1, 2);                                                           \
@@ -5497,6 +5509,7 @@ static int route_attend_launch(const int8_t* q8, const float* sq, const int8_t* 
         ROUTE_CASE(128)
     }
 #undef ROUTE_CASE
+#undef ROUTE_ROWS
 #undef ROUTE_LAUNCH
     return launched("htrc_route_attend");
 }
