@@ -2861,13 +2861,17 @@ __device__ __forceinline__ RowMax<RB> route_exact_max(const int8_t* dq8, const f
 constexpr int SEG_MIN_BLOCKS = 128;
 constexpr int SEG_MAX = 4;
 constexpr int64_t SEG_SPLIT_TILES = 384;             // launches of at most this many tiles run the segments apart
+// The layer's (head, tile) pairs: up to two a CU the whole-tile kernels split each tile's keys over several wave parts
+// (313 tiles in one window 168 us a call, segments 177); past four a CU a launch of the whole layer runs more tiles a CU
+// than the in-turn kernel's registers allow (1250 tiles of one window 839 us whole, 922 in turn; 625 tiles 453 and 457).
+constexpr int64_t SEG_TILES_MIN = 512, SEG_TILES_MAX = 1024;
 enum RouteMode { ROUTE_WHOLE = 0, ROUTE_PART = 1, ROUTE_SEGS = 2 };
 constexpr int SEG_QUARTERS = 4;                      // workgroups per tile that combine its partial sums
 
 // (heads of more than ROUTE_NB_LDS leaves, whose select works from global keys, keep whole tiles)
-inline int route_segments(int64_t nb, int kxe, int leaf) {
+inline int route_segments(int64_t tiles, int64_t nb, int kxe, int leaf) {
     const int64_t blocks = (nb + 31) / 32 + ((int64_t)kxe * leaf + 31) / 32;
-    if (blocks <= SEG_MIN_BLOCKS || nb > ROUTE_NB_LDS) return 1;
+    if (tiles <= SEG_TILES_MIN || tiles > SEG_TILES_MAX || blocks <= SEG_MIN_BLOCKS || nb > ROUTE_NB_LDS) return 1;
     const int64_t n = (blocks + 31) / 32;
     return (int)(n < SEG_MAX ? n : SEG_MAX);
 }
@@ -5441,7 +5445,7 @@ static int route_attend_launch(const int8_t* q8, const float* sq, const int8_t* 
     const size_t dyn = route_dyn_bytes(nb, kxe);
     // Long tiles (segs: the caller runs them segmented, with workspace for the partial sums where
     // the launch is small; see route_segments)
-    const int nseg = segs ? route_segments(nb, kxe, leaf) : 1;
+    const int nseg = segs ? route_segments(nt * heads, nb, kxe, leaf) : 1;
     if (nseg > 1) {
         REQUIRE(route_static_bytes(1) + dyn <= ROUTE_LDS_MAX, "htrc_route_attend: near list and exclusion bits exceed the LDS");
         const int64_t units = ntw * heads;
@@ -5530,7 +5534,7 @@ int htrc_route_segments(int64_t heads, int64_t nq, int64_t nk, int leaf, int kx,
     if (route_shapes("htrc_route_segments", heads, nq, nk, leaf, D, kx, tile, group, g0, gn, nb, nt, ng, tb, ntw, kxe) !=
         HTRC_OK)
         return 0;
-    return ntw * heads <= SEG_SPLIT_TILES ? route_segments(nb, kxe, leaf) : 1;
+    return ntw * heads <= SEG_SPLIT_TILES ? route_segments(nt * heads, nb, kxe, leaf) : 1;
 }
 
 int htrc_route_seg(const int8_t* q8, const float* sq, const int8_t* dq8, const float* sdq, const int8_t* g8,

@@ -488,7 +488,7 @@ def route(packed: dict, state: dict, *, nq: int, leaf: int, kx: int, scale: floa
     keys = _keys_ws(ws, h, gn, nb, dev)
     # partial sums of the segments of a long tile, where a small window runs them apart
     units = h * (min(nt, (g0 + gn) * int(group)) - g0 * int(group))
-    segs = route_segments(units, nb, kxe, int(leaf))
+    segs = route_segments(h * nt, units, nb, kxe, int(leaf))
     parts = _buf(ws, "parts", (units * segs * tile * (D + 1),), torch.float32, dev) if segs > 1 else None
     call("htrc_route_seg", ptr(q8), ptr(sq), ptr(dq8), ptr(sdq), ptr(g8), ptr(sg), ptr(lz), ptr(vb), ptr(k8), ptr(ks),
          ptr(v), h, nq, nk, int(leaf), d, int(kx), int(sink), int(stride), tile, int(group), g0, gn, ptr(perm),
@@ -648,7 +648,7 @@ def run_windows(packed: dict, q, mu, *, nb: int, leaf: int, kx: int, scale: floa
         elif store == torch.int8:
             b["sg"] = rows("sg", (nbp,), torch.float32)
             b["keys"] = rows("route_keys", (nbp,), torch.int32) if nb > ROUTE_NB_LDS else None
-            size = max(h * tiles(*w) * (s if (s := route_segments(h * tiles(*w), nb, kx, leaf)) > 1 else 0) for w in mine)
+            size = max(h * tiles(*w) * (s if (s := route_segments(h * nt, h * tiles(*w), nb, kx, leaf)) > 1 else 0) for w in mine)
             b["parts"] = None
             if size:
                 live.append(_buf(ws, "parts", (size * tile * (D + 1),), torch.float32, dev))

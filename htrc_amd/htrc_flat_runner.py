@@ -63,15 +63,15 @@ def _ceil(a: int, b: int) -> int:
 F32_UNSPLIT_TILES = 2048
 
 
-# Fused int8 route: the segments whose partial sums a launch of ``units`` (head, tile) pairs keeps in
-# workspace (htrc_route_segments of the C ABI): tiles of more than 128 blocks of 32 keys, in launches of at
-# most 384 pairs and heads of at most 16384 leaves.
-SEG_MIN_BLOCKS, SEG_MAX, SEG_SPLIT_TILES, SEG_MAX_NB = 128, 4, 384, 16384
+# Fused int8 route: the segments whose partial sums a launch of ``units`` of a layer's ``tiles`` (head, tile) pairs
+# keeps in workspace (htrc_route_segments of the C ABI): tiles of more than 128 blocks of 32 keys, in layers of 513 to
+# 1024 pairs and launches of at most 384, and heads of at most 16384 leaves.
+SEG_MIN_BLOCKS, SEG_MAX, SEG_SPLIT_TILES, SEG_MAX_NB, SEG_TILES_MIN, SEG_TILES_MAX = 128, 4, 384, 16384, 512, 1024
 
 
-def route_segments(units: int, nb: int, kx: int, leaf: int) -> int:
+def route_segments(tiles: int, units: int, nb: int, kx: int, leaf: int) -> int:
     blocks = _ceil(nb, 32) + _ceil(kx * leaf, 32)
-    if units > SEG_SPLIT_TILES or blocks <= SEG_MIN_BLOCKS or nb > SEG_MAX_NB:
+    if not SEG_TILES_MIN < tiles <= SEG_TILES_MAX or units > SEG_SPLIT_TILES or blocks <= SEG_MIN_BLOCKS or nb > SEG_MAX_NB:
         return 1
     return min(SEG_MAX, _ceil(blocks, 32))
 
@@ -117,7 +117,7 @@ def workspace_bytes(queries: int, keys: int, leaf: int = 16, dim: int = 128, hea
     if fused and store == "int8":
         # partial sums of long tiles (the last window's where only that one is small enough)
         for t in (tw, nt - (_ceil(nt, tw) - 1) * tw):
-            segs = route_segments(int(heads) * t, nb, kx, int(leaf))
+            segs = route_segments(int(heads) * nt, int(heads) * t, nb, kx, int(leaf))
             if segs > 1:
                 window += t * segs * int(tile) * (dim + 1) * 4
                 break

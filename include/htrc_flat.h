@@ -167,7 +167,7 @@ int htrc_route(const int8_t* q8, const float* sq, const int8_t* dq8, const float
                float* logz, int32_t* idx, float* rowmax, uint32_t* keys_ws, void* stream);
 
 /* htrc_route for tiles of many keys: a tile of more than 128 32-key blocks (far leaves and near
- * tokens) is summed in htrc_route_segments() segments whose order the tile's block count alone
+ * tokens) in a layer of 513 to 1024 (head, tile) pairs is summed in segments whose order its block count
  * fixes, so every window and launch of a layer gives the same bits.  parts (fp32, 16-byte aligned,
  * heads * tiles of the window * segments * T * 129 floats; NULL when htrc_route_segments() is 1)
  * takes the segments' sums where the window is small enough that they run as workgroups of their

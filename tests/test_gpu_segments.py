@@ -17,8 +17,9 @@ from htrc_amd._lib import call, ptr, stream_handle
 pytestmark = pytest.mark.gpu
 
 
-def _route(device, n, m, leaf, kx, tile, heads, group, spike):
-    q, k, v = workloads.clustered_runs(n=max(n, m), runs=-(-max(n, m) // 64), heads=heads, seed=leaf + tile)
+def _route(device, n, m, leaf, kx, tile, group, g0, gn, spike):
+    """The window [g0, g0 + gn) of tile groups of one head through the three forms -> (segments, outputs of its rows)."""
+    q, k, v = workloads.clustered_runs(n=max(n, m), runs=-(-max(n, m) // 64), heads=1, seed=leaf + tile)
     q, k, v = q[:, :n].clone(), k[:, :m].contiguous(), v[:, :m].contiguous().to(device)
     if spike:                             # key 3 (leaf 0, always near) far above row 5's far-field maximum
         q, k = (q.float() * 0.3).to(torch.bfloat16), (k.float() * 0.3).to(torch.bfloat16)
@@ -28,38 +29,45 @@ def _route(device, n, m, leaf, kx, tile, heads, group, spike):
     mu, q8, sq, dq8, sdq = hip.pack_q(q, tile=tile, group=group)
     k8, ks = hip.pack_k(k)
     nb, nt, scale = m // leaf, -(-n // tile), 1 / math.sqrt(128)
-    g8, lz, vb, sg, _ = hip.leaf_stats(mu, k, v, nb, scale, leaf=leaf)
-    ng = int(mu.shape[1])
+    units = min(nt, (g0 + gn) * group) - g0 * group
+    rows = slice(g0 * group * tile, min(n, (g0 * group + units) * tile))
+    g8, lz, vb, sg, _ = hip.leaf_stats(mu, k, v, nb, scale, leaf=leaf, c0=g0, cn=gn)
     kxe = min(kx, nb)
-    segs = hip.library().htrc_route_segments(heads, n, m, leaf, kx, tile, group, 0, ng)
-    assert segs == htrc_flat_runner.route_segments(heads * nt, nb, kxe, leaf)
+    segs = hip.library().htrc_route_segments(1, n, m, leaf, kx, tile, group, g0, gn)
+    assert segs == htrc_flat_runner.route_segments(nt, units, nb, kxe, leaf)
     outs = []
     for entry, parts in (("htrc_route_seg", True), ("htrc_route_seg", False), ("htrc_route", None)):
-        out, lzr = torch.full((heads, n, 128), 7.0, device=device), torch.full((heads, n), 7.0, device=device)
-        idx = torch.empty((heads, ng, kxe), dtype=torch.int32, device=device)
-        rowmax = torch.empty((heads, nt * tile), device=device)
-        buf = torch.empty((heads * nt * segs * tile * 129,), device=device) if parts and segs > 1 else None
+        out, lzr = torch.full((1, n, 128), 7.0, device=device), torch.full((1, n), 7.0, device=device)
+        idx = torch.empty((1, gn, kxe), dtype=torch.int32, device=device)
+        rowmax = torch.empty((1, nt * tile), device=device)
+        buf = torch.empty((units * segs * tile * 129,), device=device) if parts and segs > 1 else None
         extra = () if parts is None else (ptr(buf),)
-        call(entry, *[ptr(t) for t in (q8, sq, dq8, sdq, g8, sg, lz, vb, k8, ks, v)], heads, n, m, leaf, 128, kx,
-             int(spike), 1, tile, group, 0, ng, None, scale, ptr(out), ptr(lzr), ptr(idx), ptr(rowmax), None, *extra,
+        call(entry, *[ptr(t) for t in (q8, sq, dq8, sdq, g8, sg, lz, vb, k8, ks, v)], 1, n, m, leaf, 128, kx,
+             int(spike), 1, tile, group, g0, gn, None, scale, ptr(out), ptr(lzr), ptr(idx), ptr(rowmax), None, *extra,
              stream_handle(device))
-        outs.append((out, lzr))
+        outs.append((out[0, rows], lzr[0, rows]))
+        # no other row is written
+        assert bool((out[0, : rows.start] == 7).all()) and bool((out[0, rows.stop:] == 7).all())
     torch.cuda.synchronize()
     return segs, outs
 
 
-@pytest.mark.parametrize("n,m,leaf,kx,tile,heads,group,spike,segs", [
-    (200, 4128, 16, 240, 64, 1, 1, False, 4),       # 9 + 120 blocks: the shortest segmented tile
-    (200, 4112, 16, 239, 64, 1, 1, False, 4),       # 9 + 119.5 blocks: a half-empty last block
-    (193, 2048, 16, 128, 64, 1, 1, False, 1),       # 4 + 64 blocks: whole tiles
-    (200, 4128, 32, 129, 32, 2, 1, False, 4),       # 5 + 129 blocks, 32-row tiles
-    (1000, 40752, 16, 256, 64, 1, 2, False, 4),     # 80 + 128 blocks, shared centres
-    (130, 33024, 128, 100, 64, 1, 1, False, 4),     # 9 + 400 blocks, a partial last tile
-    (4160, 8192, 64, 66, 32, 4, 1, False, 1),       # 4 + 132 blocks, 520 tiles: in turn, no workspace
-    (500, 8192, 16, 300, 64, 1, 1, True, 4),        # a row whose reference misses: the tile is redone
-    (500, 8192, 64, 64, 32, 1, 1, True, 4)])
-def test_segmented_route(device, n, m, leaf, kx, tile, heads, group, spike, segs):
-    got, ((o1, z1), (o2, z2), (o3, z3)) = _route(device, n, m, leaf, kx, tile, heads, group, spike)
+@pytest.mark.parametrize("n,m,leaf,kx,tile,group,g0,gn,spike,segs", [
+    (33000, 4128, 16, 240, 64, 1, 513, 3, False, 4),    # 9 + 120 blocks: the shortest segmented tile; a partial last tile
+    (33000, 4112, 16, 239, 64, 1, 0, 4, False, 4),      # 9 + 119.5 blocks: a half-empty last block
+    (33000, 2048, 16, 128, 64, 1, 0, 3, False, 1),      # 4 + 64 blocks: whole tiles
+    (32768, 4128, 16, 240, 64, 1, 0, 3, False, 1),      # 512 tiles in the layer: whole tiles
+    (65600, 4128, 16, 240, 64, 1, 0, 3, False, 1),      # 1025 tiles
+    (65536, 4128, 16, 240, 64, 1, 0, 3, False, 4),      # 1024 tiles
+    (17000, 4128, 32, 129, 32, 1, 5, 6, False, 4),      # 5 + 129 blocks, 32-row tiles
+    (33000, 40752, 16, 256, 64, 2, 100, 8, False, 4),   # 80 + 128 blocks, shared centres
+    (33000, 33024, 128, 100, 64, 1, 0, 3, False, 4),    # 9 + 400 blocks
+    (33000, 8192, 64, 66, 64, 1, 0, 384, False, 4),     # the largest launch that runs segments apart
+    (33000, 8192, 64, 66, 64, 1, 0, 385, False, 1),     # in turn, no workspace
+    (33000, 8192, 16, 300, 64, 1, 0, 8, True, 4),       # a row whose reference misses: the tile is redone
+    (17000, 8192, 64, 64, 32, 1, 0, 8, True, 4)])
+def test_segmented_route(device, n, m, leaf, kx, tile, group, g0, gn, spike, segs):
+    got, ((o1, z1), (o2, z2), (o3, z3)) = _route(device, n, m, leaf, kx, tile, group, g0, gn, spike)
     assert got == segs
     assert torch.equal(o1, o2) and torch.equal(z1, z2)
     assert bool(torch.isfinite(o1).all()) and bool(torch.isfinite(z1).all())
