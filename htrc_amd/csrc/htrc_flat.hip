@@ -2499,13 +2499,15 @@ struct RowsN {         // softmax state of the 16 RB rows of one wave
     f32x4 o[RB][8];    // O^T per row block: dims 16db + 4grp + i of row 16rb + lane%16
 };
 
-// 0 when every partial output of the wave's row block is finite, else NaN.
+// 0 when every partial output of the wave's row block is at most 1 / PARTS of the largest float, so that the sum
+// of PARTS such blocks is finite too, else NaN.
+template <int PARTS>
 __device__ __forceinline__ float finite_zero(const f32x4 (&o)[8]) {
     float z = 0.0f;
 #pragma unroll
     for (int db = 0; db < 8; ++db)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) z = __fmaf_rn(o[db][i], 0.0f, z);
+        for (int i = 0; i < 4; ++i) z = __fmaf_rn(__fmul_rn(o[db][i], (float)PARTS), 0.0f, z);
     return z;
 }
 
@@ -2549,7 +2551,8 @@ constexpr int MAX_PASSES = 2;
 // tokens whose scores spread by 11 nats a row's total is -0.2 to 116 octaves above its largest far-field score,
 // and with the range [-60, 64] a quarter of the tiles were computed twice.  Totals in [REF_MIN, REF_MAX]
 // are 48 octaves below to 136 above it, and keep every key of weight 2^-42 or more in a float's normal
-// range; a row of outputs that overflows at such a total (values past 2^27) also sends its tile to the redo.
+// range; a row of outputs that overflows at such a total (values past 2^27), or could once its key parts or
+// segments are added, also sends its tile to the redo.
 constexpr float REF_SHIFT = 36.0f, REF_MIN = 0x1p-84f, REF_MAX = 0x1p100f;
 __device__ __forceinline__ float row_reference(float m) {
     return m == -INFINITY ? 0.0f : __fadd_rn(__fmul_rn(m, LOG2E), REF_SHIFT);
@@ -3263,7 +3266,7 @@ __device__ __forceinline__ void route_body(
         if constexpr (MODE == ROUTE_SEGS) {
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
-                sum.l[rb] = __fadd_rn(sum.l[rb], grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero(st.o[rb])) : st.l[rb]));
+                sum.l[rb] = __fadd_rn(sum.l[rb], grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero<SEG_MAX>(st.o[rb])) : st.l[rb]));
 #pragma unroll
                 for (int db = 0; db < 8; ++db)
 #pragma unroll
@@ -3277,7 +3280,7 @@ __device__ __forceinline__ void route_body(
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
                 const int r = 16 * RB * hr + 16 * rb + col;
-                const float lt = grp_sum(__fadd_rn(st.l[rb], finite_zero(st.o[rb])));
+                const float lt = grp_sum(__fadd_rn(st.l[rb], finite_zero<SEG_MAX>(st.o[rb])));
                 if (grp == 0) part_l[pb + r] = lt;
 #pragma unroll
                 for (int db = 0; db < 8; ++db) *(f32x4*)(part_o + (pb + r) * D + 16 * db + 4 * grp) = st.o[rb][db];
@@ -3292,7 +3295,7 @@ __device__ __forceinline__ void route_body(
         for (int rb = 0; rb < RB; ++rb) {
             float lt;
             if constexpr (MODE == ROUTE_SEGS) lt = sum.l[rb];
-            else lt = grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero(st.o[rb])) : st.l[rb]);
+            else lt = grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero<NP>(st.o[rb])) : st.l[rb]);
             if (grp == 0) red_l[pr][16 * RB * hr + 16 * rb + col] = lt;
         }
         if (threadIdx.x == 0) redo = 0;
@@ -4026,7 +4029,7 @@ __global__ __launch_bounds__(64 * NW, 2) void route16_kernel(
         // once at every row's exact largest score, where each row total lies in [1, keys]
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-            const float lt = grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero(st.o[rb])) : st.l[rb]);
+            const float lt = grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero<1>(st.o[rb])) : st.l[rb]);
             if (grp == 0) red_l[16 * RB * wv + 16 * rb + col] = lt;
         }
         if (threadIdx.x == 0) redo = 0;

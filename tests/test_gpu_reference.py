@@ -41,3 +41,32 @@ def test_scores_far_above_the_reference(device, store, heads, mag, vexp):
     s = 2.0 ** -vexp
     assert rel_l2(out[h, :64].cpu().numpy() * s, np.asarray(ref["out"]) * s) <= OUT_REL_L2
     assert np.abs(logz[h, :64].cpu().numpy() - ref["logz"]).max() <= LOGZ_ABS
+
+
+@pytest.mark.parametrize("heads,n,m,sink,far,chunk", [
+    (1, 4096, 4096, 8, 7, None),      # four key parts: the two keys in the first and the last
+    (6, 4096, 4096, 8, 7, None),      # two key parts
+    (8, 4096, 4096, 8, 7, None),      # one key part
+    (1, 33000, 8192, 66, 40, None),   # four segments in turn: the two keys in the first and the third
+    (1, 33000, 8192, 66, 40, 128)])   # the segments as workgroups of their own
+def test_sums_over_parts_that_overflow(device, heads, n, m, sink, far, chunk):
+    """Two near keys of one weight (121 octaves) in different parts of the tile's key stream, their value 1.5 * 2^e: at one
+    e of the sweep each part's output is finite and their sum is not.  Their common value is the
+    row's output (every other weight is below 2^-90 of theirs), up to the weights' bf16 rounding."""
+    leaf, row, mag = 64, 5, 30.75
+    q, k, v = (x.to(device) for x in workloads.clustered_runs(n=max(n, m), runs=max(n, m) // 64, heads=heads, seed=19))
+    q, k = ((x.float() * 0.3).to(torch.bfloat16) for x in (q[:, :n], k[:, :m]))
+    v = v[:, :m].contiguous()
+    keys = [3, far * leaf + 3]
+    q[:, row], k[:, keys] = 0, 0
+    q[..., 0], k[..., 0] = 0, 0           # dim 0 is theirs alone: no other row's centre or leaf mean points at them
+    q[:, row, 0] = mag
+    k[:, keys, 0] = mag
+    ws = {}
+    for e in range(72):
+        v[:, keys] = 1.5 * 2.0 ** e
+        out, logz = htrc_flat.flat_attention(q, k, v, backend="hip", store="int8", dot="bf16", leaf=leaf, exact_leaves=0,
+                                             sink_leaves=sink, tile_chunk=chunk, ws=ws, return_logz=True)
+        finite = bool(torch.isfinite(out).all()) and bool(torch.isfinite(logz).all())
+        assert finite, e
+        assert float((out[:, row] * (2.0 ** -e / 1.5) - 1).abs().max()) <= 1e-2, e
