@@ -2545,18 +2545,17 @@ constexpr size_t ROUTE_LDS_MAX = 160 * 1024;         // LDS of one workgroup on 
 // Passes of a tile in the route kernels: one at the select launch's reference, and when a row
 // total leaves range one more at every row's exact largest score (in range by construction).
 constexpr int MAX_PASSES = 2;
-// The fixed softmax reference of a row is its largest far-field score plus REF_SHIFT octaves.  A leaf's
-// far-field score is a lower bound of the leaf's exact log-mass (the log-sum-exp is convex in the row),
-// so a near leaf's exact score can lie far above the reference and hardly below: over heads of 40759
-// tokens whose scores spread by 11 nats a row's total is -0.2 to 116 octaves above its largest far-field score,
-// and with the range [-60, 64] a quarter of the tiles were computed twice.  Totals in [REF_MIN, REF_MAX]
-// are 48 octaves below to 136 above it, and keep every key of weight 2^-42 or more in a float's normal
-// range; a row of outputs that overflows at such a total (values past 2^27), or could once its key parts or
-// segments are added, also sends its tile to the redo.
-constexpr float REF_SHIFT = 36.0f, REF_MIN = 0x1p-84f, REF_MAX = 0x1p100f;
-__device__ __forceinline__ float row_reference(float m) {
-    return m == -INFINITY ? 0.0f : __fadd_rn(__fmul_rn(m, LOG2E), REF_SHIFT);
-}
+// The fixed softmax reference of a row is its largest far-field score.  A leaf's far-field score is a lower bound of
+// the leaf's exact log-mass (the log-sum-exp is convex in the row), so a near leaf's exact score can lie far
+// above the reference and hardly below: over heads of 40759 tokens whose scores spread by 11 nats a row's total is -0.2
+// to 116 octaves above it, and with totals up to 2^64 a quarter of those tiles were computed twice.  Totals in
+// [REF_MIN, REF_MAX] are taken as they are: all that a float holds but for the room that keeps 1 / total a normal
+// number.  A row of outputs that overflows at such a total, or could once its key parts or segments are
+// added, also sends its tile to the redo.  (A reference 36 octaves higher takes totals up to 2^136: six of those heads
+// a call 3672 us against 3692 here, 0.5 % between runs.  But it puts an ordinary row's outputs at 2^-36 of its
+// values, and values below 2^-66 then lose bits.)
+constexpr float REF_MIN = 0x1p-60f, REF_MAX = 0x1p125f;
+__device__ __forceinline__ float row_reference(float m) { return m == -INFINITY ? 0.0f : __fmul_rn(m, LOG2E); }
 // Merge: the wave pairs' partial O, 64 rows x 128 dims each, rows padded to 132 floats.
 constexpr int MRG_STRIDE = 132;
 // Ring slots per pair: blocks are loaded RS - 1 ahead.  Two slots (one block in flight while the
@@ -3445,8 +3444,8 @@ __global__ __launch_bounds__(64 * NH, RB == 2 ? 2 : 3) void route_seg_kernel(ROU
 //     are read.  Far: score = (dq . g) (* 256 sg) + lz, PV with
 //     fp16(p * 256 sv) . vb (fp8) or bf16(p) . vb (bf16); near: score = (q . k) * scale (bf16),
 //     PV bf16(p) . v -- the products of tile16_kernel, in one softmax whose reference is the
-//     row's far-field maximum, REF_SHIFT octaves up for the bf16 store (redone with a moved reference
-//     if a row total leaves its range, as route_kernel).
+//     row's far-field maximum (redone with a moved reference if a row total leaves its range, as
+//     route_kernel).
 // ---------------------------------------------------------------------------------------------
 // 16-byte position of chunk c of row r of 128-byte rows (e4m3 codes) staged in LDS: c ^ sw8(r).
 // A read of 8 bytes per lane whose 32 lanes touch 16 rows, rows 16 h + 0..15 or 4 g + 0..3,
@@ -3787,7 +3786,7 @@ __global__ __launch_bounds__(64 * NW, 2) void route16_kernel(
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
         const float m = rowmax[prow0 + 16 * rb];
-        mref[rb] = FP8 ? (m == -INFINITY ? 0.0f : __fmul_rn(m, LOG2E)) : row_reference(m);   // (fp8: far P is fp16)
+        mref[rb] = row_reference(m);
     }
     // B operands of the rows: q - mu through the far blocks, then q through the near blocks (one
     // register set, reloaded at the switch)
@@ -4024,9 +4023,10 @@ __global__ __launch_bounds__(64 * NW, 2) void route16_kernel(
                 if (bi + 1 < nblk) near_step(P1(), bi + 1);
             }
         }
-        // row totals: outside [REF_MIN, REF_MAX] the reference missed the row's maximum (below 2^-8 with the fp8 store: its far-field P is fp16, whose subnormals would hold
-        // the far leaves of a row whose total is that small with too few bits): the tile is redone
-        // once at every row's exact largest score, where each row total lies in [1, keys]
+        // row totals: outside [REF_MIN, REF_MAX] the reference missed the row's maximum (below 2^-8
+        // with the fp8 store: its far-field P is fp16, whose subnormals would hold the far leaves of
+        // a row whose total is that small with too few bits): the tile is redone once at every row's
+        // exact largest score, where each row total lies in [1, keys]
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
             const float lt = grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero<1>(st.o[rb])) : st.l[rb]);

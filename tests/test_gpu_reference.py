@@ -70,3 +70,22 @@ def test_sums_over_parts_that_overflow(device, heads, n, m, sink, far, chunk):
         finite = bool(torch.isfinite(out).all()) and bool(torch.isfinite(logz).all())
         assert finite, e
         assert float((out[:, row] * (2.0 ** -e / 1.5) - 1).abs().max()) <= 1e-2, e
+
+
+@pytest.mark.parametrize("store,heads", [("int8", 1), ("int8", 6), ("int8", 8), ("bf16", 1)])
+@pytest.mark.parametrize("vexp", [-60, -90, -100, -110])
+def test_small_values(device, store, heads, vexp):
+    """Values scaled by a power of two scale the outputs by it, in every dim or in half of them: a row's weights lie near
+    1 or above, so outputs of 2^-110 are sums whose roundings, 2^-150 each where they fall below the normal range,
+    are 4096 keys * 2^-40 of them at most.  (The statistics' own roundings move by 4e-7 under the scale.)"""
+    n, leaf, ex = 4096, 64, 4
+    q, k, v = (x.to(device) for x in workloads.clustered_runs(n=n, runs=n // 64, heads=heads, seed=23))
+    kw = dict(backend="hip", store=store, dot="bf16", leaf=leaf, exact_leaves=ex, tile_chunk=None)
+    want = htrc_flat.flat_attention(q, k, v, **kw)
+    s = 2.0 ** vexp
+    for dims in (slice(0, 128), slice(64, 128)):
+        small = v.clone()
+        small[..., dims] *= s
+        got = htrc_flat.flat_attention(q, k, small, **kw)
+        rel = rel_l2((got[..., dims] / s).cpu().numpy(), want[..., dims].cpu().numpy())
+        assert rel <= 2e-6, (dims, rel)

@@ -11,9 +11,9 @@ reference-max retry on the GPU, against the CPU oracle.
 * 20000 leaves per head: route_select keeps its top-k keys in global memory, the stage top-k
   reads rows from global memory.
 * A query row aligned with a near-field outlier key scores 80 or 362 nats above its far-field
-  maximum (or, under a sampled tile reference, every other row scores ~300 nats below it), so the
-  fixed softmax reference misses by more than 60 octaves and the tile is redone at every row's
-  exact largest score.
+  maximum (or, under a sampled tile reference, every other row scores ~300 nats below it): the
+  first is near the top of the row totals the fixed softmax reference takes (2^125), the others
+  leave their range and the tile is redone at every row's exact largest score.
 
 Routing is compared with the oracle through the measured SEL error (helpers.routing_report):
 a tile's near set may differ only where the oracle's top-k boundary gap is at most twice the
@@ -186,8 +186,8 @@ def test_many_leaves_vs_oracle(device, fused):
 def test_reference_max_retry(device, heads, store, mag, stride):
     """Row r of tile 0 is mag e_0 and key 3 of leaf 0 (a sink, so always near) is mag e_0: its exact
     score mag^2 / sqrt(128) (80 nats at mag 30, 362 at 64) sits far above the row's far-field
-    maximum, the row total at the fixed reference leaves [2^-60, 2^64] (overflows fp32 at 64) and
-    the tile is redone at every row's exact largest score.  With sel_stride 2 the row is sampled
+    maximum: at mag 30 the row total stays within [2^-60, 2^125] (2^115 at most), at 64 it overflows
+    fp32 and the tile is redone at every row's exact largest score.  With sel_stride 2 the row is sampled
     and its far-field maximum (~300 nats at 64) is the reference of the whole tile: every other
     row's total underflows to zero and is redone too.  1, 6 and 8 heads of 64 tiles take the attend
     kernel's four-, two- and one-pair shapes; the 16-bit stores take their own fused route."""
