@@ -358,25 +358,22 @@ def flat_attention(q, k, v, *, tile=64, exact_leaves=64, order="seq", curvature=
     if pipe:
         cur = torch.cuda.current_stream(qh.device)
         side = _window_streams(qh.device, nst)
-        for s in side:
-            s.wait_stream(cur)
         wsw = (None,) * nst if ws is None else tuple(ws.setdefault(f"window_{i}", {}) for i in range(nst))
     # Without checks, stage timing or state changes between the stages, one native call launches every
-    # window (its buffers from the caller's stream: the side streams are joined below before they are freed)
+    # window (its buffers allocated on the caller's stream, to which it orders the side streams itself)
     native = (prof is None and state is None and not quant.get("state") and select == "max"
               and (fused or (f32dots and kx > 0)))
     if native:
-        try:
-            with torch.cuda.device(qh.device) if pipe else contextlib.nullcontext():
-                hip.run_windows(packed, qsrc, mu, nb=nb, leaf=int(leaf), kx=kx, scale=scale, store=sdt, f32dots=f32dots,
-                                wins=wins, sink=sink, stride=stride, tile=tile, group=group, perm=perm, prec=prec,
-                                splits=max(1, int(splits)), bn=int(kern.get("tile_bn", 32)), unsplit=F32_UNSPLIT_TILES,
-                                rowmax=rowmax, out=out, logz=logz, wss=wsw if pipe else (ws,),
-                                streams=[s.cuda_stream for s in side] if pipe else [hip.stream_handle(qh.device)])
-        finally:
-            for s in side if pipe else ():
-                cur.wait_stream(s)
+        with torch.cuda.device(qh.device) if pipe else contextlib.nullcontext():
+            hip.run_windows(packed, qsrc, mu, nb=nb, leaf=int(leaf), kx=kx, scale=scale, store=sdt, f32dots=f32dots,
+                            wins=wins, sink=sink, stride=stride, tile=tile, group=group, perm=perm, prec=prec,
+                            splits=max(1, int(splits)), bn=int(kern.get("tile_bn", 32)), unsplit=F32_UNSPLIT_TILES,
+                            rowmax=rowmax, out=out, logz=logz, wss=wsw if pipe else (ws,),
+                            side=side if pipe else (), cur=cur if pipe else None)
         pipe, wins = False, []
+    if pipe:
+        for s in side:
+            s.wait_stream(cur)
     for wi, (g0, gn) in enumerate(wins):
         with torch.cuda.stream(side[wi % nst]) if pipe else contextlib.nullcontext():
             _window(wsw[wi % nst] if pipe else ws, g0, gn)

@@ -604,10 +604,13 @@ def route16_fits(nb: int, kx: int) -> bool:
 
 def run_windows(packed: dict, q, mu, *, nb: int, leaf: int, kx: int, scale: float, store, f32dots: bool, wins, sink: int,
                 stride: int, tile: int, group: int, perm, prec: str, splits: int, bn: int, unsplit: int, rowmax, out, logz,
-                wss, streams):
+                wss, side=(), cur=None):
     """The tile windows ``wins`` [(g0, gn), ...] of a layer in one native call (htrc_windows_*): window i on the stream
-    handle streams[i % n] with the buffers of the workspace wss[i % n] (the names and sizes of the per-stage
-    functions above).  packed, q, mu as flat_attention builds them; kx > 0 for the fp32 dots."""
+    side[i % n] (n = 1 without side streams: the current one) with the buffers of the workspace wss[i % n] (the names and
+    sizes of the per-stage functions above).  packed, q, mu as flat_attention builds them; kx > 0 for the fp32 dots.
+    The buffers are allocated on the caller's stream ``cur`` and used on the side streams: those wait for it after the last
+    allocation, since a block may come from another thread of the same stream whose kernels still read it, and it for
+    them before the first buffer is dropped, since the next owner's kernels wait for ``cur`` alone."""
     k, v = packed["k"], packed["v"]
     _need(mu, torch.float32, "mu")
     _need(k, torch.bfloat16, "k")
@@ -625,8 +628,8 @@ def run_windows(packed: dict, q, mu, *, nb: int, leaf: int, kx: int, scale: floa
     def tiles(g0, gn):
         return min(nt, (g0 + gn) * group) - g0 * group
 
-    live, bufs = [], []
-    n = len(streams)
+    live, bufs = [], []                                 # live: the buffers, held until the streams are joined
+    n = max(1, len(side))
     for i in range(n):
         ws, mine = wss[i], wins[i::n]
         gn = mine[0][1]                                 # the largest window of the stream (only the layer's last is smaller)
@@ -661,18 +664,25 @@ def run_windows(packed: dict, q, mu, *, nb: int, leaf: int, kx: int, scale: floa
             names = ("terms", "g", "sg", "vb", "sv", "lz", "idx")
         bufs += [b[x] for x in names]
     bufs = (ctypes.c_void_p * len(bufs))(*bufs)
-    handles = (ctypes.c_void_p * n)(*streams)
+    handles = (ctypes.c_void_p * n)(*([s.cuda_stream for s in side] or [stream_handle(dev)]))
     shape = (h, nq, nk, leaf, d, kx, sink, stride, tile, group, wins[0][1])
     tail = (float(scale), ptr(rowmax), ptr(out), ptr(logz), n, bufs, handles)
-    if f32dots:
-        call("htrc_windows_f32", ptr(q), int(q.dtype == torch.bfloat16), ptr(mu), ptr(k), ptr(v), *shape, splits, bn, unsplit,
-             ptr(perm), int(store == torch.bfloat16), tf32, tail[0], *tail[2:])
-    elif store == torch.int8:
-        call("htrc_windows_i8", ptr(mu), ptr(k), ptr(v), *(ptr(packed[x]) for x in ("q8", "sq", "dq8", "sdq", "k8", "ks")),
-             *shape, ptr(perm), tf32, *tail)
-    else:
-        call("htrc_windows_16", ptr(mu), ptr(k), ptr(v), ptr(packed["q16"]), ptr(packed["dq16"]), *shape, ptr(perm),
-             int(fp8), tf32, *tail)
+    for s in side:
+        s.wait_stream(cur)
+    try:
+        if f32dots:
+            call("htrc_windows_f32", ptr(q), int(q.dtype == torch.bfloat16), ptr(mu), ptr(k), ptr(v), *shape, splits, bn, unsplit,
+                 ptr(perm), int(store == torch.bfloat16), tf32, tail[0], *tail[2:])
+        elif store == torch.int8:
+            call("htrc_windows_i8", ptr(mu), ptr(k), ptr(v), *(ptr(packed[x]) for x in ("q8", "sq", "dq8", "sdq", "k8", "ks")),
+                 *shape, ptr(perm), tf32, *tail)
+        else:
+            call("htrc_windows_16", ptr(mu), ptr(k), ptr(v), ptr(packed["q16"]), ptr(packed["dq16"]), *shape, ptr(perm),
+                 int(fp8), tf32, *tail)
+    finally:
+        for s in side:
+            cur.wait_stream(s)
+    del live
 
 
 def tail_merge(q, tk, tv, *, scale: float, out, logz, f32dots: bool = False, prec: str = "ieee"):
