@@ -367,9 +367,9 @@ def flat_attention(q, k, v, *, tile=64, exact_leaves=64, order="seq", curvature=
         with torch.cuda.device(qh.device) if pipe else contextlib.nullcontext():
             hip.run_windows(packed, qsrc, mu, nb=nb, leaf=int(leaf), kx=kx, scale=scale, store=sdt, f32dots=f32dots,
                             wins=wins, sink=sink, stride=stride, tile=tile, group=group, perm=perm, prec=prec,
-                            splits=max(1, int(splits)), bn=int(kern.get("tile_bn", 32)), unsplit=F32_UNSPLIT_TILES,
-                            rowmax=rowmax, out=out, logz=logz, wss=wsw if pipe else (ws,),
-                            side=side if pipe else (), cur=cur if pipe else None)
+                            splits=splits, bn=kern.get("tile_bn", 32), unsplit=F32_UNSPLIT_TILES, rowmax=rowmax,
+                            out=out, logz=logz, wss=wsw if pipe else (ws,), side=side if pipe else (),
+                            cur=cur if pipe else None)
         pipe, wins = False, []
     if pipe:
         for s in side:

@@ -77,3 +77,17 @@ def test_side_streams_are_ordered_around_the_buffers(events, kw, streams, ws, re
         assert joins and at < max(joins)
         assert all(i > max(joins) for i in drops), "a buffer is dropped before the streams are joined"
     assert ws or refused or len(drops) == len(allocs)
+
+
+@pytest.mark.parametrize("store,chunk", [("int8", 2), ("int8", None), ("fp8", 2), ("bf16", None)])
+def test_fused_routes_do_not_look_at_the_split_knobs(events, store, chunk):
+    q, k, v = (torch.zeros((n, 128), dtype=torch.bfloat16) for n in (300, 256, 256))
+    htrc_flat.flat_attention(q, k, v, backend="hip", store=store, dot="bf16", leaf=32, exact_leaves=2, tile_chunk=chunk,
+                             splits=None, kern={"tile_bn": None})
+    assert [e for e in events if e[0] == "call" and e[1].startswith("htrc_windows")]
+
+
+def test_unsplit_windows_do_not_look_at_splits(events):
+    q, k = torch.zeros((2, 65536, 128), dtype=torch.bfloat16), torch.zeros((2, 512, 128), dtype=torch.bfloat16)
+    htrc_flat.flat_attention(q, k, k, backend="hip", leaf=128, exact_leaves=1, tile_chunk=None, splits=None)
+    assert ("call", "htrc_windows_f32") in events
