@@ -2849,34 +2849,39 @@ __device__ __forceinline__ RowMax<RB> route_exact_max(const int8_t* dq8, const f
     return mx;
 }
 
-// Long tiles: a tile whose far and near fields are more than SEG_MIN_BLOCKS 32-key blocks has its
-// block stream (far, then near) cut into route_segments() equal segments, each summed from zero,
-// and the segments' sums added in order.  That order is fixed by the tile's block count alone, so the
-// segments may run as workgroups of their own (route_part_kernel, partial sums in workspace,
-// combined by route_seg_kernel) or one after the other in one workgroup (route_seg_kernel), bit for bit alike:
-// the launch takes the first where a window's tiles alone leave the CUs short of waves.
-// Measured on heads of 40759 tokens (leaf 16): a 128-tile window of 208 blocks 178 us whole (one wave
-// pair a tile: 256 waves for 1024 SIMDs), 50 + 22 us in parts (the head 965 -> 706 us a call); 256 tiles
-// of 592 blocks 507 -> 270 + 30 us; 768 tiles of 318 blocks 605 whole, 587 + 92 in parts, 556 in turn,
-// so launches of more than 384 tiles run in turn (384 tiles split 1521, in turn 1559 us a call; 512 1983 and 1911).  4 segments against 6, 8 and 16: 706 / 715 / 720 /
-// 720 us.  Below 128 blocks the whole-tile kernels' key halves and quarters serve.
+// Long tiles: in layers of a middling number of tiles, a tile whose far and near fields are more than SEG_MIN_BLOCKS
+// 32-key blocks has its block stream (far, then near) cut into SEG_MAX equal segments, each summed from zero, and
+// the segments' sums added in order.  The rule looks at the layer's shape alone (its tiles, leaves and near leaves),
+// so every windowing of a layer sums in the same order: the segments may run as workgroups of their own
+// (route_part_kernel, partial sums in workspace, combined by route_seg_kernel) or one after the other in
+// one workgroup (route_seg_kernel), bit for bit alike.  The launch takes the first where its own tiles leave
+// the CUs short of waves: a 128-tile window of whole tiles is one wave pair a tile, 256 waves for 1024 SIMDs.
+// The lines, in tiles per CU (256 CUs; us a call without and with segments, leaf 16, 256 near leaves unless said):
+//   SEG_TILES_MIN, SEG_TILES_MAX: 516 tiles in windows of 128 702 -> 447, 637 819 -> 555, 1024 1571 -> 1141; in one window
+//   385 -> 387, 478 -> 481, 987 -> 975.  Windows gain outside too (469 tiles 400 -> 345, 1094 1958 -> 1389, 1274
+//   1316 -> 1033), but the rule may not look at the window, and one-window calls lose there: 469 tiles 287 -> 339 (their
+//   whole-tile kernels split each tile's keys over several wave parts), 1094 1228 -> 1330, 1274 848 -> 935, 2548
+//   1566 -> 1637 (more tiles a CU than the in-turn kernel's registers allow).
+//   segments_apart: of 1024 tiles, windows of 300 in turn 1184, apart 1128; of 400 1075 and 1105; of 640 1015 and 1059.
+//   SEG_MIN_BLOCKS: 637 tiles of 208 blocks gain as above, of 592 (1024 near leaves) in windows of 256 1427 -> 753.
+//   Fewer blocks would gain in windows of 128 too (112 blocks 606 -> 485, 84 398 -> 317, 52 326 -> 289, 42 271 -> 269),
+//   not in one window (84 blocks 210 -> 212; 768 tiles of 34 blocks 94 -> 98).
+//   SEG_MAX: 4 segments against 6, 8 and 16 of 208 blocks: 706 / 715 / 720 / 720 us.
 constexpr int SEG_MIN_BLOCKS = 128;
 constexpr int SEG_MAX = 4;
-constexpr int64_t SEG_SPLIT_TILES = 384;             // launches of at most this many tiles run the segments apart
-// The layer's (head, tile) pairs: up to two a CU the whole-tile kernels split each tile's keys over several wave parts
-// (313 tiles in one window 168 us a call, segments 177); past four a CU a launch of the whole layer runs more tiles a CU
-// than the in-turn kernel's registers allow (1250 tiles of one window 839 us whole, 922 in turn; 625 tiles 453 and 457).
-constexpr int64_t SEG_TILES_MIN = 512, SEG_TILES_MAX = 1024;
+constexpr int64_t SEG_TILES_MIN = 2, SEG_TILES_MAX = 4;   // (head, tile) pairs of the layer per CU: above, up to
 enum RouteMode { ROUTE_WHOLE = 0, ROUTE_PART = 1, ROUTE_SEGS = 2 };
 constexpr int SEG_QUARTERS = 4;                      // workgroups per tile that combine its partial sums
 
-// (heads of more than ROUTE_NB_LDS leaves, whose select works from global keys, keep whole tiles)
-inline int route_segments(int64_t tiles, int64_t nb, int kxe, int leaf) {
+// Segments of a layer's tiles.  (Heads of more than ROUTE_NB_LDS leaves, whose select works from global keys, keep
+// whole tiles.)
+inline int route_segments(int64_t tiles, int64_t nb, int kxe, int leaf, int64_t cus) {
     const int64_t blocks = (nb + 31) / 32 + ((int64_t)kxe * leaf + 31) / 32;
-    if (tiles <= SEG_TILES_MIN || tiles > SEG_TILES_MAX || blocks <= SEG_MIN_BLOCKS || nb > ROUTE_NB_LDS) return 1;
-    const int64_t n = (blocks + 31) / 32;
-    return (int)(n < SEG_MAX ? n : SEG_MAX);
+    const bool middling = tiles > SEG_TILES_MIN * cus && tiles <= SEG_TILES_MAX * cus;
+    return middling && blocks > SEG_MIN_BLOCKS && nb <= ROUTE_NB_LDS ? SEG_MAX : 1;
 }
+// Whether a launch of `units` tiles runs them apart: up to one and a half tiles a CU.
+inline bool segments_apart(int64_t units, int64_t cus) { return 2 * units <= 3 * cus; }
 
 // RB 16-row blocks per wave, NH waves per key part (NH = 2: halves of the tile's rows; NH = 4, RB = 1: quarters of
 // a 64-row tile, the same sums per row); NP key parts of NH waves; RS ring slots per part.  MODE ROUTE_WHOLE: the tile's keys in one sum.  ROUTE_PART: workgroup
@@ -3408,16 +3413,17 @@ template <int LEAF, int RB, int NP, int RS>
 __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_kernel(ROUTE_PARAMS) {
     route_body<LEAF, RB, NP, RS, ROUTE_WHOLE, 2>(ROUTE_ARGS, nullptr, nullptr, 1);
 }
-// 64-row tiles with four waves of 16 rows per key part, where there are several: the same sums per row, twice the waves to hide
-// each block's loads in (16 x 32-leaf tiles of two heads of 11008 tokens 97.8 -> 95.5 us a call, one head of 24000
-// tokens 94.9 -> 93.4; 256 tiles and fewer within 1 %).  One key part keeps two waves of 32 rows: there
-// several tiles share a CU, and each LDS read feeds twice the products.
+// 64-row tiles with four waves of 16 rows per key part, where there are several: the same sums per row, twice the waves to
+// hide each block's loads in.  Against two waves of 32 rows, us a call: two key parts, two heads of 11008 tokens 97.8 ->
+// 95.5, one of 24000 94.9 -> 93.4; four, 8192 queries on 32768 keys 93.7 -> 91.5, 16384 tokens in leaf-16
+// windows of 64 tiles 241 -> 233, in one leaf-64 window 68.4 -> 68.3, 4096 tokens 64.6 -> 66.5 (3 % between runs).  One
+// key part keeps two waves of 32 rows: there several tiles share a CU, and each LDS read feeds twice the products.
 template <int LEAF, int NP>
 __global__ __launch_bounds__(256 * NP, NP == 4 ? 4 : 2) void route_rows_kernel(ROUTE_PARAMS) {
     route_body<LEAF, 1, NP, ROUTE_RS, ROUTE_WHOLE, 4>(ROUTE_ARGS, nullptr, nullptr, 1);
 }
 template <int LEAF, int RB, int NH>
-__global__ __launch_bounds__(64 * NH, RB == 2 ? 3 : 4) void route_part_kernel(ROUTE_PARAMS, float* __restrict__ part_o,
+__global__ __launch_bounds__(64 * NH, 4) void route_part_kernel(ROUTE_PARAMS, float* __restrict__ part_o,
                                                                              float* __restrict__ part_l, int nseg) {
     route_body<LEAF, RB, 1, ROUTE_RS, ROUTE_PART, NH>(ROUTE_ARGS, part_o, part_l, nseg);
 }
@@ -5448,11 +5454,11 @@ static int route_attend_launch(const int8_t* q8, const float* sq, const int8_t* 
     const size_t dyn = route_dyn_bytes(nb, kxe);
     // Long tiles (segs: the caller runs them segmented, with workspace for the partial sums where
     // the launch is small; see route_segments)
-    const int nseg = segs ? route_segments(nt * heads, nb, kxe, leaf) : 1;
+    const int nseg = segs ? route_segments(nt * heads, nb, kxe, leaf, cus) : 1;
     if (nseg > 1) {
         REQUIRE(route_static_bytes(1) + dyn <= ROUTE_LDS_MAX, "htrc_route_attend: near list and exclusion bits exceed the LDS");
         const int64_t units = ntw * heads;
-        const bool split = parts && units <= SEG_SPLIT_TILES;
+        const bool split = parts && segments_apart(units, cus);
         REQUIRE(!split || aligned(parts, 16), "htrc_route_attend: misaligned buffer");
         float* part_o = split ? parts : nullptr;
         float* part_l = split ? parts + units * nseg * tile * D : nullptr;
@@ -5460,10 +5466,10 @@ static int route_attend_launch(const int8_t* q8, const float* sq, const int8_t* 
     hipLaunchKernelGGL((K<L, RB, NH>), dim3((unsigned)(units * (N))), dim3(64 * NH), dyn, s, q8, sq, dq8, sdq, g8, sg, lz, \
                        vb, k8, ks, v, idx, rowmax, nq, (int)nt, group, (int)g0, (int)gn, perm, nk, (int)nb, nbp, kxe,  \
                        scale, out, logz, part_o, part_l, nseg)
-        // A 64-row tile's segments run with its rows over four waves (16 each, three or four waves a SIMD): the
-        // launches are short of waves, and each hides the others' loads (128-tile windows of the 40759-token head
-        // 648 -> 587 us a call, 512-tile ones of four heads 1978 -> 1946).  In turn, two waves of 32 rows, whose LDS reads feed twice
-        // the products: 768 tiles a window 3530 against 3612 us a call with four, 2048 tiles 2100 against 2236.
+        // A 64-row tile's segments run with its rows over four waves (16 each, four waves a SIMD): the launches
+        // are short of waves, and each hides the others' loads (128-tile windows of the 40759-token head 648 -> 587 us
+        // a call).  In turn, two waves of 32 rows, whose LDS reads feed twice the products: 768 tiles a window 3530
+        // against 3612 us a call with four.
 #define SEG_SPLIT(L, RB, NH)                                                                                    \
     SEG_LAUNCH(route_part_kernel, L, RB, NH, nseg);                                                             \
     SEG_LAUNCH(route_seg_kernel, L, RB, NH, SEG_QUARTERS);
@@ -5537,7 +5543,8 @@ int htrc_route_segments(int64_t heads, int64_t nq, int64_t nk, int leaf, int kx,
     if (route_shapes("htrc_route_segments", heads, nq, nk, leaf, D, kx, tile, group, g0, gn, nb, nt, ng, tb, ntw, kxe) !=
         HTRC_OK)
         return 0;
-    return ntw * heads <= SEG_SPLIT_TILES ? route_segments(nt * heads, nb, kxe, leaf) : 1;
+    const int64_t cus = device_cus();
+    return segments_apart(ntw * heads, cus) ? route_segments(nt * heads, nb, kxe, leaf, cus) : 1;
 }
 
 int htrc_route_seg(const int8_t* q8, const float* sq, const int8_t* dq8, const float* sdq, const int8_t* g8,

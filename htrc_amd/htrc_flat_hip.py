@@ -438,6 +438,17 @@ ROUTE_MAX_KX = 8192        # near leaves per tile the fused route kernel holds i
 ROUTE_MAX_NB = 262144      # leaves per head of the fused route (exclusion bits in LDS)
 
 
+_CUS: dict = {}
+
+
+def _cus(device) -> int:
+    """Compute units of the device (the launch rules count tiles per CU)."""
+    n = _CUS.get(device)
+    if n is None:
+        n = _CUS[device] = torch.cuda.get_device_properties(device).multi_processor_count
+    return n
+
+
 def route_fits(nb: int, kx: int) -> bool:
     """Whether the fused route takes this shape (else the split tile path runs it)."""
     return int(nb) <= ROUTE_MAX_NB and min(int(kx), int(nb)) <= ROUTE_MAX_KX
@@ -488,7 +499,7 @@ def route(packed: dict, state: dict, *, nq: int, leaf: int, kx: int, scale: floa
     keys = _keys_ws(ws, h, gn, nb, dev)
     # partial sums of the segments of a long tile, where a small window runs them apart
     units = h * (min(nt, (g0 + gn) * int(group)) - g0 * int(group))
-    segs = route_segments(h * nt, units, nb, kxe, int(leaf))
+    segs = route_segments(h * nt, units, nb, kxe, int(leaf), _cus(dev))
     parts = _buf(ws, "parts", (units * segs * tile * (D + 1),), torch.float32, dev) if segs > 1 else None
     call("htrc_route_seg", ptr(q8), ptr(sq), ptr(dq8), ptr(sdq), ptr(g8), ptr(sg), ptr(lz), ptr(vb), ptr(k8), ptr(ks),
          ptr(v), h, nq, nk, int(leaf), d, int(kx), int(sink), int(stride), tile, int(group), g0, gn, ptr(perm),
@@ -654,7 +665,8 @@ def run_windows(packed: dict, q, mu, *, nb: int, leaf: int, kx: int, scale: floa
         elif store == torch.int8:
             b["sg"] = rows("sg", (nbp,), torch.float32)
             b["keys"] = rows("route_keys", (nbp,), torch.int32) if nb > ROUTE_NB_LDS else None
-            size = max(h * tiles(*w) * (s if (s := route_segments(h * nt, h * tiles(*w), nb, kx, leaf)) > 1 else 0) for w in mine)
+            units = [h * tiles(*w) for w in mine]
+            size = max((u * s for u in units if (s := route_segments(h * nt, u, nb, kx, leaf, _cus(dev))) > 1), default=0)
             b["parts"] = None
             if size:
                 live.append(_buf(ws, "parts", (size * tile * (D + 1),), torch.float32, dev))

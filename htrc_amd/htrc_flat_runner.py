@@ -64,16 +64,16 @@ F32_UNSPLIT_TILES = 2048
 
 
 # Fused int8 route: the segments whose partial sums a launch of ``units`` of a layer's ``tiles`` (head, tile) pairs
-# keeps in workspace (htrc_route_segments of the C ABI): tiles of more than 128 blocks of 32 keys, in layers of 513 to
-# 1024 pairs and launches of at most 384, and heads of at most 16384 leaves.
-SEG_MIN_BLOCKS, SEG_MAX, SEG_SPLIT_TILES, SEG_MAX_NB, SEG_TILES_MIN, SEG_TILES_MAX = 128, 4, 384, 16384, 512, 1024
+# keeps in workspace (htrc_route_segments of the C ABI): tiles of more than 128 blocks of 32 keys, in layers of more than
+# two and up to four pairs a CU and launches of at most one and a half, and heads of at most 16384 leaves.
+SEG_MIN_BLOCKS, SEG_MAX, SEG_MAX_NB = 128, 4, 16384
+CUS = 256                              # compute units of an MI355X: the memory model's device
 
 
-def route_segments(tiles: int, units: int, nb: int, kx: int, leaf: int) -> int:
+def route_segments(tiles: int, units: int, nb: int, kx: int, leaf: int, cus: int = CUS) -> int:
     blocks = _ceil(nb, 32) + _ceil(kx * leaf, 32)
-    if not SEG_TILES_MIN < tiles <= SEG_TILES_MAX or units > SEG_SPLIT_TILES or blocks <= SEG_MIN_BLOCKS or nb > SEG_MAX_NB:
-        return 1
-    return min(SEG_MAX, _ceil(blocks, 32))
+    segmented = 2 * cus < tiles <= 4 * cus and 2 * units <= 3 * cus and blocks > SEG_MIN_BLOCKS and nb <= SEG_MAX_NB
+    return SEG_MAX if segmented else 1
 
 
 def workspace_bytes(queries: int, keys: int, leaf: int = 16, dim: int = 128, heads: int = 1, splits: int = 1,

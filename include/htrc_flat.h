@@ -166,12 +166,12 @@ int htrc_route(const int8_t* q8, const float* sq, const int8_t* dq8, const float
                int stride, int tile, int group, int64_t g0, int64_t gn, const int32_t* perm, float scale, float* out,
                float* logz, int32_t* idx, float* rowmax, uint32_t* keys_ws, void* stream);
 
-/* htrc_route for tiles of many keys: a tile of more than 128 32-key blocks (far leaves and near
- * tokens) in a layer of 513 to 1024 (head, tile) pairs is summed in segments whose order its block count
- * fixes, so every window and launch of a layer gives the same bits.  parts (fp32, 16-byte aligned,
- * heads * tiles of the window * segments * T * 129 floats; NULL when htrc_route_segments() is 1)
- * takes the segments' sums where the window is small enough that they run as workgroups of their
- * own; without it, and in larger windows, one workgroup runs a tile's segments in turn.
+/* htrc_route for tiles of many keys: in a layer of more than two and up to four (head, tile) pairs a CU (513 to 1024 on
+ * 256 CUs), a tile of more than 128 32-key blocks (far leaves and near tokens) is summed in four segments, whose
+ * order the layer's shape fixes, so every window and launch of a layer gives the same bits.  parts (fp32,
+ * 16-byte aligned, heads * tiles of the window * segments * T * 129 floats; NULL when htrc_route_segments() is 1)
+ * takes the segments' sums where the window is small enough that they run as workgroups of their own
+ * (one and a half tiles a CU); without it, and in larger windows, one workgroup runs a tile's segments in turn.
  * htrc_route_segments: the segments per tile that the window's launch keeps in parts, 1 when it needs
  * none, 0 with an error set when the arguments are invalid. */
 int htrc_route_segments(int64_t heads, int64_t nq, int64_t nk, int leaf, int kx, int tile, int group, int64_t g0,

@@ -49,6 +49,7 @@ def events(monkeypatch):
     monkeypatch.setattr(hip, "_need", lambda *a: None)
     monkeypatch.setattr(hip, "call", launch)
     monkeypatch.setattr(hip, "stream_handle", lambda *a: 0)
+    monkeypatch.setattr(hip, "_cus", lambda dev: 256)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: cur)
     monkeypatch.setattr(torch.cuda, "device", lambda *a: contextlib.nullcontext())
     monkeypatch.setattr(htrc_flat, "_window_streams", lambda dev, n: side[:n])
