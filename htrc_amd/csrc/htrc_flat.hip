@@ -38,10 +38,10 @@ __device__ __forceinline__ u32x2 pack8_i8(const int (&c)[8]) {
     return u32x2{pack4_i8(c[0], c[1], c[2], c[3]), pack4_i8(c[4], c[5], c[6], c[7])};
 }
 
-// pad_dims: rows of d < 128 values (fp32 or bf16) to rows of 128 (fp32 or bf16, rounded to nearest even) with zeros past
-// d, for up to three tensors (blockIdx.y) in one launch: four output dims per thread.  What counts is the launches: a clear
-// and a converting copy per tensor were six, 22 us of kernels and 20 us of host time in a call of 1024 queries and 4096 keys of 64
-// dims (103 us; 82 with this one launch of 4.5 us).
+// pad_dims: rows of d < 128 values (fp32 or bf16) to rows of 128 (fp32 or bf16, rounded to nearest even)
+// with zeros past d, for up to three tensors (blockIdx.y) in one launch: four output dims per thread.  What
+// counts is the launches: a clear and a converting copy per tensor were six, 22 us of kernels and 20 us of
+// host time in a call of 1024 queries and 4096 keys of 64 dims (103 us; 82 with this one launch of 4.5 us).
 struct PadTensor {
     const void* src;
     void* dst;
@@ -2444,10 +2444,11 @@ __global__ __launch_bounds__(256) void select_f32_kernel(const void* __restrict_
     }
 }
 
-// merge: (h3/htrc_flat_triton.py:257-273) + logZ = mm + log(den).  32 threads per row, four dims each, 8 rows per
-// workgroup: every load and store is a row's contiguous 512 bytes, and a tile's rows spread over 8 workgroups
-// (with four threads per row and one workgroup per tile, 32 tiles of 8 splits took 14.4 us for 9.4 MB; 8.3 now).
-// Tiles [t0, t0 + tn) of each head (gridDim.x = tn * tile / 8); the partials are the launch's own [H, tn, ns, tile].
+// merge: (h3/htrc_flat_triton.py:257-273) + logZ = mm + log(den).  32 threads per row, four dims each, 8
+// rows per workgroup: every load and store is a row's contiguous 512 bytes, and a tile's rows spread over 8
+// workgroups (with four threads per row and one workgroup per tile, 32 tiles of 8 splits took 14.4 us for
+// 9.4 MB; 8.3 now). Tiles [t0, t0 + tn) of each head (gridDim.x = tn * tile / 8); the partials are the
+// launch's own [H, tn, ns, tile].
 __global__ __launch_bounds__(256) void merge_kernel(const float* __restrict__ pm, const float* __restrict__ pl,
                                                     const float* __restrict__ pacc, int ns, int64_t nq, int t0,
                                                     int tile, const int32_t* __restrict__ perm,
@@ -2545,15 +2546,16 @@ constexpr size_t ROUTE_LDS_MAX = 160 * 1024;         // LDS of one workgroup on 
 // Passes of a tile in the route kernels: one at the select launch's reference, and when a row
 // total leaves range one more at every row's exact largest score (in range by construction).
 constexpr int MAX_PASSES = 2;
-// The fixed softmax reference of a row is its largest far-field score.  A leaf's far-field score is a lower bound of
-// the leaf's exact log-mass (the log-sum-exp is convex in the row), so a near leaf's exact score can lie far
-// above the reference and hardly below: over heads of 40759 tokens whose scores spread by 11 nats a row's total is -0.2
-// to 116 octaves above it, and with totals up to 2^64 a quarter of those tiles were computed twice.  Totals in
-// [REF_MIN, REF_MAX] are taken as they are: all that a float holds but for the room that keeps 1 / total a normal
-// number.  A row of outputs that overflows at such a total, or could once its key parts or segments are
-// added, also sends its tile to the redo.  (A reference 36 octaves higher takes totals up to 2^136: six of those heads
-// a call 3672 us against 3692 here, 0.5 % between runs.  But it puts an ordinary row's outputs at 2^-36 of its
-// values, and values below 2^-66 then lose bits.)
+// The fixed softmax reference of a row is its largest far-field score.  A leaf's far-field score is a lower
+// bound of the leaf's exact log-mass (the log-sum-exp is convex in the row), so a near leaf's exact score
+// can lie far above the reference and hardly below: over heads of 40759 tokens whose scores spread by 11
+// nats a row's total is -0.2 to 116 octaves above it, and with totals up to 2^64 a quarter of those tiles
+// were computed twice.  Totals in [REF_MIN, REF_MAX] are taken as they are: all that a float holds but for
+// the room that keeps 1 / total a normal number.  A row of outputs that overflows at such a total, or could
+// once its key parts or segments are added, also sends its tile to the redo.  (A reference 36 octaves
+// higher takes totals up to 2^136: six of those heads a call 3672 us against 3692 here, 0.5 % between
+// runs.  But it puts an ordinary row's outputs at 2^-36 of its values, and values below 2^-66 then lose
+// bits.)
 constexpr float REF_MIN = 0x1p-60f, REF_MAX = 0x1p125f;
 __device__ __forceinline__ float row_reference(float m) { return m == -INFINITY ? 0.0f : __fmul_rn(m, LOG2E); }
 // Merge: the wave pairs' partial O, 64 rows x 128 dims each, rows padded to 132 floats.
@@ -2632,9 +2634,10 @@ __device__ __forceinline__ void dma_rows47(const uint16_t* x1, const BlockOffset
 // LDS, for rows of more leaves than the LDS holds.  The launch covers tile groups
 // [g0, g0 + ng) of each head; the state rows and idx are the launch's own ([H, ng, ...]).
 constexpr int SEL_RING = 3;                         // route_select ring slots per wave
-// NW waves per workgroup: the leaf groups are dealt over them, so a launch of few tile groups takes 8 or 16 (the
-// device has four SIMDs a CU whatever the groups are): 128 groups of 2547 leaves (kx 256) 42 -> 28.6 us.  With fewer
-// leaves than eight 16-leaf groups a wave the extra waves cost more in barriers (256 leaves: 11.3 us at 4 waves, 13.1 at 16).
+// NW waves per workgroup: the leaf groups are dealt over them, so a launch of few tile groups takes 8 or 16
+// (the device has four SIMDs a CU whatever the groups are): 128 groups of 2547 leaves (kx 256) 42 -> 28.6
+// us.  With fewer leaves than eight 16-leaf groups a wave the extra waves cost more in barriers (256
+// leaves: 11.3 us at 4 waves, 13.1 at 16).
 constexpr int ROUTE_NB_LDS = 16384;                 // leaves per head whose keys route_select keeps in LDS
 template <bool MULTI, int NRB, bool GK, int NW>
 __global__ __launch_bounds__(64 * NW, 4) void route_select_kernel(
@@ -2849,23 +2852,26 @@ __device__ __forceinline__ RowMax<RB> route_exact_max(const int8_t* dq8, const f
     return mx;
 }
 
-// Long tiles: in layers of a middling number of tiles, a tile whose far and near fields are more than SEG_MIN_BLOCKS
-// 32-key blocks has its block stream (far, then near) cut into SEG_MAX equal segments, each summed from zero, and
-// the segments' sums added in order.  The rule looks at the layer's shape alone (its tiles, leaves and near leaves),
-// so every windowing of a layer sums in the same order: the segments may run as workgroups of their own
-// (route_part_kernel, partial sums in workspace, combined by route_seg_kernel) or one after the other in
-// one workgroup (route_seg_kernel), bit for bit alike.  The launch takes the first where its own tiles leave
-// the CUs short of waves: a 128-tile window of whole tiles is one wave pair a tile, 256 waves for 1024 SIMDs.
-// The lines, in tiles per CU (256 CUs; us a call without and with segments, leaf 16, 256 near leaves unless said):
-//   SEG_TILES_MIN, SEG_TILES_MAX: 516 tiles in windows of 128 702 -> 447, 637 819 -> 555, 1024 1571 -> 1141; in one window
-//   385 -> 387, 478 -> 481, 987 -> 975.  Windows gain outside too (469 tiles 400 -> 345, 1094 1958 -> 1389, 1274
-//   1316 -> 1033), but the rule may not look at the window, and one-window calls lose there: 469 tiles 287 -> 339 (their
-//   whole-tile kernels split each tile's keys over several wave parts), 1094 1228 -> 1330, 1274 848 -> 935, 2548
-//   1566 -> 1637 (more tiles a CU than the in-turn kernel's registers allow).
-//   segments_apart: of 1024 tiles, windows of 300 in turn 1184, apart 1128; of 400 1075 and 1105; of 640 1015 and 1059.
-//   SEG_MIN_BLOCKS: 637 tiles of 208 blocks gain as above, of 592 (1024 near leaves) in windows of 256 1427 -> 753.
-//   Fewer blocks would gain in windows of 128 too (112 blocks 606 -> 485, 84 398 -> 317, 52 326 -> 289, 42 271 -> 269),
-//   not in one window (84 blocks 210 -> 212; 768 tiles of 34 blocks 94 -> 98).
+// Long tiles: in layers of a middling number of tiles, a tile whose far and near fields are more than
+// SEG_MIN_BLOCKS 32-key blocks has its block stream (far, then near) cut into SEG_MAX equal segments, each
+// summed from zero, and the segments' sums added in order.  The rule looks at the layer's shape alone (its
+// tiles, leaves and near leaves), so every windowing of a layer sums in the same order: the segments may
+// run as workgroups of their own (route_part_kernel, partial sums in workspace, combined by
+// route_seg_kernel) or one after the other in one workgroup (route_seg_kernel), bit for bit alike.  The
+// launch takes the first where its own tiles leave the CUs short of waves: a 128-tile window of whole tiles
+// is one wave pair a tile, 256 waves for 1024 SIMDs. The lines, in tiles per CU (256 CUs; us a call without
+// and with segments, leaf 16, 256 near leaves unless said):
+//   SEG_TILES_MIN, SEG_TILES_MAX: 516 tiles in windows of 128 702 -> 447, 637 819 -> 555, 1024 1571 ->
+//   1141; in one window 385 -> 387, 478 -> 481, 987 -> 975.  Windows gain outside too (469 tiles 400 ->
+//   345, 1094 1958 -> 1389, 1274 1316 -> 1033), but the rule may not look at the window, and one-window
+//   calls lose there: 469 tiles 287 -> 339 (their whole-tile kernels split each tile's keys over several
+//   wave parts), 1094 1228 -> 1330, 1274 848 -> 935, 2548 1566 -> 1637 (more tiles a CU than the in-turn
+//   kernel's registers allow).
+//   segments_apart: of 1024 tiles, windows of 300 in turn 1184, apart 1128; of 400 1075 and 1105; of 640
+//   1015 and 1059.
+//   SEG_MIN_BLOCKS: 637 tiles of 208 blocks gain as above, of 592 (1024 near leaves) in windows of 256
+//   1427 -> 753.  Fewer blocks would gain in windows of 128 too (112 blocks 606 -> 485, 84 398 -> 317, 52
+//   326 -> 289, 42 271 -> 269), not in one window (84 blocks 210 -> 212; 768 tiles of 34 blocks 94 -> 98).
 //   SEG_MAX: 4 segments against 6, 8 and 16 of 208 blocks: 706 / 715 / 720 / 720 us.
 constexpr int SEG_MIN_BLOCKS = 128;
 constexpr int SEG_MAX = 4;
@@ -2883,11 +2889,12 @@ inline int route_segments(int64_t tiles, int64_t nb, int kxe, int leaf, int64_t 
 // Whether a launch of `units` tiles runs them apart: up to one and a half tiles a CU.
 inline bool segments_apart(int64_t units, int64_t cus) { return 2 * units <= 3 * cus; }
 
-// RB 16-row blocks per wave, NH waves per key part (NH = 2: halves of the tile's rows; NH = 4, RB = 1: quarters of
-// a 64-row tile, the same sums per row); NP key parts of NH waves; RS ring slots per part.  MODE ROUTE_WHOLE: the tile's keys in one sum.  ROUTE_PART: workgroup
-// (tile, segment), the segment's O and row sums to part_o / part_l [tile of the launch][segment].
-// ROUTE_SEGS: with part_o, SEG_QUARTERS workgroups per tile add the tile's partial sums (the redo of a
-// tile whose reference missed is the first one's); without, one workgroup runs the segments in turn.
+// RB 16-row blocks per wave, NH waves per key part (NH = 2: halves of the tile's rows; NH = 4, RB = 1:
+// quarters of a 64-row tile, the same sums per row); NP key parts of NH waves; RS ring slots per part.
+// MODE ROUTE_WHOLE: the tile's keys in one sum.  ROUTE_PART: workgroup (tile, segment), the segment's O and
+// row sums to part_o / part_l [tile of the launch][segment]. ROUTE_SEGS: with part_o, SEG_QUARTERS
+// workgroups per tile add the tile's partial sums (the redo of a tile whose reference missed is the first
+// one's); without, one workgroup runs the segments in turn.
 template <int LEAF, int RB, int NP, int RS, int MODE, int NH>
 __device__ __forceinline__ void route_body(
     const int8_t* __restrict__ q8, const float* __restrict__ sq, const int8_t* __restrict__ dq8,
@@ -3270,7 +3277,8 @@ __device__ __forceinline__ void route_body(
         if constexpr (MODE == ROUTE_SEGS) {
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
-                sum.l[rb] = __fadd_rn(sum.l[rb], grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero<SEG_MAX>(st.o[rb])) : st.l[rb]));
+                const float lt = pass == 0 ? __fadd_rn(st.l[rb], finite_zero<SEG_MAX>(st.o[rb])) : st.l[rb];
+                sum.l[rb] = __fadd_rn(sum.l[rb], grp_sum(lt));
 #pragma unroll
                 for (int db = 0; db < 8; ++db)
 #pragma unroll
@@ -3313,7 +3321,6 @@ __device__ __forceinline__ void route_body(
         if (bad) redo = 1;
         __syncthreads();
         if (__builtin_expect(redo == 0 || pass + 1 == MAX_PASSES, 1)) break;
-        
         if constexpr (MODE == ROUTE_SEGS) lo = 0, hi = nb, e_lo = 0, e_hi = e_n;
         const RowMax<RB> mx = route_exact_max<LEAF, RB>(dq8, sdq, q8, sq, scale, g8, sg, lz, exbits, srow0, lo, hi, k8,
                                                         ks, sidx, kh, e_lo, e_hi, th * TR + 16 * RB * hr);
@@ -3413,11 +3420,12 @@ template <int LEAF, int RB, int NP, int RS>
 __global__ __launch_bounds__(128 * NP, route_waves_per_simd<NP>()) void route_kernel(ROUTE_PARAMS) {
     route_body<LEAF, RB, NP, RS, ROUTE_WHOLE, 2>(ROUTE_ARGS, nullptr, nullptr, 1);
 }
-// 64-row tiles with four waves of 16 rows per key part, where there are several: the same sums per row, twice the waves to
-// hide each block's loads in.  Against two waves of 32 rows, us a call: two key parts, two heads of 11008 tokens 97.8 ->
-// 95.5, one of 24000 94.9 -> 93.4; four, 8192 queries on 32768 keys 93.7 -> 91.5, 16384 tokens in leaf-16
-// windows of 64 tiles 241 -> 233, in one leaf-64 window 68.4 -> 68.3, 4096 tokens 64.6 -> 66.5 (3 % between runs).  One
-// key part keeps two waves of 32 rows: there several tiles share a CU, and each LDS read feeds twice the products.
+// 64-row tiles with four waves of 16 rows per key part, where there are several: the same sums per row,
+// twice the waves to hide each block's loads in.  Against two waves of 32 rows, us a call: two key parts,
+// two heads of 11008 tokens 97.8 -> 95.5, one of 24000 94.9 -> 93.4; four, 8192 queries on 32768 keys 93.7
+// -> 91.5, 16384 tokens in leaf-16 windows of 64 tiles 241 -> 233, in one leaf-64 window 68.4 -> 68.3, 4096
+// tokens 64.6 -> 66.5 (3 % between runs).  One key part keeps two waves of 32 rows: there several tiles
+// share a CU, and each LDS read feeds twice the products.
 template <int LEAF, int NP>
 __global__ __launch_bounds__(256 * NP, NP == 4 ? 4 : 2) void route_rows_kernel(ROUTE_PARAMS) {
     route_body<LEAF, 1, NP, ROUTE_RS, ROUTE_WHOLE, 4>(ROUTE_ARGS, nullptr, nullptr, 1);
@@ -4137,10 +4145,11 @@ __global__ __launch_bounds__(256) void tail_kernel(const void* __restrict__ q, c
     if (qd == 0) logz[row] = nz;
 }
 
-// The same for at most TAIL_SMALL keys: the keys' operands staged once per workgroup in LDS (the kernel above
-// reads them from global memory for every row and pass, each key's latency in turn) and each row's scores
-// kept in registers between the passes; the same sums in the same order.  What is left is the
-// rows' own traffic (q read, out read and written): 40759 rows x 7 keys 69 -> 20 us, with 63 MB to move; six heads 370 -> 101.
+// The same for at most TAIL_SMALL keys: the keys' operands staged once per workgroup in LDS (the kernel
+// above reads them from global memory for every row and pass, each key's latency in turn) and each row's
+// scores kept in registers between the passes; the same sums in the same order.  What is left is the rows'
+// own traffic (q read, out read and written): 40759 rows x 7 keys 69 -> 20 us, with 63 MB to move; six
+// heads 370 -> 101.
 constexpr int TAIL_SMALL = 16;
 template <bool IN_BF16, int MODE>
 __global__ __launch_bounds__(256) void tail_small_kernel(const void* __restrict__ q, const float* __restrict__ tk,
@@ -4430,11 +4439,11 @@ __global__ __launch_bounds__(128) void km_update_kernel(const void* __restrict__
     if (cnt > 0) cen[((int64_t)h * C + j) * D + tid] = __fdiv_rn(acc, (float)cnt);
 }
 
-// The same for few centres in flight (heads x clusters <= KM_WIDE): eight waves per centre list its samples,
-// each its own run of the sample, and gather 64 rows at a time into one of two LDS buffers, the next
-// 64 on their way while lane d sums dim d of the current ones in list order.  With a centre on every CU the other
-// kernel's two waves hide each other's gathers (24 heads: 45 us; staged rows were slower there); with one head's 32 centres on 256
-// CUs each gather's latency stood alone: 16.7 -> 9.8 us.
+// The same for few centres in flight (heads x clusters <= KM_WIDE): eight waves per centre list its
+// samples, each its own run of the sample, and gather 64 rows at a time into one of two LDS buffers, the
+// next 64 on their way while lane d sums dim d of the current ones in list order.  With a centre on every
+// CU the other kernel's two waves hide each other's gathers (24 heads: 45 us; staged rows were slower
+// there); with one head's 32 centres on 256 CUs each gather's latency stood alone: 16.7 -> 9.8 us.
 constexpr int KM_WIDE = 256;
 template <bool IN_BF16>
 __global__ __launch_bounds__(512) void km_update_wide_kernel(const void* __restrict__ q, int64_t nq, int m, int C,
@@ -4909,13 +4918,13 @@ static int leaf_stats_launch(const char* who, const float* mu, const uint16_t* m
         return bad("misaligned buffer");
     const int64_t nb = nk / leaf;
     const int nbp = htrc_nb_pad(nb);
-    // leaf-stationary: NL leaves (64 KB of K / V) per workgroup; the centre groups of a head dealt
-    // over ncs workgroups when the leaf groups alone give fewer than two workgroups per CU (each
-    // wave keeps at least one group of 16 centres)
-    // (leaf 16: 32 KB where the leaf groups are fewer than two per CU: three workgroups then share a CU's registers and LDS
-    // with TF32 operands, and twice the workgroups share the few centre groups of a short window.  One head of 40752 keys,
-    // 128 centres 46.2 -> 40.0 us, 637 centres 172.6 -> 156.2; 32 centres of 12336 keys, fp32 store, 31.0 -> 21.5.  Not the
-    // IEEE operands of longer windows (637 centres, fp8: 144 -> 161), nor six heads (231 -> 249).)
+    // leaf-stationary: NL leaves (64 KB of K / V) per workgroup; the centre groups of a head dealt over ncs
+    // workgroups when the leaf groups alone give fewer than two workgroups per CU (each wave keeps at least
+    // one group of 16 centres).  Leaf 16: 32 KB where the leaf groups are fewer than two per CU: three
+    // workgroups then share a CU's registers and LDS with TF32 operands, and twice the workgroups share the
+    // few centre groups of a short window.  One head of 40752 keys, 128 centres 46.2 -> 40.0 us, 637
+    // centres 172.6 -> 156.2; 32 centres of 12336 keys, fp32 store, 31.0 -> 21.5.  Not the IEEE operands of
+    // longer windows (637 centres, fp8: 144 -> 161), nor six heads (231 -> 249).
     const int64_t want = 2 * (int64_t)device_cus();
     const bool half = leaf == 16 && nbp / 8 * heads < want && (TF32 || cn <= 64) && mut;
     const int nl = half ? 4 : 65536 / (512 * leaf);
@@ -5466,10 +5475,10 @@ static int route_attend_launch(const int8_t* q8, const float* sq, const int8_t* 
     hipLaunchKernelGGL((K<L, RB, NH>), dim3((unsigned)(units * (N))), dim3(64 * NH), dyn, s, q8, sq, dq8, sdq, g8, sg, lz, \
                        vb, k8, ks, v, idx, rowmax, nq, (int)nt, group, (int)g0, (int)gn, perm, nk, (int)nb, nbp, kxe,  \
                        scale, out, logz, part_o, part_l, nseg)
-        // A 64-row tile's segments run with its rows over four waves (16 each, four waves a SIMD): the launches
-        // are short of waves, and each hides the others' loads (128-tile windows of the 40759-token head 648 -> 587 us
-        // a call).  In turn, two waves of 32 rows, whose LDS reads feed twice the products: 768 tiles a window 3530
-        // against 3612 us a call with four.
+        // A 64-row tile's segments run with its rows over four waves (16 each, four waves a SIMD): the
+        // launches are short of waves, and each hides the others' loads (128-tile windows of the
+        // 40759-token head 648 -> 587 us a call).  In turn, two waves of 32 rows, whose LDS reads feed
+        // twice the products: 768 tiles a window 3530 against 3612 us a call with four.
 #define SEG_SPLIT(L, RB, NH)                                                                                    \
     SEG_LAUNCH(route_part_kernel, L, RB, NH, nseg);                                                             \
     SEG_LAUNCH(route_seg_kernel, L, RB, NH, SEG_QUARTERS);
@@ -5671,10 +5680,11 @@ int htrc_route16(const uint16_t* q16, const uint16_t* dq16, const void* g, const
                                g0, gn, perm, fp8, scale, out, logz, stream);
 }
 
-// The tile windows of a layer, each the centres' terms, the statistics and the routing of `chunk` tile groups, dealt in
-// turn over the caller's streams: the launches of the entry points above in their order, issued here because a window's
-// five to seven launches cost a Python caller longer than a small window runs (the fp32 path on 12345 queries in seven
-// windows of 32 tiles: 554 us of host time a call launched one by one, 321 here, the call 563 -> 373).
+// The tile windows of a layer, each the centres' terms, the statistics and the routing of `chunk` tile
+// groups, dealt in turn over the caller's streams: the launches of the entry points above in their order,
+// issued here because a window's five to seven launches cost a Python caller longer than a small window
+// runs (the fp32 path on 12345 queries in seven windows of 32 tiles: 554 us of host time a call launched
+// one by one, 321 here, the call 563 -> 373).
 int htrc_windows_i8(const float* mu, const uint16_t* k, const uint16_t* v, const int8_t* q8, const float* sq,
                     const int8_t* dq8, const float* sdq, const int8_t* k8, const float* ks, int64_t heads, int64_t nq,
                     int64_t nk, int leaf, int d, int kx, int sink, int stride, int tile, int group, int64_t chunk,

@@ -616,13 +616,15 @@ def route16_fits(nb: int, kx: int) -> bool:
 def run_windows(packed: dict, q, mu, *, nb: int, leaf: int, kx: int, scale: float, store, f32dots: bool, wins, sink: int,
                 stride: int, tile: int, group: int, perm, prec: str, splits, bn, unsplit: int, rowmax, out, logz, wss,
                 side=(), cur=None):
-    """The tile windows ``wins`` [(g0, gn), ...] of a layer in one native call (htrc_windows_*): window i on the stream
-    side[i % n] (n = 1 without side streams: the current one) with the buffers of the workspace wss[i % n] (the names and
-    sizes of the per-stage functions above).  packed, q, mu as flat_attention builds them; kx > 0 for the fp32 dots, which alone look at bn, and
-    at splits where a window has fewer than ``unsplit`` (head, tile) pairs.
-    The buffers are allocated on the caller's stream ``cur`` and used on the side streams: those wait for it after the last
-    allocation, since a block may come from another thread of the same stream whose kernels still read it, and it for
-    them before the first buffer is dropped, since the next owner's kernels wait for ``cur`` alone."""
+    """The tile windows ``wins`` [(g0, gn), ...] of a layer in one native call (htrc_windows_*): window i on the
+    stream side[i % n] (n = 1 without side streams: the current one) with the buffers of the workspace
+    wss[i % n] (the names and sizes of the per-stage functions above).  packed, q, mu as flat_attention
+    builds them; kx > 0 for the fp32 dots, which alone look at bn, and at splits where a window has fewer
+    than ``unsplit`` (head, tile) pairs.
+    The buffers are allocated on the caller's stream ``cur`` and used on the side streams: those wait for it
+    after the last allocation, since a block may come from another thread of the same stream whose kernels
+    still read it, and it for them before the first buffer is dropped, since the next owner's kernels wait
+    for ``cur`` alone."""
     k, v = packed["k"], packed["v"]
     _need(mu, torch.float32, "mu")
     _need(k, torch.bfloat16, "k")

@@ -625,6 +625,21 @@ def test_kmeans_order_bitexact(device, n, clusters, sample, iters, qdtype):
         assert np.array_equal(_np(perm[h]), want), f"head {h}"
 
 
+@pytest.mark.parametrize("heads,n", [(8, 700), (9, 700),          # 256 centres and 288: either side of the wide update
+                                     (4, 4100), (5, 4100),        # 256 and 320 waves of sample rows: eight and four waves a row
+                                     (16, 4100), (17, 4100)])     # 1024 and 1088: four and one
+@pytest.mark.parametrize("qdtype", ["bf16", "fp32"])
+def test_kmeans_order_of_many_heads(device, heads, n, qdtype):
+    """The launches that a call of many heads takes, 32 centres a head: the permutation is the oracle's, bit for bit."""
+    q, _, _ = _data(n, nk=64, seed=n + heads, heads=heads)
+    if qdtype == "fp32":
+        q = q.float() + 1e-3 * torch.randn(q.shape, generator=torch.Generator().manual_seed(6))
+    perm = hip.kmeans_order(q.to(device).contiguous(), clusters=32, sample=4096, iters=3)
+    torch.cuda.synchronize()
+    for h in range(heads):
+        assert np.array_equal(_np(perm[h]), flat_i8.kmeans_order(q[h].float().numpy(), 32, 4096, 3)), f"head {h}"
+
+
 # ---- fp8 state store (store="fp8", h3/htrc_flat_triton.py:65-72, 104-108, 132-153, 214-254)
 
 @pytest.mark.parametrize("nq,group", [(4096, 1), (1000, 2)])

@@ -7,7 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from htrc_amd import htrc_flat, htrc_flat_hip as hip, workloads
+from htrc_amd import htrc_flat, htrc_flat_hip as hip, htrc_flat_runner, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -28,6 +28,28 @@ def test_native_windows_equal_the_stage_loop(device, kw, chunk, streams, group, 
         got = htrc_flat.flat_attention(q, k, v, ws=space, **kw)
         torch.cuda.synchronize()
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("heads,n,order,group,ws", [(2, 17000, "seq", 1, True), (2, 17000, "kmeans", 1, False),
+                                                     (3, 11000, "seq", 2, True), (3, 11000, "kmeans", 2, False)])
+def test_segmented_layers_of_several_heads(device, heads, n, order, group, ws):
+    """Layers of 532 and 516 (head, tile) pairs of 129 key blocks: one window (the segments in turn), small windows (as workgroups
+    of their own, the last one shorter) and windows of more than 384 pairs before a short one (both forms
+    in one call): the same bits from every one, natively and stage by stage."""
+    q, k, v = (x.to(device) for x in workloads.clustered_runs(n=n, runs=-(-n // 64), heads=heads, seed=heads))
+    k, v = k[:, :4128].contiguous(), v[:, :4128].contiguous()
+    nt = -(-n // 64)
+    assert 512 < heads * nt <= 1024 and htrc_flat_runner.route_segments(heads * nt, heads * 60, 258, 240, 16) == 4
+    kw = dict(backend="hip", store="int8", dot="bf16", leaf=16, exact_leaves=240, order=order, kern={"group": group},
+              return_logz=True)
+    want = [x.clone() for x in htrc_flat.flat_attention(q, k, v, tile_chunk=None, **kw)]
+    space = {} if ws else None
+    for chunk in (400 // heads, 60):
+        staged = htrc_flat.flat_attention(q, k, v, tile_chunk=chunk, state={}, **kw)
+        native = htrc_flat.flat_attention(q, k, v, tile_chunk=chunk, ws=space, **kw)
+        torch.cuda.synchronize()
+        for got in (staged, native):
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), chunk
 
 
 @pytest.mark.parametrize("kw", [dict(store="int8", dot="bf16"), dict(store="fp32", dot="tf32")])

@@ -83,7 +83,8 @@ def test_segmented_route(device, n, m, leaf, kx, tile, group, g0, gn, spike, seg
 def test_route_select_wave_counts(device, groups, nb, kx, sink, group, ties):
     """route_select's launches of 4, 8 and 16 waves per tile group (more than 512, 257 to 512, fewer groups; heads
     whose keys leave no room for 16 rings), and its top-k at and beside each bound of its methods: index sets
-    equal to the stage select and top-k on the same state, row maxima to a 4-wave launch's."""
+    equal to the stage select and top-k on the same state, row maxima to the largest of the row's scores in 64 bits (four
+    roundings of 2^-24 of at most 127^2 * 128 * 1e-4 + 5 here: 5e-5)."""
     torch.manual_seed(nb + kx)
     nbp, nt = -(-nb // 32) * 32, groups * group
     dq8 = torch.randint(-127, 128, (1, nt * 64, 128), device=device, dtype=torch.int8)
@@ -101,6 +102,13 @@ def test_route_select_wave_counts(device, groups, nb, kx, sink, group, ties):
     sel = hip.rowmax_select(g=g8, lz=lz, sg=sg, nb=nb, dq8=dq8, sdq=sdq, group=group)
     want, _ = hip.topk_excl(sel, nb, kx, sink)
     assert torch.equal(idx, want)
+    rows, step = 64 * group, max(1, 1 << 22 >> nbp.bit_length())
+    q64, s64, m64 = dq8.view(groups, rows, 128).double(), sdq.view(groups, rows, 1).double(), rowmax.view(groups, rows)
+    for g in range(0, groups, max(1, step // rows)):
+        e = min(groups, g + max(1, step // rows))
+        dots = torch.bmm(q64[g:e], g8[0, g:e, :nb].double().transpose(1, 2).contiguous())
+        best = (dots * s64[g:e] * sg[0, g:e, None, :nb].double() + lz[0, g:e, None, :nb].double()).amax(2)
+        assert float((best - m64[g:e]).abs().max()) <= 5e-5
     # the same groups inside a window: the launch's first groups alone
     few = min(groups, 2)
     part = {k: x[:, :few].contiguous() for k, x in state.items()}
