@@ -17,6 +17,7 @@ shapes.  ``prec`` is always IEEE fp32 accumulate (there is no TF32 on CDNA4).
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 
 import torch
@@ -621,10 +622,12 @@ def run_windows(packed: dict, q, mu, *, nb: int, leaf: int, kx: int, scale: floa
     wss[i % n] (the names and sizes of the per-stage functions above).  packed, q, mu as flat_attention
     builds them; kx > 0 for the fp32 dots, which alone look at bn, and at splits where a window has fewer
     than ``unsplit`` (head, tile) pairs.
-    The buffers are allocated on the caller's stream ``cur`` and used on the side streams: those wait for it
-    after the last allocation, since a block may come from another thread of the same stream whose kernels
-    still read it, and it for them before the first buffer is dropped, since the next owner's kernels wait
-    for ``cur`` alone."""
+    The buffers of a new workspace are allocated on their side stream, whose freed blocks the next workspace
+    takes up again (a runner warms up on a stream of its own: 3.5 ms of its 24 to 30 went to fresh device
+    memory when they came from there).  Others come from the caller's stream ``cur``.  Either way the side
+    streams wait for ``cur`` after the last allocation, since a block may be one that another thread of that
+    stream freed while its kernels still read it, and ``cur`` for them before the first buffer is dropped,
+    since the next owner's kernels wait for ``cur`` alone."""
     k, v = packed["k"], packed["v"]
     _need(mu, torch.float32, "mu")
     _need(k, torch.bfloat16, "k")
@@ -648,38 +651,39 @@ def run_windows(packed: dict, q, mu, *, nb: int, leaf: int, kx: int, scale: floa
     n = max(1, len(side))
     for i in range(n):
         ws, mine = wss[i], wins[i::n]
-        gn = mine[0][1]                                 # the largest window of the stream (only the layer's last is smaller)
+        with torch.cuda.stream(side[i]) if side and ws == {} else contextlib.nullcontext():
+            gn = mine[0][1]                                 # the largest window of the stream (only the layer's last is smaller)
 
-        def rows(name, tail, dtype, r=gn):
-            t = _buf(ws, name, (h * r, *tail), dtype, dev)
-            live.append(t)
-            return t.data_ptr()
+            def rows(name, tail, dtype, r=gn):
+                t = _buf(ws, name, (h * r, *tail), dtype, dev)
+                live.append(t)
+                return t.data_ptr()
 
-        b = {"terms": rows("mu_terms", (MUT_ROW,), torch.int16), "g": rows(gname, (nbp, d), store),
-             "vb": rows(vname, (nbp, d), vdt), "lz": rows("lz", (nbp,), torch.float32),
-             "idx": rows("idx", (kx,), torch.int32) if kx > 0 else None}
-        if f32dots:
-            b["sel"], b["excl"] = rows("sel", (nbp,), torch.float32), rows("excl", (nbp,), torch.int8)
-            part = next((tiles(*w) for w in mine if splits > 1 and h * tiles(*w) < unsplit), 0)
-            for name, tail in (("pm", (splits, tile)), ("pl", (splits, tile)), ("pacc", (splits, tile, d))):
-                b[name] = rows(name, tail, torch.float32, part) if part else None
-            names = ("terms", "g", "vb", "lz", "sel", "idx", "excl", "pm", "pl", "pacc")
-        elif store == torch.int8:
-            b["sg"] = rows("sg", (nbp,), torch.float32)
-            b["keys"] = rows("route_keys", (nbp,), torch.int32) if nb > ROUTE_NB_LDS else None
-            units = [h * tiles(*w) for w in mine]
-            size = max((u * s for u in units if (s := route_segments(h * nt, u, nb, kx, leaf, _cus(dev))) > 1), default=0)
-            b["parts"] = None
-            if size:
-                live.append(_buf(ws, "parts", (size * tile * (D + 1),), torch.float32, dev))
-                b["parts"] = live[-1].data_ptr()
-            names = ("terms", "g", "sg", "vb", "lz", "idx", "keys", "parts")
-        else:
-            fp8 = store == torch.float8_e4m3fn
-            b["sg"] = rows("sg", (nbp,), torch.float32) if fp8 else None
-            b["sv"] = rows("sv", (nbp,), torch.float32) if fp8 else None
-            names = ("terms", "g", "sg", "vb", "sv", "lz", "idx")
-        bufs += [b[x] for x in names]
+            b = {"terms": rows("mu_terms", (MUT_ROW,), torch.int16), "g": rows(gname, (nbp, d), store),
+                 "vb": rows(vname, (nbp, d), vdt), "lz": rows("lz", (nbp,), torch.float32),
+                 "idx": rows("idx", (kx,), torch.int32) if kx > 0 else None}
+            if f32dots:
+                b["sel"], b["excl"] = rows("sel", (nbp,), torch.float32), rows("excl", (nbp,), torch.int8)
+                part = next((tiles(*w) for w in mine if splits > 1 and h * tiles(*w) < unsplit), 0)
+                for name, tail in (("pm", (splits, tile)), ("pl", (splits, tile)), ("pacc", (splits, tile, d))):
+                    b[name] = rows(name, tail, torch.float32, part) if part else None
+                names = ("terms", "g", "vb", "lz", "sel", "idx", "excl", "pm", "pl", "pacc")
+            elif store == torch.int8:
+                b["sg"] = rows("sg", (nbp,), torch.float32)
+                b["keys"] = rows("route_keys", (nbp,), torch.int32) if nb > ROUTE_NB_LDS else None
+                units = [h * tiles(*w) for w in mine]
+                size = max((u * s for u in units if (s := route_segments(h * nt, u, nb, kx, leaf, _cus(dev))) > 1), default=0)
+                b["parts"] = None
+                if size:
+                    live.append(_buf(ws, "parts", (size * tile * (D + 1),), torch.float32, dev))
+                    b["parts"] = live[-1].data_ptr()
+                names = ("terms", "g", "sg", "vb", "lz", "idx", "keys", "parts")
+            else:
+                fp8 = store == torch.float8_e4m3fn
+                b["sg"] = rows("sg", (nbp,), torch.float32) if fp8 else None
+                b["sv"] = rows("sv", (nbp,), torch.float32) if fp8 else None
+                names = ("terms", "g", "sg", "vb", "sv", "lz", "idx")
+            bufs += [b[x] for x in names]
     bufs = (ctypes.c_void_p * len(bufs))(*bufs)
     handles = (ctypes.c_void_p * n)(*([s.cuda_stream for s in side] or [stream_handle(dev)]))
     shape = (h, nq, nk, leaf, d, kx, sink, stride, tile, group, wins[0][1])

@@ -1,9 +1,9 @@
 """The order in which a call of several tile windows allocates, waits, launches and drops its buffers, on the host: streams and
-launches are stand-ins that write down what happens, tensors live in host memory.  The window buffers belong to
-the caller's stream, which other threads may share, and are used on the side streams.  So a side stream has to wait
-for the caller's stream after the last of its buffers is allocated (the block may be one that another thread
-freed while its kernels still run), and the caller's stream for the side streams before the first is dropped (the
-next owner's kernels wait for the caller's stream alone).
+launches are stand-ins that write down what happens, tensors live in host memory.  The window buffers are used on the
+side streams and may belong to the caller's stream, which other threads may share.  So a side stream has to wait for
+the caller's stream after the last of its buffers is allocated (the block may be one that another thread freed while
+its kernels still run), and the caller's stream for the side streams before the first is dropped (the next owner's
+kernels wait for the caller's stream alone).
 """
 from __future__ import annotations
 
@@ -33,10 +33,19 @@ def events(monkeypatch):
     cur, side = _Stream("cur", log), tuple(_Stream(f"side{i}", log) for i in range(3))
     buf = hip._buf
 
+    owner = ["cur"]
+
+    @contextlib.contextmanager
+    def on(stream):
+        before, owner[0] = owner[0], stream.name
+        yield
+        owner[0] = before
+
     def traced(ws, name, shape, dtype, device):
+        held = ws is not None and name in ws
         t = buf(ws, name, shape, dtype, device)
-        if name in WINDOW:
-            log.append(("alloc", name))
+        if name in WINDOW and not held:
+            log.append(("alloc", name, owner[0]))
             weakref.finalize(t, log.append, ("drop", name))
         return t
 
@@ -51,6 +60,7 @@ def events(monkeypatch):
     monkeypatch.setattr(hip, "stream_handle", lambda *a: 0)
     monkeypatch.setattr(hip, "_cus", lambda dev: 256)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: cur)
+    monkeypatch.setattr(torch.cuda, "stream", on)
     monkeypatch.setattr(torch.cuda, "device", lambda *a: contextlib.nullcontext())
     monkeypatch.setattr(htrc_flat, "_window_streams", lambda dev, n: side[:n])
     return log
@@ -78,6 +88,13 @@ def test_side_streams_are_ordered_around_the_buffers(events, kw, streams, ws, re
         assert joins and at < max(joins)
         assert all(i > max(joins) for i in drops), "a buffer is dropped before the streams are joined"
     assert ws or refused or len(drops) == len(allocs)
+    # a new workspace's blocks are the side streams', so that the next one, of whatever stream, takes them up again
+    assert {e[2] for e in events if e[0] == "alloc"} == ({f"side{s}" for s in range(streams)} if ws else {"cur"})
+    if ws:                                # a kept one allocates nothing
+        del events[:]
+        htrc_flat.flat_attention(q, k, v, backend="hip", leaf=32, exact_leaves=4, tile_chunk=2, ws=space,
+                                 kern={"window_streams": streams}, **kw)
+        assert not [e for e in events if e[0] == "alloc"]
 
 
 @pytest.mark.parametrize("store,chunk", [("int8", 2), ("int8", None), ("fp8", 2), ("bf16", None)])
