@@ -623,7 +623,7 @@ def run_windows(packed: dict, q, mu, *, nb: int, leaf: int, kx: int, scale: floa
     builds them; kx > 0 for the fp32 dots, which alone look at bn, and at splits where a window has fewer
     than ``unsplit`` (head, tile) pairs.
     The buffers of a new workspace are allocated on their side stream, whose freed blocks the next workspace
-    takes up again (a runner warms up on a stream of its own: 3.5 ms of its 24 to 30 went to fresh device
+    takes up again (a runner warms up on a stream of its own: 2 to 3 ms of its 22 to 28 went to fresh device
     memory when they came from there).  Others come from the caller's stream ``cur``.  Either way the side
     streams wait for ``cur`` after the last allocation, since a block may be one that another thread of that
     stream freed while its kernels still read it, and ``cur`` for them before the first buffer is dropped,
