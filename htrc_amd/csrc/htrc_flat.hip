@@ -2500,16 +2500,19 @@ struct RowsN {         // softmax state of the 16 RB rows of one wave
     f32x4 o[RB][8];    // O^T per row block: dims 16db + 4grp + i of row 16rb + lane%16
 };
 
-// 0 when every partial output of the wave's row block is at most 1 / PARTS of the largest float, so that the sum
-// of PARTS such blocks is finite too, else NaN.
+// 0 when every partial output of the wave's row block is at most 1 / PARTS of the largest float, so that
+// the sum of PARTS such blocks is finite too, else NaN.  (The maximum that keeps NaN: v_maximum3_f32, two
+// values an instruction.)
 template <int PARTS>
 __device__ __forceinline__ float finite_zero(const f32x4 (&o)[8]) {
     float z = 0.0f;
 #pragma unroll
     for (int db = 0; db < 8; ++db)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) z = __fmaf_rn(__fmul_rn(o[db][i], (float)PARTS), 0.0f, z);
-    return z;
+        for (int i = 0; i < 4; i += 2)
+            z = __builtin_elementwise_maximum(__builtin_elementwise_maximum(z, __builtin_fabsf(o[db][i])),
+                                              __builtin_fabsf(o[db][i + 1]));
+    return __fmul_rn(__fmul_rn(z, (float)PARTS), 0.0f);
 }
 
 // p = 2^(u - m) for the log2-domain scores u[rb][0..7] of the RB row blocks (keys

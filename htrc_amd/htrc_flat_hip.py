@@ -17,7 +17,6 @@ shapes.  ``prec`` is always IEEE fp32 accumulate (there is no TF32 on CDNA4).
 """
 from __future__ import annotations
 
-import contextlib
 import ctypes
 
 import torch
@@ -444,9 +443,9 @@ _CUS: dict = {}
 
 def _cus(device) -> int:
     """Compute units of the device (the launch rules count tiles per CU)."""
-    n = _CUS.get(device)
+    n = _CUS.get(device.index)
     if n is None:
-        n = _CUS[device] = torch.cuda.get_device_properties(device).multi_processor_count
+        n = _CUS[device.index] = torch.cuda.get_device_properties(device).multi_processor_count
     return n
 
 
@@ -647,45 +646,60 @@ def run_windows(packed: dict, q, mu, *, nb: int, leaf: int, kx: int, scale: floa
 
     if f32dots:
         bn, splits = int(bn), max(1, int(splits)) if any(h * tiles(*w) < unsplit for w in wins) else 1
+    fp8 = store == torch.float8_e4m3fn
     live, bufs = [], []                                 # live: the buffers, held until the streams are joined
-    n = max(1, len(side))
-    for i in range(n):
-        ws, mine = wss[i], wins[i::n]
-        with torch.cuda.stream(side[i]) if side and ws == {} else contextlib.nullcontext():
-            gn = mine[0][1]                                 # the largest window of the stream (only the layer's last is smaller)
 
-            def rows(name, tail, dtype, r=gn):
-                t = _buf(ws, name, (h * r, *tail), dtype, dev)
-                live.append(t)
-                return t.data_ptr()
+    def buffers(ws, mine):
+        """A stream's buffers, of its largest window (its first: only the layer's last is smaller)."""
+        gn = mine[0][1]
 
-            b = {"terms": rows("mu_terms", (MUT_ROW,), torch.int16), "g": rows(gname, (nbp, d), store),
-                 "vb": rows(vname, (nbp, d), vdt), "lz": rows("lz", (nbp,), torch.float32),
-                 "idx": rows("idx", (kx,), torch.int32) if kx > 0 else None}
-            if f32dots:
-                b["sel"], b["excl"] = rows("sel", (nbp,), torch.float32), rows("excl", (nbp,), torch.int8)
-                part = next((tiles(*w) for w in mine if splits > 1 and h * tiles(*w) < unsplit), 0)
-                for name, tail in (("pm", (splits, tile)), ("pl", (splits, tile)), ("pacc", (splits, tile, d))):
-                    b[name] = rows(name, tail, torch.float32, part) if part else None
-                names = ("terms", "g", "vb", "lz", "sel", "idx", "excl", "pm", "pl", "pacc")
-            elif store == torch.int8:
-                b["sg"] = rows("sg", (nbp,), torch.float32)
-                b["keys"] = rows("route_keys", (nbp,), torch.int32) if nb > ROUTE_NB_LDS else None
-                units = [h * tiles(*w) for w in mine]
-                size = max((u * s for u in units if (s := route_segments(h * nt, u, nb, kx, leaf, _cus(dev))) > 1), default=0)
-                b["parts"] = None
-                if size:
-                    live.append(_buf(ws, "parts", (size * tile * (D + 1),), torch.float32, dev))
-                    b["parts"] = live[-1].data_ptr()
-                names = ("terms", "g", "sg", "vb", "lz", "idx", "keys", "parts")
+        def rows(name, tail, dtype, r=gn):
+            t = _buf(ws, name, (h * r, *tail), dtype, dev)
+            live.append(t)
+            return t.data_ptr()
+
+        b = {"terms": rows("mu_terms", (MUT_ROW,), torch.int16), "g": rows(gname, (nbp, d), store),
+             "vb": rows(vname, (nbp, d), vdt), "lz": rows("lz", (nbp,), torch.float32),
+             "idx": rows("idx", (kx,), torch.int32) if kx > 0 else None}
+        if f32dots:
+            b["sel"], b["excl"] = rows("sel", (nbp,), torch.float32), rows("excl", (nbp,), torch.int8)
+            part = next((tiles(*w) for w in mine if splits > 1 and h * tiles(*w) < unsplit), 0)
+            for name, tail in (("pm", (splits, tile)), ("pl", (splits, tile)), ("pacc", (splits, tile, d))):
+                b[name] = rows(name, tail, torch.float32, part) if part else None
+            names = ("terms", "g", "vb", "lz", "sel", "idx", "excl", "pm", "pl", "pacc")
+        elif store == torch.int8:
+            b["sg"] = rows("sg", (nbp,), torch.float32)
+            b["keys"] = rows("route_keys", (nbp,), torch.int32) if nb > ROUTE_NB_LDS else None
+            b["parts"], size = None, 0
+            for w in mine:
+                units = h * tiles(*w)
+                segs = route_segments(h * nt, units, nb, kx, leaf, cus)
+                if segs > 1:
+                    size = max(size, units * segs)
+            if size:
+                live.append(_buf(ws, "parts", (size * tile * (D + 1),), torch.float32, dev))
+                b["parts"] = live[-1].data_ptr()
+            names = ("terms", "g", "sg", "vb", "lz", "idx", "keys", "parts")
+        else:
+            b["sg"] = rows("sg", (nbp,), torch.float32) if fp8 else None
+            b["sv"] = rows("sv", (nbp,), torch.float32) if fp8 else None
+            names = ("terms", "g", "sg", "vb", "sv", "lz", "idx")
+        return [b[x] for x in names]
+
+    cus = _cus(dev) if store == torch.int8 else 0
+    if side:
+        for i, s in enumerate(side):
+            if wss[i] == {}:
+                with torch.cuda.stream(s):
+                    bufs += buffers(wss[i], wins[i::len(side)])
             else:
-                fp8 = store == torch.float8_e4m3fn
-                b["sg"] = rows("sg", (nbp,), torch.float32) if fp8 else None
-                b["sv"] = rows("sv", (nbp,), torch.float32) if fp8 else None
-                names = ("terms", "g", "sg", "vb", "sv", "lz", "idx")
-            bufs += [b[x] for x in names]
+                bufs += buffers(wss[i], wins[i::len(side)])
+        streams = [s.cuda_stream for s in side]
+    else:
+        bufs, streams = buffers(wss[0], wins), [stream_handle(dev)]
+    n = len(streams)
     bufs = (ctypes.c_void_p * len(bufs))(*bufs)
-    handles = (ctypes.c_void_p * n)(*([s.cuda_stream for s in side] or [stream_handle(dev)]))
+    handles = (ctypes.c_void_p * n)(*streams)
     shape = (h, nq, nk, leaf, d, kx, sink, stride, tile, group, wins[0][1])
     tail = (float(scale), ptr(rowmax), ptr(out), ptr(logz), n, bufs, handles)
     for s in side:
