@@ -22,7 +22,7 @@ LOGZ_ABS = 1e-3
 @pytest.mark.parametrize("store,heads", [("int8", 1), ("int8", 8), ("bf16", 1), ("fp8", 1)])
 @pytest.mark.parametrize("mag,vexp", [(20, 0), (27, 0), (32, 0), (34, 0), (27, 60), (32, 90)])
 def test_scores_far_above_the_reference(device, store, heads, mag, vexp):
-    """mag^2 / sqrt(128) nats above zero: 51, 93, 131 and 147 octaves (the last past the range)."""
+    """mag^2 / sqrt(128) nats above zero: 51, 93, 131 and 147 octaves, on both sides of the range's end."""
     if store == "fp8" and vexp:
         pytest.skip("the fp8 state's fp16 weights do not hold such value scales")
     n, leaf, ex, row = 1024, 64, 4, 5
