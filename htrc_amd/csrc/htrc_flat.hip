@@ -2500,21 +2500,6 @@ struct RowsN {         // softmax state of the 16 RB rows of one wave
     f32x4 o[RB][8];    // O^T per row block: dims 16db + 4grp + i of row 16rb + lane%16
 };
 
-// 0 when every partial output of the wave's row block is at most 1 / PARTS of the largest float, so that
-// the sum of PARTS such blocks is finite too, else NaN.  (The maximum that keeps NaN: v_maximum3_f32, two
-// values an instruction.)
-template <int PARTS>
-__device__ __forceinline__ float finite_zero(const f32x4 (&o)[8]) {
-    float z = 0.0f;
-#pragma unroll
-    for (int db = 0; db < 8; ++db)
-#pragma unroll
-        for (int i = 0; i < 4; i += 2)
-            z = __builtin_elementwise_maximum(__builtin_elementwise_maximum(z, __builtin_fabsf(o[db][i])),
-                                              __builtin_fabsf(o[db][i + 1]));
-    return __fmul_rn(__fmul_rn(z, (float)PARTS), 0.0f);
-}
-
 // p = 2^(u - m) for the log2-domain scores u[rb][0..7] of the RB row blocks (keys
 // 16(e/4) + 4grp + e%4 of the block; masked keys -inf), l += p, O^T += V^T P^T.  SHIFTED:
 // the scores are u - m already.
@@ -2554,13 +2539,34 @@ constexpr int MAX_PASSES = 2;
 // can lie far above the reference and hardly below: over heads of 40759 tokens whose scores spread by 11
 // nats a row's total is -0.2 to 116 octaves above it, and with totals up to 2^64 a quarter of those tiles
 // were computed twice.  Totals in [REF_MIN, REF_MAX] are taken as they are: all that a float holds but for
-// the room that keeps 1 / total a normal number.  A row of outputs that overflows at such a total, or could
-// once its key parts or segments are added, also sends its tile to the redo.  (A reference 36 octaves
-// higher takes totals up to 2^136: six of those heads a call 3672 us against 3692 here, 0.5 % between
-// runs.  But it puts an ordinary row's outputs at 2^-36 of its values, and values below 2^-66 then lose
-// bits.)
+// the room that keeps 1 / total a normal number.  A row of outputs that overflows at a total above 2^64, or
+// could once its key parts or segments are added, also sends its tile to the redo (part_total).  (A
+// reference 36 octaves higher takes totals up to 2^136: six of those heads a call 3672 us against 3692
+// here, 0.5 % between runs.  But it puts an ordinary row's outputs at 2^-36 of its values, and values below
+// 2^-66 then lose bits.)
 constexpr float REF_MIN = 0x1p-60f, REF_MAX = 0x1p125f;
 __device__ __forceinline__ float row_reference(float m) { return m == -INFINITY ? 0.0f : __fmul_rn(m, LOG2E); }
+// One of PARTS parts' share of the totals of a wave's rows (l: its lanes' shares, o: the rows' outputs):
+// NaN, which no range holds, where a share above OVERFLOW_MIN comes with an output past 1 / PARTS of the
+// largest float, so that the sum of the parts could overflow.  Row totals up to 2^64 are taken whatever
+// their outputs: finite values overflow there from 2^63 on alone, and a value that is infinite or NaN stays
+// so in every pass.  (The maximum that keeps NaN: v_maximum3_f32, two values an instruction.)
+constexpr float OVERFLOW_MIN = 0x1p62f;              // a total above 2^64 has a share above it in up to four parts
+template <int PARTS>
+__device__ __forceinline__ float part_total(float l, const f32x4 (&o)[8]) {
+    static_assert(PARTS <= 4, "OVERFLOW_MIN");
+    const float lt = grp_sum(l);
+    if (__builtin_expect(__ballot(lt > OVERFLOW_MIN) == 0, 1)) return lt;
+    float z = 0.0f;
+#pragma unroll
+    for (int db = 0; db < 8; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; i += 2)
+            z = __builtin_elementwise_maximum(__builtin_elementwise_maximum(z, __builtin_fabsf(o[db][i])),
+                                              __builtin_fabsf(o[db][i + 1]));
+    z = grp_sum(__fmul_rn(__fmul_rn(z, (float)PARTS), 0.0f));
+    return lt > OVERFLOW_MIN ? __fadd_rn(lt, z) : lt;
+}
 // Merge: the wave pairs' partial O, 64 rows x 128 dims each, rows padded to 132 floats.
 constexpr int MRG_STRIDE = 132;
 // Ring slots per pair: blocks are loaded RS - 1 ahead.  Two slots (one block in flight while the
@@ -3280,8 +3286,7 @@ __device__ __forceinline__ void route_body(
         if constexpr (MODE == ROUTE_SEGS) {
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
-                const float lt = pass == 0 ? __fadd_rn(st.l[rb], finite_zero<SEG_MAX>(st.o[rb])) : st.l[rb];
-                sum.l[rb] = __fadd_rn(sum.l[rb], grp_sum(lt));
+                sum.l[rb] = __fadd_rn(sum.l[rb], part_total<SEG_MAX>(st.l[rb], st.o[rb]));
 #pragma unroll
                 for (int db = 0; db < 8; ++db)
 #pragma unroll
@@ -3295,7 +3300,7 @@ __device__ __forceinline__ void route_body(
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
                 const int r = 16 * RB * hr + 16 * rb + col;
-                const float lt = grp_sum(__fadd_rn(st.l[rb], finite_zero<SEG_MAX>(st.o[rb])));
+                const float lt = part_total<SEG_MAX>(st.l[rb], st.o[rb]);
                 if (grp == 0) part_l[pb + r] = lt;
 #pragma unroll
                 for (int db = 0; db < 8; ++db) *(f32x4*)(part_o + (pb + r) * D + 16 * db + 4 * grp) = st.o[rb][db];
@@ -3310,7 +3315,7 @@ __device__ __forceinline__ void route_body(
         for (int rb = 0; rb < RB; ++rb) {
             float lt;
             if constexpr (MODE == ROUTE_SEGS) lt = sum.l[rb];
-            else lt = grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero<NP>(st.o[rb])) : st.l[rb]);
+            else lt = part_total<NP>(st.l[rb], st.o[rb]);
             if (grp == 0) red_l[pr][16 * RB * hr + 16 * rb + col] = lt;
         }
         if (threadIdx.x == 0) redo = 0;
@@ -4046,7 +4051,7 @@ __global__ __launch_bounds__(64 * NW, 2) void route16_kernel(
         // exact largest score, where each row total lies in [1, keys]
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-            const float lt = grp_sum(pass == 0 ? __fadd_rn(st.l[rb], finite_zero<1>(st.o[rb])) : st.l[rb]);
+            const float lt = part_total<1>(st.l[rb], st.o[rb]);
             if (grp == 0) red_l[16 * RB * wv + 16 * rb + col] = lt;
         }
         if (threadIdx.x == 0) redo = 0;

@@ -89,3 +89,21 @@ def test_small_values(device, store, heads, vexp):
         got = htrc_flat.flat_attention(q, k, small, **kw)
         rel = rel_l2((got[..., dims] / s).cpu().numpy(), want[..., dims].cpu().numpy())
         assert rel <= 2e-6, (dims, rel)
+
+
+@pytest.mark.parametrize("store,heads,n,m,leaf,near,chunk", [
+    ("int8", 1, 4096, 4096, 64, 8, None), ("int8", 6, 4096, 4096, 64, 8, None), ("int8", 8, 4096, 4096, 64, 8, None),
+    ("bf16", 2, 4096, 4096, 64, 8, None), ("fp8", 2, 4096, 4096, 64, 8, None),
+    ("int8", 1, 33000, 8192, 64, 66, None), ("int8", 1, 33000, 8192, 64, 66, 128)])     # segments in turn, apart
+def test_a_value_that_is_not_finite_stays_in_its_dim(device, store, heads, n, m, leaf, near, chunk):
+    """A NaN among the values makes its dim NaN and leaves the others' bits: tiles within the ordinary range of totals
+    are not redone (at another reference) for it."""
+    q, k, v = (x.to(device) for x in workloads.clustered_runs(n=max(n, m), runs=-(-max(n, m) // 64), heads=heads, seed=29))
+    q, k, v = q[:, :n].contiguous(), k[:, :m].contiguous(), v[:, :m].contiguous()
+    kw = dict(backend="hip", store=store, dot="bf16", leaf=leaf, exact_leaves=near, tile_chunk=chunk)
+    want = htrc_flat.flat_attention(q, k, v, **kw)
+    v[:, 100, 7] = float("nan")
+    got = htrc_flat.flat_attention(q, k, v, **kw)
+    dims = [i for i in range(128) if i != 7]
+    assert bool(torch.isnan(got[..., 7]).all())
+    assert torch.equal(got[..., dims], want[..., dims])
