@@ -39,28 +39,56 @@ __device__ __forceinline__ u32x2 pack8_i8(const int (&c)[8]) {
 }
 
 // pad_dims: rows of d < 128 values (fp32 or bf16) to rows of 128 (fp32 or bf16, rounded to nearest even)
-// with zeros past d, for up to three tensors (blockIdx.y) in one launch: four output dims per thread.  What
-// counts is the launches: a clear and a converting copy per tensor were six, 22 us of kernels and 20 us of
-// host time in a call of 1024 queries and 4096 keys of 64 dims (103 us; 82 with this one launch of 4.5 us).
+// with zeros past d, for up to three tensors (blockIdx.y) in one launch.  Small calls are bound by launches (a
+// clear and a converting copy per tensor were six, 22 us of kernels and 20 us of host time in a call of 1024
+// queries and 4096 keys of 64 dims: 103 us a call, 82 with one launch), large ones by the rows' bytes: a
+// workgroup takes PAD_ROWS rows, whose source is one run of bytes whatever d is, through LDS in 16-byte loads
+// (4-byte ones where the tensor starts off a 16-byte boundary) and writes 16 bytes a thread.  q, k and v of 24 heads
+// x 64512 rows, bf16, us: 64 dims 290 (6.1 TB/s; by clears and copies 354, with four values a thread read
+// one by one from global memory 871), 127 dims 394 (706, 902), 33 dims 288 (555, 789).
 struct PadTensor {
     const void* src;
     void* dst;
     int64_t rows;
-    int src_bf16, dst_bf16;
+    int src_bf16, dst_bf16, wide;      // wide: src is 16-byte aligned
 };
+constexpr int PAD_ROWS = 32;           // 32 rows of d values: a multiple of 64 d bytes
 __global__ __launch_bounds__(256) void pad_dims_kernel(PadTensor a, PadTensor b, PadTensor c, int d) {
+    __shared__ __align__(16) char buf[PAD_ROWS * D * 4];
     const PadTensor t = blockIdx.y == 0 ? a : (blockIdx.y == 1 ? b : c);
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < t.rows * (D / 4); i += (int64_t)gridDim.x * 256) {
-        const int64_t row = i / (D / 4);
-        const int c0 = 4 * (int)(i % (D / 4));
-        float x[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int64_t s = row * d + c0 + e;
-            x[e] = c0 + e >= d ? 0.0f : (t.src_bf16 ? bf2f(((const uint16_t*)t.src)[s]) : ((const float*)t.src)[s]);
+    const int es = t.src_bf16 ? 2 : 4, tid = threadIdx.x;
+    const uint16_t* hb = (const uint16_t*)buf;
+    const uint32_t* wb = (const uint32_t*)buf;
+    for (int64_t r0 = (int64_t)blockIdx.x * PAD_ROWS; r0 < t.rows; r0 += (int64_t)gridDim.x * PAD_ROWS) {
+        const int nr = (int)min((int64_t)PAD_ROWS, t.rows - r0), bytes = nr * d * es;
+        const char* src = (const char*)t.src + r0 * d * es;
+        const int step = t.wide ? 16 : 4, whole = bytes / step;
+        if (t.wide) {
+            for (int i = tid; i < whole; i += 256) ((u32x4*)buf)[i] = ((const u32x4*)src)[i];
+        } else {
+            for (int i = tid; i < whole; i += 256) ((uint32_t*)buf)[i] = ((const uint32_t*)src)[i];
         }
-        if (t.dst_bf16) ((u32x2*)t.dst)[i] = u32x2{f2bf(x[0]) | (f2bf(x[1]) << 16), f2bf(x[2]) | (f2bf(x[3]) << 16)};
-        else ((f32x4*)t.dst)[i] = f32x4{x[0], x[1], x[2], x[3]};
+        const int rest = whole * step / 2 + tid;                  // the last chunk's end, in 16-bit words
+        if (rest < bytes / 2) ((uint16_t*)buf)[rest] = ((const uint16_t*)src)[rest];
+        __syncthreads();
+        const int per = t.dst_bf16 ? 8 : 4, lg = t.dst_bf16 ? 4 : 5;   // values per 16 bytes, log2 of their pieces a row
+        u32x4* dst = (u32x4*)t.dst + (r0 << lg);
+        for (int p = tid; p < nr << lg; p += 256) {
+            const int c0 = (p & ((1 << lg) - 1)) * per, at = (p >> lg) * d + c0;
+            u32x4 y = {0u, 0u, 0u, 0u};
+            if (d % 8 == 0 && t.src_bf16 == t.dst_bf16) {         // whole pieces, copied
+                if (c0 < d) y = *(const u32x4*)(buf + (int64_t)at * es);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    if (e >= per || c0 + e >= d) continue;
+                    if (t.dst_bf16) y[e / 2] |= (t.src_bf16 ? (uint32_t)hb[at + e] : f2bf(__uint_as_float(wb[at + e]))) << (16 * (e % 2));
+                    else y[e & 3] = t.src_bf16 ? (uint32_t)hb[at + e] << 16 : wb[at + e];
+                }
+            }
+            dst[p] = y;
+        }
+        __syncthreads();
     }
 }
 
@@ -4861,8 +4889,9 @@ int htrc_pack_q(const void* q, int q_is_bf16, int64_t heads, int64_t nq, int d, 
 int htrc_pad_dims(const void* a, int a_bf16, int64_t a_rows, void* a_out, int a_out_bf16, const void* b, int b_bf16,
                   int64_t b_rows, void* b_out, int b_out_bf16, const void* c, int c_bf16, int64_t c_rows, void* c_out,
                   int c_out_bf16, int d, void* stream) {
-    const PadTensor t[3] = {{a, a_out, a_rows, a_bf16, a_out_bf16}, {b, b_out, b_rows, b_bf16, b_out_bf16},
-                            {c, c_out, c_rows, c_bf16, c_out_bf16}};
+    const PadTensor t[3] = {{a, a_out, a_rows, a_bf16, a_out_bf16, aligned(a, 16)},
+                            {b, b_out, b_rows, b_bf16, b_out_bf16, aligned(b, 16)},
+                            {c, c_out, c_rows, c_bf16, c_out_bf16, aligned(c, 16)}};
     REQUIRE(d >= 1 && d < D, "htrc_pad_dims: d must be in [1, 128)");
     int64_t most = 0;
     for (const PadTensor& x : t) {
@@ -4871,8 +4900,8 @@ int htrc_pad_dims(const void* a, int a_bf16, int64_t a_rows, void* a_out, int a_
         if (x.rows > most) most = x.rows;
     }
     if (most == 0) return HTRC_OK;
-    int64_t blocks = (most * (D / 4) + 255) / 256;
-    if (blocks > 16384) blocks = 16384;
+    int64_t blocks = (most + PAD_ROWS - 1) / PAD_ROWS;
+    if (blocks > (1 << 20)) blocks = 1 << 20;
     hipLaunchKernelGGL(pad_dims_kernel, dim3((unsigned)blocks, 3), dim3(256), 0, (hipStream_t)stream, t[0], t[1], t[2], d);
     return launched("htrc_pad_dims");
 }

@@ -76,6 +76,21 @@ def test_pad_dims_equals_torch(device, d, kinds):
         assert bool((o[..., d:] == 0).all())
 
 
+@pytest.mark.parametrize("d", [1, 31, 64, 96, 127])
+@pytest.mark.parametrize("kinds", [("bf16", "bf16"), ("fp32", "bf16"), ("fp32", "fp32"), ("bf16", "fp32")])
+def test_pad_dims_of_rows_off_a_16_byte_boundary(device, d, kinds):
+    """1 to 1500 rows (whole workgroups of 32 and a remainder) that start 0, 4, 8 and 12 bytes past such a boundary."""
+    dt = {"bf16": torch.bfloat16, "fp32": torch.float32}
+    src, dst = (dt[k] for k in kinds)
+    for rows in (1, 32, 33, 1500):
+        for off in (0, 4, 8, 12):
+            raw = torch.randn((rows * d + 8,), device=device).to(src)
+            x = raw[off // raw.element_size():][:rows * d].view(1, rows, d)
+            assert x.data_ptr() % 16 == off
+            (o,) = hip.pad_dims((x,), {"a": torch.full((1, rows, 128), 9.0, device=device, dtype=dst)}, ("a",), (dst,))
+            assert torch.equal(o[..., :d], x.to(dst)) and bool((o[..., d:] == 0).all())
+
+
 def test_odd_address_keys_take_the_copying_path(device):
     """Rows of 31 bf16 values at an address that is not a multiple of four: the same result."""
     q, k, v = (x[..., :31].contiguous().to(device) for x in workloads.clustered_runs(n=256, runs=4, heads=1, seed=2))
