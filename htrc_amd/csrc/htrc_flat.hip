@@ -2904,13 +2904,16 @@ __device__ __forceinline__ RowMax<RB> route_exact_max(const int8_t* dq8, const f
 //   calls lose there: 469 tiles 287 -> 339 (their whole-tile kernels split each tile's keys over several
 //   wave parts), 1094 1228 -> 1330, 1274 848 -> 935, 2548 1566 -> 1637 (more tiles a CU than the in-turn
 //   kernel's registers allow).
-//   segments_apart: of 1024 tiles, windows of 300 in turn 1184, apart 1128; of 400 1075 and 1105; of 640
-//   1015 and 1059.
+//   segments_apart (whole tiles / in turn / apart), up to one and a half tiles a CU whatever the blocks: 1024
+//   tiles of 256 blocks in windows of 300 1256 / 1184 / 1163; up to two from SEG_LONG_BLOCKS on: of 512 1041 /
+//   1110 / 1058, of 450 1224 / 1038 / 1111; of 640 blocks in windows of 512 1454 / 1693 / 1442; 637 tiles of 592
+//   996 / 879 / 763; shorter tiles not: 813 tiles of 230 765 / 753 / 772, 1024 of 136 264 / 267 / 282; and no
+//   further: 1024 of 256 in windows of 640 1016 / 1033 / 1050, in one 986 / 971 / 1052.
 //   SEG_MIN_BLOCKS: 637 tiles of 208 blocks gain as above, of 592 (1024 near leaves) in windows of 256
 //   1427 -> 753.  Fewer blocks would gain in windows of 128 too (112 blocks 606 -> 485, 84 398 -> 317, 52
 //   326 -> 289, 42 271 -> 269), not in one window (84 blocks 210 -> 212; 768 tiles of 34 blocks 94 -> 98).
 //   SEG_MAX: 4 segments against 6, 8 and 16 of 208 blocks: 706 / 715 / 720 / 720 us.
-constexpr int SEG_MIN_BLOCKS = 128;
+constexpr int SEG_MIN_BLOCKS = 128, SEG_LONG_BLOCKS = 256;
 constexpr int SEG_MAX = 4;
 constexpr int64_t SEG_TILES_MIN = 2, SEG_TILES_MAX = 4;   // (head, tile) pairs of the layer per CU: above, up to
 enum RouteMode { ROUTE_WHOLE = 0, ROUTE_PART = 1, ROUTE_SEGS = 2 };
@@ -2918,13 +2921,15 @@ constexpr int SEG_QUARTERS = 4;                      // workgroups per tile that
 
 // Segments of a layer's tiles.  (Heads of more than ROUTE_NB_LDS leaves, whose select works from global keys, keep
 // whole tiles.)
+inline int64_t tile_blocks(int64_t nb, int kxe, int leaf) { return (nb + 31) / 32 + ((int64_t)kxe * leaf + 31) / 32; }
 inline int route_segments(int64_t tiles, int64_t nb, int kxe, int leaf, int64_t cus) {
-    const int64_t blocks = (nb + 31) / 32 + ((int64_t)kxe * leaf + 31) / 32;
     const bool middling = tiles > SEG_TILES_MIN * cus && tiles <= SEG_TILES_MAX * cus;
-    return middling && blocks > SEG_MIN_BLOCKS && nb <= ROUTE_NB_LDS ? SEG_MAX : 1;
+    return middling && tile_blocks(nb, kxe, leaf) > SEG_MIN_BLOCKS && nb <= ROUTE_NB_LDS ? SEG_MAX : 1;
 }
-// Whether a launch of `units` tiles runs them apart: up to one and a half tiles a CU.
-inline bool segments_apart(int64_t units, int64_t cus) { return 2 * units <= 3 * cus; }
+// Whether a launch of `units` such tiles runs their segments apart.
+inline bool segments_apart(int64_t units, int64_t blocks, int64_t cus) {
+    return 2 * units <= 3 * cus || (units <= 2 * cus && blocks >= SEG_LONG_BLOCKS);
+}
 
 // RB 16-row blocks per wave, NH waves per key part (NH = 2: halves of the tile's rows; NH = 4, RB = 1:
 // quarters of a 64-row tile, the same sums per row); NP key parts of NH waves; RS ring slots per part.
@@ -5504,7 +5509,7 @@ static int route_attend_launch(const int8_t* q8, const float* sq, const int8_t* 
     if (nseg > 1) {
         REQUIRE(route_static_bytes(1) + dyn <= ROUTE_LDS_MAX, "htrc_route_attend: near list and exclusion bits exceed the LDS");
         const int64_t units = ntw * heads;
-        const bool split = parts && segments_apart(units, cus);
+        const bool split = parts && segments_apart(units, tile_blocks(nb, kxe, leaf), cus);
         REQUIRE(!split || aligned(parts, 16), "htrc_route_attend: misaligned buffer");
         float* part_o = split ? parts : nullptr;
         float* part_l = split ? parts + units * nseg * tile * D : nullptr;
@@ -5590,7 +5595,7 @@ int htrc_route_segments(int64_t heads, int64_t nq, int64_t nk, int leaf, int kx,
         HTRC_OK)
         return 0;
     const int64_t cus = device_cus();
-    return segments_apart(ntw * heads, cus) ? route_segments(nt * heads, nb, kxe, leaf, cus) : 1;
+    return segments_apart(ntw * heads, tile_blocks(nb, kxe, leaf), cus) ? route_segments(nt * heads, nb, kxe, leaf, cus) : 1;
 }
 
 int htrc_route_seg(const int8_t* q8, const float* sq, const int8_t* dq8, const float* sdq, const int8_t* g8,

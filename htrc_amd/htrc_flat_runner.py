@@ -65,15 +65,17 @@ F32_UNSPLIT_TILES = 2048
 
 # Fused int8 route: the segments whose partial sums a launch of ``units`` of a layer's ``tiles`` (head, tile) pairs
 # keeps in workspace (htrc_route_segments of the C ABI): tiles of more than 128 blocks of 32 keys, in layers of more than
-# two and up to four pairs a CU and launches of at most one and a half, and heads of at most 16384 leaves.
-SEG_MIN_BLOCKS, SEG_MAX, SEG_MAX_NB = 128, 4, 16384
+# two and up to four pairs a CU, heads of at most 16384 leaves, and launches of at most one and a half pairs a CU, or two
+# where a tile has 256 blocks or more.
+SEG_MIN_BLOCKS, SEG_LONG_BLOCKS, SEG_MAX, SEG_MAX_NB = 128, 256, 4, 16384
 CUS = 256                              # compute units of an MI355X: the memory model's device
 
 
 def route_segments(tiles: int, units: int, nb: int, kx: int, leaf: int, cus: int = CUS) -> int:
     blocks = _ceil(nb, 32) + _ceil(kx * leaf, 32)
-    segmented = 2 * cus < tiles <= 4 * cus and 2 * units <= 3 * cus and blocks > SEG_MIN_BLOCKS and nb <= SEG_MAX_NB
-    return SEG_MAX if segmented else 1
+    segmented = 2 * cus < tiles <= 4 * cus and blocks > SEG_MIN_BLOCKS and nb <= SEG_MAX_NB
+    apart = 2 * units <= 3 * cus or (units <= 2 * cus and blocks >= SEG_LONG_BLOCKS)
+    return SEG_MAX if segmented and apart else 1
 
 
 def workspace_bytes(queries: int, keys: int, leaf: int = 16, dim: int = 128, heads: int = 1, splits: int = 1,

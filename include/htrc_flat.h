@@ -171,7 +171,7 @@ int htrc_route(const int8_t* q8, const float* sq, const int8_t* dq8, const float
  * order the layer's shape fixes, so every window and launch of a layer gives the same bits.  parts (fp32,
  * 16-byte aligned, heads * tiles of the window * segments * T * 129 floats; NULL when htrc_route_segments() is 1)
  * takes the segments' sums where the window is small enough that they run as workgroups of their own
- * (one and a half tiles a CU); without it, and in larger windows, one workgroup runs a tile's segments in turn.
+ * (one and a half tiles a CU, two for tiles of 256 blocks or more); without it, and in larger windows, one workgroup runs a tile's segments in turn.
  * htrc_route_segments: the segments per tile that the window's launch keeps in parts, 1 when it needs
  * none, 0 with an error set when the arguments are invalid. */
 int htrc_route_segments(int64_t heads, int64_t nq, int64_t nk, int leaf, int kx, int tile, int group, int64_t g0,

@@ -64,6 +64,9 @@ def _route(device, n, m, leaf, kx, tile, group, g0, gn, spike):
     (33000, 33024, 128, 100, 64, 1, 0, 3, False, 4),    # 9 + 400 blocks
     (33000, 8192, 64, 66, 64, 1, 0, 384, False, 4),     # the largest launch that runs segments apart
     (33000, 8192, 64, 66, 64, 1, 0, 385, False, 1),     # in turn, no workspace
+    (33000, 16128, 64, 124, 64, 1, 0, 512, False, 4),   # 8 + 248 = 256 blocks: two tiles a CU apart
+    (33000, 16128, 64, 124, 64, 1, 0, 513, False, 1),
+    (33000, 16128, 64, 123, 64, 1, 0, 385, False, 1),   # 254 blocks
     (33000, 8192, 16, 300, 64, 1, 0, 8, True, 4),       # a row whose reference misses: the tile is redone
     (17000, 8192, 64, 64, 32, 1, 0, 8, True, 4)])
 def test_segmented_route(device, n, m, leaf, kx, tile, group, g0, gn, spike, segs):
