@@ -5447,10 +5447,14 @@ int htrc_route_select(const int8_t* dq8, const float* sdq, const int8_t* g8, con
     REQUIRE(!gk || keys_ws, "htrc_route_select: keys_ws [H, gn, nb_pad] is required above 16384 leaves per head");
     const int nbp = htrc_nb_pad(nb);
     const size_t dyn = gk ? 0 : (size_t)4 * nbp;
-    // waves per group: four where the groups alone give every SIMD two waves or a wave would have fewer than eight
-    // 16-leaf groups, more below that (the keys in global memory: heads of many leaves, four)
+    // waves per group: 16 up to half a group per CU, 8 up to one, unless a wave would have fewer than eight 16-leaf
+    // groups, else four (the keys in global memory: heads of many leaves, four).  More waves fill the CUs, and
+    // take them from the launches beside, above all another window's on the second stream.  us a call with 4 / 8
+    // / 16 waves (256 CUs): 128 groups of 2547 leaves, one head in windows 583 / - / 558, 256 groups of 2547, two heads
+    // in windows 1142 / 1145 / 1311, 256 of 4096 in one window 254 / 234 / 237; and above one group a CU 4 / 8: 384
+    // of 2547, three heads in windows 1543 / 1642, 500 of 2000 in one window 232 / 239, 313 of 1250 184 / 184.
     const int64_t cus = device_cus();
-    int nw = gk || nb < 1024 || gn * heads > 2 * cus ? 4 : (nb < 2048 || gn * heads > cus ? 8 : 16);
+    int nw = gk || nb < 1024 || gn * heads > cus ? 4 : (nb < 2048 || 2 * gn * heads > cus ? 8 : 16);
     if (nw == 16 && route_select_static_bytes(16) + dyn > ROUTE_LDS_MAX) nw = 8;   // (11 k leaves beside 16 rings)
 #define RSEL(M, N, G, NW)                                                                                       \
     hipLaunchKernelGGL((route_select_kernel<M, N, G, NW>), dim3((unsigned)(gn * heads)), dim3(64 * NW), dyn,     \

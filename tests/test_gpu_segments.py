@@ -79,15 +79,18 @@ def test_segmented_route(device, n, m, leaf, kx, tile, group, g0, gn, spike, seg
 
 
 @pytest.mark.parametrize("groups,nb,kx,sink,group", [
-    (300, 1008, 64, 0, 1), (40, 2547, 256, 0, 1), (40, 2547, 476, 220, 1), (300, 300, 128, 3, 1), (40, 130, 129, 0, 2), (300, 1500, 49, 0, 1), (300, 1500, 48, 0, 1),
+    (300, 1008, 64, 0, 1), (40, 2547, 256, 0, 1), (40, 2547, 476, 220, 1), (300, 300, 128, 3, 1), (40, 130, 129, 0, 2),
+    (300, 1500, 49, 0, 1), (300, 1500, 48, 0, 1),
     (600, 500, 57, 0, 1), (600, 1008, 56, 0, 1), (3, 12000, 100, 0, 1), (3, 11264, 129, 0, 1), (20, 257, 128, 0, 1),
-    (20, 66, 60, 0, 1)])
+    (20, 66, 60, 0, 1),
+    (128, 2100, 64, 0, 1), (129, 2100, 64, 0, 1), (256, 2100, 49, 3, 1), (257, 2100, 64, 0, 1), (256, 1024, 48, 0, 1),
+    (256, 1023, 64, 0, 1), (200, 1500, 49, 0, 1)])
 @pytest.mark.parametrize("ties", [False, True])
 def test_route_select_wave_counts(device, groups, nb, kx, sink, group, ties):
-    """route_select's launches of 4, 8 and 16 waves per tile group (more than 512, 257 to 512, fewer groups; heads
-    whose keys leave no room for 16 rings), and its top-k at and beside each bound of its methods: index sets
-    equal to the stage select and top-k on the same state, row maxima to the largest of the row's scores in 64 bits (four
-    roundings of 2^-24 of at most 127^2 * 128 * 1e-4 + 5 here: 5e-5)."""
+    """route_select's launches of 4, 8 and 16 waves per tile group (more than 256, 129 to 256, fewer groups; heads of
+    fewer than 1024 and 2048 leaves, and those whose keys leave no room for 16 rings), and its top-k at and beside
+    each bound of its methods: index sets equal to the stage select and top-k on the same state, row maxima to the
+    largest of the row's scores in 64 bits (four roundings of 2^-24 of at most 127^2 * 128 * 1e-4 + 5 here: 5e-5)."""
     torch.manual_seed(nb + kx)
     nbp, nt = -(-nb // 32) * 32, groups * group
     dq8 = torch.randint(-127, 128, (1, nt * 64, 128), device=device, dtype=torch.int8)
